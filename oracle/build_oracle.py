@@ -48,8 +48,8 @@ def build_oracle_native(out_dir) -> Path:
 
 
 def build_ref() -> Path | None:
-    if not Path("/root/reference").is_dir():
-        return None
+    if not Path("/root/reference/src/hmat/cluster/cluster.cc").is_file():
+        return None  # the reference's sources are not mounted
     script = HERE / "ref" / "build_ref.sh"
     res = subprocess.run(["bash", str(script)], capture_output=True, text=True)
     if res.returncode != 0:
