@@ -1,18 +1,15 @@
 """Launch-schedule autotuner for the slab kernels.
 
-Three knobs shape a matvec's schedule on the device:
+Two knobs shape a matvec's schedule on the device:
 
-- the unroll depth of ``k_slab`` (loads in flight per lane: 4, 8 or 16),
+- the unroll depth of ``k_slab`` (loads in flight per lane: 4 or 8),
   switchable per handle at no cost (``bw_hip_set_unroll``);
-- the schedule of the MFMA kernels of the batched matvec (group pairs per
-  step, depth of the load pipeline; ``bw_hip_set_mfma_schedule``, per
-  precision), also free;
 - the work-item size (bytes of factors one workgroup streams), fixed when the
   layout is built (``bw_hip_set_tuning`` before ``HipHmat``).
 
 ``tune_unroll`` times each unroll depth on the handle's own data with the
-engine's HIP-event timers and keeps the fastest one for each pass; ``tune_mfma`` does the
-same for the MFMA schedules.  ``tune_layout`` rebuilds
+engine's HIP-event timers and keeps the fastest one for each pass; ``tune_mfma``
+times the batched product.  ``tune_layout`` rebuilds
 the handle for each candidate work-item size (a full re-layout and upload, so
 only worth it for matrices that are applied many times) and returns the best.
 Results are cached per matrix signature in ``~/.cache/bigwham_dev_amd/tune.json``
@@ -25,10 +22,8 @@ import json
 import os
 from dataclasses import dataclass, field
 
-UNROLLS = (4, 8, 16)
-MFMA_SCHEDULES = (0, 1, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15)   # 2 spills registers on gfx950
-MFMA64_SCHEDULES = (0, 4, 5, 6, 7, 8, 9, 10, 11)       # 1-3 are 0 for FP64
-WI_BYTES = (64 << 10, 96 << 10, 192 << 10, 384 << 10)
+UNROLLS = (4, 8)
+WI_BYTES = (128 << 10, 192 << 10, 384 << 10, 768 << 10)
 
 
 @dataclass
@@ -116,28 +111,20 @@ def tune_unroll(dev, precisions=None, reps: int = 5, use_cache: bool = True) -> 
 
 
 def tune_mfma(dev, nrhs: int = 32, reps: int = 5, precision: str = "fp32") -> dict:
-    """Time the schedules of the batched MFMA kernel of one precision (group
-    pairs per step, depth of the load pipeline) on `nrhs` right-hand sides
-    and keep the fastest.  Returns {schedule: ms per batched call, "best":
-    schedule}."""
+    """Time the batched product of one precision on `nrhs` right-hand sides.
+    Its kernels have one schedule (0): returns {0: ms per call, "best": 0}."""
     import time
 
     import torch
     X = torch.ones((dev.n_cols, nrhs), dtype=torch.float64, device=dev.torch_device)
     Y = torch.empty((dev.n_rows, nrhs), dtype=torch.float64, device=dev.torch_device)
-    ms = {}
-    for sch in (MFMA_SCHEDULES if precision == "fp32" else MFMA64_SCHEDULES):
-        dev.set_mfma_schedule(sch, precision)
+    dev.matvec_batched(X, precision=precision, out=Y)
+    torch.cuda.synchronize()
+    t0 = time.perf_counter()
+    for _ in range(reps):
         dev.matvec_batched(X, precision=precision, out=Y)
-        torch.cuda.synchronize()
-        t0 = time.perf_counter()
-        for _ in range(reps):
-            dev.matvec_batched(X, precision=precision, out=Y)
-        torch.cuda.synchronize()
-        ms[sch] = (time.perf_counter() - t0) / reps * 1e3
-    best = min(ms, key=ms.get)
-    dev.set_mfma_schedule(best, precision)
-    return {**ms, "best": best}
+    torch.cuda.synchronize()
+    return {0: (time.perf_counter() - t0) / reps * 1e3, "best": 0}
 
 
 def tune_layout(make_dev, precisions=("fp64", "fp32"), candidates=WI_BYTES, reps: int = 5):

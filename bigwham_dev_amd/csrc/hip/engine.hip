@@ -1,6 +1,6 @@
 // MI355X (gfx950) hierarchical-matrix matvec engine and its C-ABI.
 //
-// One matvec y = H x is five kernels on the caller's stream:
+// One matvec y = H x is three to five kernels on the caller's stream:
 //   k_gather   x -> xt[0:n]   (permutation of matvecOriginal, hmat.cc:586-593,
 //                              or a copy; converts to the factor precision)
 //   k_slab     pass 1: t = W x   (W_k = B_k), each row written through the
@@ -23,6 +23,7 @@
 #include <mutex>
 #include <string>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "../../../include/bigwham_hip.h"
@@ -60,1251 +61,31 @@ int fail(int code, const std::string& m) {
       return fail(BW_EHIP, std::string(#expr) + ": " + hipGetErrorString(e_));    \
   } while (0)
 
-typedef double dbl2 __attribute__((ext_vector_type(2)));
-typedef float flt4 __attribute__((ext_vector_type(4)));
+#include "slab_kernels.h"
+#include "batched_kernels.h"
 
-template <typename T>
-struct Vec;
-template <>
-struct Vec<double> {
-  static constexpr int V = 2;
-  typedef dbl2 type;
-};
-template <>
-struct Vec<float> {
-  static constexpr int V = 4;
-  typedef flt4 type;
-};
-
-// Workgroups are dispatched round-robin over the 8 XCDs of the MI355X
-// (workgroup b runs on XCD b % 8).  Each XCD gets a contiguous range of work
-// items of about equal bytes (neighbouring row clusters share x entries in
-// that XCD's L2, and no XCD is left with the tail); its workgroups take the
-// range WAVES WIs at a time (WAVES = waves per workgroup).  Returns the WI of
-// this wave, or -1.
-struct XcdSplit {
-  int32_t s[bwl::kXcds + 1];
-};
-
-template <int WAVES = 4>
-__device__ __forceinline__ int xcd_work_item(const XcdSplit& xs) {
-  const int x = blockIdx.x % bwl::kXcds;
-  const int k = blockIdx.x / bwl::kXcds;
-  const int w = xs.s[x] + WAVES * k + static_cast<int>(threadIdx.x >> 6);
-  return w < xs.s[x + 1] ? w : -1;
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void k_gather(const double* __restrict__ x,
-                                                T* __restrict__ xt, int64_t n,
-                                                const int64_t* __restrict__ perm, int dof) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  int64_t src = i;
-  if (perm) {
-    const int64_t p = i / dof;
-    src = dof * perm[p] + (i - p * dof);
-  }
-  xt[i] = static_cast<T>(x[src]);
-}
-
-template <typename OutT>
-__device__ __forceinline__ int64_t out_index(int64_t idx, const int64_t* perm, int dof) {
-  if (!perm) return idx;
-  // row indices fit in 32 bits (checked when the layout is built)
-  const int i = static_cast<int>(idx);
-  const int p = i / dof;
-  return dof * perm[p] + (i - p * dof);
-}
-
-// One wavefront per work item and per workgroup: work items differ in size
-// (small pass-1 slabs next to long ones), and a workgroup of several waves
-// would hold its slot until its longest wave ends.
-// T: factor / accumulation type; OutT: output type (T for pass 1, double
-// for pass 2); U: unroll depth (independent 16-byte loads in flight per lane);
-// PASS only names the two launches apart in profiles.
-template <typename T, typename OutT, int U, int PASS>
-__global__ __launch_bounds__(64) void k_slab(const bwl::WorkItem* __restrict__ wis, XcdSplit xs,
-                                              const int32_t* __restrict__ gidx,
-                                              const T* __restrict__ data,
-                                              const T* __restrict__ xin,
-                                              OutT* __restrict__ out, T* __restrict__ part,
-                                              const int64_t* __restrict__ perm, int dof,
-                                              const int32_t* __restrict__ rowmap) {
-  typedef typename Vec<T>::type VT;
-  constexpr int V = Vec<T>::V;
-  const int lane = threadIdx.x & 63;
-  const int w = xcd_work_item<1>(xs);
-  if (w < 0) return;
-  const bwl::WorkItem wi = wis[w];
-  const int R = wi.rows;
-  const int ng = wi.ngroups;
-  const VT* __restrict__ base = reinterpret_cast<const VT*>(data + wi.data_off);
-  const int32_t* __restrict__ gi = gidx + wi.gbeg;
-  T acc0 = 0, acc1 = 0;
-  int nsplit = 1;
-  int split = 0;
-  if (R > 32) {
-    // One column group per iteration for the whole wavefront: group index
-    // and input entries are wave-uniform (scalar loads).
-    if (lane < R) {
-      const VT* p = base + lane;
-      int g = 0;
-      // Full batches of U groups through two register buffers: the loads of
-      // batch b + 1 go out before the FMAs of batch b, so a batch's loads are
-      // in flight while the previous one is consumed (one buffer drained to
-      // nothing before the next loads went out).  The loop body issues the
-      // same loads on every trip and the last one or two batches are peeled,
-      // so the waits the compiler places are the same on every path.  Same
-      // groups, same accumulator per group and same order: same bits.
-      const int nfull = ng / U;
-      if (nfull > 0) {
-        VT a[U], b[U];
-        int za[U], zb[U];
-        auto load = [&](int g0, VT (&buf)[U], int (&zz)[U]) {
-#pragma unroll
-          for (int u = 0; u < U; ++u) zz[u] = gi[g0 + u];
-#pragma unroll
-          for (int u = 0; u < U; ++u) buf[u] = __builtin_nontemporal_load(p + (g0 + u) * R);
-        };
-        auto use = [&](const VT (&buf)[U], const int (&zz)[U]) {
-#pragma unroll
-          for (int u = 0; u < U; ++u) {
-            // unsigned: no sign extension of the loaded offset is placed
-            // (and waited for) next to its load
-            const uint32_t z = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(zz[u]));
-#pragma unroll
-            for (int v = 0; v < V; ++v) {
-              if (u & 1)
-                acc1 += buf[u][v] * xin[z + v];
-              else
-                acc0 += buf[u][v] * xin[z + v];
-            }
-          }
-        };
-        load(0, a, za);
-        int bt = 0;
-        for (; bt + 2 < nfull; bt += 2) {
-          __builtin_amdgcn_sched_barrier(0);
-          load((bt + 1) * U, b, zb);
-          __builtin_amdgcn_sched_barrier(0);
-          use(a, za);
-          __builtin_amdgcn_sched_barrier(0);
-          load((bt + 2) * U, a, za);
-          __builtin_amdgcn_sched_barrier(0);
-          use(b, zb);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        if (bt + 2 == nfull) {
-          load((bt + 1) * U, b, zb);
-          __builtin_amdgcn_sched_barrier(0);
-          use(a, za);
-          __builtin_amdgcn_sched_barrier(0);
-          use(b, zb);
-        } else {
-          use(a, za);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        g = nfull * U;
-      }
-      // the last, partial batch in steps of four groups, then one at a time
-      for (; g + 4 <= ng; g += 4) {
-        VT a[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) a[u] = __builtin_nontemporal_load(p + (g + u) * R);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int z = __builtin_amdgcn_readfirstlane(gi[g + u]);
-#pragma unroll
-          for (int v = 0; v < V; ++v) acc0 += a[u][v] * xin[z + v];
-        }
-      }
-      for (; g < ng; ++g) {
-        const VT a = __builtin_nontemporal_load(p + g * R);
-        const int z = __builtin_amdgcn_readfirstlane(gi[g]);
-#pragma unroll
-        for (int v = 0; v < V; ++v) acc0 += a[v] * xin[z + v];
-      }
-    }
-  } else {
-    // Several column groups per iteration: lane = split * R + row.
-    nsplit = 64 / R;
-    split = lane / R;
-    const int row = lane - split * R;
-    if (split < nsplit && ng > 0) {
-      const VT* p = base + row;
-      const int step = U * nsplit;
-      // The input offsets of a step are loaded one step ahead, so the input
-      // entries are requested together with the factors and one memory
-      // round trip covers both (offsets past the end are clamped, unused).
-      int zc[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) zc[u] = gi[min(split + u * nsplit, ng - 1)];
-      int g = split;
-      for (; g + (U - 1) * nsplit < ng; g += step) {
-        VT a[U];
-        T xv[U][V];
-        int zn[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) a[u] = __builtin_nontemporal_load(p + (g + u * nsplit) * R);
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-          for (int v = 0; v < V; ++v) xv[u][v] = xin[zc[u] + v];
-#pragma unroll
-        for (int u = 0; u < U; ++u) zn[u] = gi[min(g + step + u * nsplit, ng - 1)];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-#pragma unroll
-          for (int v = 0; v < V; ++v) {
-            if (u & 1)
-              acc1 += a[u][v] * xv[u][v];
-            else
-              acc0 += a[u][v] * xv[u][v];
-          }
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) zc[u] = zn[u];
-      }
-      for (; g < ng; g += nsplit) {
-        const VT a = __builtin_nontemporal_load(p + g * R);
-        const int z = gi[g];
-#pragma unroll
-        for (int v = 0; v < V; ++v) acc0 += a[v] * xin[z + v];
-      }
-    }
-  }
-  T acc = acc0 + acc1;
-  // fold the column splits onto lanes 0..R-1, in split order
-  for (int s = 1; s < nsplit; ++s) {
-    const T o = __shfl(acc, lane + s * R, 64);
-    if (split == 0) acc += o;
-  }
-  if (wi.part_off < 0) {
-    if (lane < R) {
-      // pass 1 rows go to their t entries through the row map
-      const int64_t orow = rowmap ? rowmap[wi.out_row + lane] : static_cast<int64_t>(wi.out_row) + lane;
-      out[out_index<OutT>(orow, perm, dof)] = static_cast<OutT>(acc);
-    }
-    return;
-  }
-  // Split slab: the partial sums are added in work-item order by k_reduce.
-  // (A last-work-item-reduces variant needs agent-scope release/acquire
-  // fences, which write back and invalidate the per-XCD L2 and cost more than
-  // the separate pass saves.)
-  if (lane < R) part[wi.part_off + lane] = acc;
-}
-
-template <typename T, typename OutT>
-__global__ __launch_bounds__(64) void k_reduce(const bwl::Reduce* __restrict__ reds, int nred,
-                                               const T* __restrict__ part, OutT* out,
-                                               const int64_t* __restrict__ perm, int dof,
-                                               const int32_t* __restrict__ rowmap) {
-  const int r = blockIdx.x;
-  if (r >= nred) return;
-  const bwl::Reduce rd = reds[r];
-  const int t = threadIdx.x;
-  if (t >= rd.rows) return;
-  // four interleaved partial sums keep four loads in flight; the order of
-  // the additions is fixed, so the result is deterministic
-  const T* p = part + rd.part_off + t;
-  const int R = rd.rows;
-  T s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-  int q = 0;
-  for (; q + 4 <= rd.nparts; q += 4) {
-    s0 += p[(q + 0) * R];
-    s1 += p[(q + 1) * R];
-    s2 += p[(q + 2) * R];
-    s3 += p[(q + 3) * R];
-  }
-  for (; q < rd.nparts; ++q) s0 += p[q * R];
-  const T s = (s0 + s1) + (s2 + s3);
-  const int64_t orow = rowmap ? rowmap[rd.out_row + t] : static_cast<int64_t>(rd.out_row) + t;
-  out[out_index<OutT>(orow, perm, dof)] = static_cast<OutT>(s);
-}
-
-// Sub-matrix selection: the input is scattered into the (zeroed) x part of xt
-// at the permuted points of the selected columns, and the output gathered
-// from a full permuted y at the selected rows.
-template <typename T>
-__global__ __launch_bounds__(256) void k_scatter_sel(const double* __restrict__ x,
-                                                     T* __restrict__ xt,
-                                                     const int64_t* __restrict__ src,
-                                                     const int64_t* __restrict__ dst, int64_t n,
-                                                     int dof) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n * dof) return;
-  const int64_t p = i / dof;
-  const int64_t c = i - p * dof;
-  xt[dof * dst[p] + c] = static_cast<T>(x[dof * src[p] + c]);
-}
-
-__global__ __launch_bounds__(256) void k_gather_sel(const double* __restrict__ yfull,
-                                                    double* __restrict__ y,
-                                                    const int64_t* __restrict__ dst, int64_t n,
-                                                    int dof) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n * dof) return;
-  const int64_t p = i / dof;
-  y[i] = yfull[dof * dst[p] + (i - p * dof)];
-}
-
-// ---------------------------------------------------------------------------
-// Many right-hand sides on FP32 MFMA.
-//
-// The FP32 slab layout serves as the A operand of v_mfma_f32_32x32x2f32
-// without change: lanes 0-31 read rows 0-31 of column group g, lanes 32-63
-// rows 0-31 of group g+1, 16 bytes (4 columns) each; element s of a lane's
-// vector is A[row][k] of MFMA step s, with k = lane / 32 selecting the group.
-// The B operand is the gathered input XB[z][n] (row-major, kRhs columns):
-// lane l reads XB[z(g + l/32) + s][l % 32], 128 contiguous bytes per
-// half-wavefront.  The 32 x 32 accumulator holds rows x right-hand sides;
-// element j of lane l is row 8*(j/4) + 4*(l/32) + j%4, column l % 32.
-constexpr int kRhs = 32;
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-
-template <typename T>
-__global__ __launch_bounds__(256) void k_gather_b(const double* __restrict__ X, int64_t xr,
-                                                  int64_t xc,
-                                                  int nrhs, T* __restrict__ XB, int64_t n,
-                                                  const int64_t* __restrict__ perm, int dof) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * (blockDim.x / kRhs) + threadIdx.x / kRhs;
-  const int c = threadIdx.x % kRhs;
-  if (i >= n) return;
-  int64_t src = i;
-  if (perm) {
-    const int64_t p = i / dof;
-    src = dof * perm[p] + (i - p * dof);
-  }
-  XB[i * kRhs + c] = c < nrhs ? static_cast<T>(X[src * xr + c * xc]) : T(0);
-}
-
-// The same gather for a row-major X (unit column stride, even row stride,
-// 16-byte aligned): eight threads per row, four columns each, two 16-byte
-// loads and one 16-byte (FP32) or two (FP64) stores per thread.
-template <typename T>
-__global__ __launch_bounds__(256) void k_gather_b4(const double* __restrict__ X, int64_t xr,
-                                                   int nrhs, T* __restrict__ XB, int64_t n,
-                                                   const int64_t* __restrict__ perm, int dof) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * (blockDim.x / 8) + threadIdx.x / 8;
-  const int c0 = 4 * (threadIdx.x % 8);
-  if (i >= n) return;
-  int64_t src = i;
-  if (perm) {
-    const int64_t p = i / dof;
-    src = dof * perm[p] + (i - p * dof);
-  }
-  const double* __restrict__ row = X + src * xr + c0;
-  double v[4];
-  if (c0 + 4 <= nrhs) {
-    const dbl2 a = *reinterpret_cast<const dbl2*>(row);
-    const dbl2 b = *reinterpret_cast<const dbl2*>(row + 2);
-    v[0] = a.x; v[1] = a.y; v[2] = b.x; v[3] = b.y;
-  } else {
-#pragma unroll
-    for (int k = 0; k < 4; ++k) v[k] = c0 + k < nrhs ? row[k] : 0.0;
-  }
-  T* dst = XB + i * kRhs + c0;
-  if constexpr (sizeof(T) == 4) {
-    *reinterpret_cast<flt4*>(dst) = flt4{static_cast<float>(v[0]), static_cast<float>(v[1]),
-                                         static_cast<float>(v[2]), static_cast<float>(v[3])};
-  } else {
-    *reinterpret_cast<dbl2*>(dst) = dbl2{v[0], v[1]};
-    *reinterpret_cast<dbl2*>(dst + 2) = dbl2{v[2], v[3]};
-  }
-}
-
-// KU group pairs per step; PIPE: the loads of step i+1 are issued before the
-// MFMAs of step i.  Addresses are clamped into the work item, so every lane
-// loads valid data; a group past the end gets B = 0 (its A rows then add
-// nothing), and rows past R are never stored.  The mask is applied at the
-// MFMA, not at the load, so no VALU op waits on a load of the next step.
-// Output of the batched kernels: pass 1 writes t (row through rowmap, kRhs
-// values per row), pass 2 writes Y (row through the point permutation, row
-// stride yr, column stride yc).
-// batched_rows maps N output rows of a work item (indices already clamped
-// into range) to the rows they are stored at, with straight-line code per
-// case, so that all index loads go out before the first one is waited for:
-// pass 1 through rowmap, pass 2 through the point permutation.  Row indices
-// and permutation entries are below 2^31 (checked when the layout is built),
-// so the low word of each permutation entry is the whole value.
-template <int PASS, int N>
-__device__ __forceinline__ void batched_rows(const int (&idx)[N], const int32_t* rowmap,
-                                             const int64_t* perm, int dof, int (&out)[N]) {
-  if (PASS == 1) {
-#pragma unroll
-    for (int j = 0; j < N; ++j) out[j] = rowmap[idx[j]];
-  } else if (perm) {
-    const int32_t* plo = reinterpret_cast<const int32_t*>(perm);
-    int pv[N];
-#pragma unroll
-    for (int j = 0; j < N; ++j) pv[j] = plo[2 * (idx[j] / dof)];
-#pragma unroll
-    for (int j = 0; j < N; ++j) out[j] = dof * pv[j] + idx[j] % dof;
-  } else {
-#pragma unroll
-    for (int j = 0; j < N; ++j) out[j] = idx[j];
-  }
-}
-
-template <int PASS, typename T>
-__device__ __forceinline__ void batched_put(T* tout, double* Y, int64_t yr, int64_t yc, int row,
-                                            int n, T v) {
-  if (PASS == 1)
-    tout[static_cast<int64_t>(row) * kRhs + n] = v;
-  else
-    Y[row * yr + n * yc] = static_cast<double>(v);
-}
-
-template <int KU, bool PIPE, bool TWO>
-__device__ __forceinline__ void mfma_stream(const flt4* __restrict__ base,
-                                            const int32_t* __restrict__ gi,
-                                            const float* __restrict__ XB, int ng, int R, int half,
-                                            int r0, floatx16& acc0, floatx16& acc1) {
-  const int rA0 = min(r0, R - 1), rA1 = min(r0 + 32, R - 1);
-  auto load_z = [&](int g0, int (&z)[KU]) {
-#pragma unroll
-    for (int u = 0; u < KU; ++u) z[u] = gi[min(g0 + 2 * u + half, ng - 1)];
-  };
-  auto load_ab = [&](int g0, const int (&z)[KU], flt4 (&a0)[KU], flt4 (&a1)[KU],
-                     float (&b)[KU][4], bool (&ok)[KU]) {
-#pragma unroll
-    for (int u = 0; u < KU; ++u) {
-      const int gg = g0 + 2 * u + half;
-      ok[u] = gg < ng;
-      const int ga = min(gg, ng - 1);
-      a0[u] = __builtin_nontemporal_load(base + ga * R + rA0);
-      if (TWO) a1[u] = __builtin_nontemporal_load(base + ga * R + rA1);
-#pragma unroll
-      for (int s = 0; s < 4; ++s) b[u][s] = XB[static_cast<int64_t>(z[u] + s) * kRhs + r0];
-    }
-  };
-  auto compute = [&](const flt4 (&a0)[KU], const flt4 (&a1)[KU], const float (&b)[KU][4],
-                     const bool (&ok)[KU]) {
-#pragma unroll
-    for (int u = 0; u < KU; ++u)
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const float bv = ok[u] ? b[u][s] : 0.0f;
-        acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[u][s], bv, acc0, 0, 0, 0);
-        if (TWO) acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[u][s], bv, acc1, 0, 0, 0);
-      }
-  };
-  int z[KU];
-  load_z(0, z);
-  if (!PIPE) {
-    for (int g0 = 0; g0 < ng; g0 += 2 * KU) {
-      int zn[KU];
-      load_z(g0 + 2 * KU, zn);
-      flt4 a0[KU], a1[KU];
-      float b[KU][4];
-      bool ok[KU];
-      load_ab(g0, z, a0, a1, b, ok);
-      compute(a0, a1, b, ok);
-#pragma unroll
-      for (int u = 0; u < KU; ++u) z[u] = zn[u];
-    }
-  } else {
-    // ping-pong buffers, two steps per trip, so no register copies sit
-    // between the loads of one step and the MFMAs of the other
-    flt4 pa0[KU], pa1[KU], qa0[KU], qa1[KU];
-    float pb[KU][4], qb[KU][4];
-    bool pok[KU], qok[KU];
-    load_ab(0, z, pa0, pa1, pb, pok);
-    load_z(2 * KU, z);  // offsets of step 1
-    for (int g0 = 0; g0 < ng; g0 += 4 * KU) {
-      int zn[KU];
-      load_z(g0 + 4 * KU, zn);
-      load_ab(g0 + 2 * KU, z, qa0, qa1, qb, qok);
-      __builtin_amdgcn_sched_barrier(0);
-      compute(pa0, pa1, pb, pok);
-      if (g0 + 2 * KU >= ng) break;
-      load_z(g0 + 6 * KU, z);
-      load_ab(g0 + 4 * KU, zn, pa0, pa1, pb, pok);
-      __builtin_amdgcn_sched_barrier(0);
-      compute(qa0, qa1, qb, qok);
-    }
-  }
-}
-
-// Deep variant: D step buffers in registers used as a ring.  At stage j the
-// loads of step s + D - 1 go out before the MFMAs of step s, so D - 1 steps
-// of factor and input loads are in flight per wave while its MFMAs run (the
-// two-buffer pipeline above keeps one).  Steps past the end load clamped,
-// in-bounds addresses and skip their MFMAs (a wave-uniform branch).  zz[k]
-// holds the input offsets of the next step to be loaded into buffer k.
-template <int KU, int D, bool TWO>
-__device__ __forceinline__ void mfma_stream_deep(const flt4* __restrict__ base,
-                                                 const int32_t* __restrict__ gi,
-                                                 const float* __restrict__ XB, int ng, int R,
-                                                 int half, int r0, floatx16& acc0,
-                                                 floatx16& acc1) {
-  constexpr int G = 2 * KU;  // groups per step
-  const int rA0 = min(r0, R - 1), rA1 = min(r0 + 32, R - 1);
-  const int nsteps = (ng + G - 1) / G;
-  flt4 a0[D][KU], a1[D][KU];
-  float b[D][KU][4];
-  int zz[D][KU];
-  auto gz = [&](int step, int u) { return gi[min(step * G + 2 * u + half, ng - 1)]; };
-  auto load = [&](int step, const int (&z)[KU], flt4 (&x0)[KU], flt4 (&x1)[KU],
-                  float (&bb)[KU][4]) {
-#pragma unroll
-    for (int u = 0; u < KU; ++u) {
-      const int ga = min(step * G + 2 * u + half, ng - 1);
-      x0[u] = __builtin_nontemporal_load(base + ga * R + rA0);
-      if (TWO) x1[u] = __builtin_nontemporal_load(base + ga * R + rA1);
-#pragma unroll
-      for (int s = 0; s < 4; ++s) bb[u][s] = XB[static_cast<int64_t>(z[u] + s) * kRhs + r0];
-    }
-  };
-  auto compute = [&](int step, const flt4 (&x0)[KU], const flt4 (&x1)[KU],
-                     const float (&bb)[KU][4]) {
-#pragma unroll
-    for (int u = 0; u < KU; ++u) {
-      const bool ok = step * G + 2 * u + half < ng;
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const float bv = ok ? bb[u][s] : 0.0f;
-        acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(x0[u][s], bv, acc0, 0, 0, 0);
-        if (TWO) acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(x1[u][s], bv, acc1, 0, 0, 0);
-      }
-    }
-  };
-#pragma unroll
-  for (int k = 0; k < D; ++k)
-#pragma unroll
-    for (int u = 0; u < KU; ++u) zz[k][u] = gz(k, u);
-#pragma unroll
-  for (int k = 0; k < D - 1; ++k) {
-    load(k, zz[k], a0[k], a1[k], b[k]);
-#pragma unroll
-    for (int u = 0; u < KU; ++u) zz[k][u] = gz(k + D, u);
-  }
-  for (int s0 = 0; s0 < nsteps; s0 += D) {
-#pragma unroll
-    for (int j = 0; j < D; ++j) {
-      const int s = s0 + j;
-      const int k = (j + D - 1) % D;  // buffer freed by the previous stage
-      load(s + D - 1, zz[k], a0[k], a1[k], b[k]);
-#pragma unroll
-      for (int u = 0; u < KU; ++u) zz[k][u] = gz(s + 2 * D - 1, u);
-      __builtin_amdgcn_sched_barrier(0);
-      if (s < nsteps) compute(s, a0[j], a1[j], b[j]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  }
-}
-
-// Ring variant with the loads issued in the order they are consumed: at
-// stage j the MFMAs of buffer j run (its loads went out one trip, D stages,
-// earlier), then buffer j is refilled with the step D ahead and the input
-// offsets of the step after that.  The prologue fills the buffers in the same
-// order as the loop, so every stage has the same D - 1 younger steps in
-// flight on every path (the loop above refills a buffer before the MFMAs and
-// its prologue order differs from the loop's, so the wait at the top of the
-// loop covered only one step).  Loads and MFMAs are unconditional, so that
-// the loop body is one basic block and its waits are the same on every
-// path: past the last step the loads read clamped, in-bounds addresses and
-// the MFMAs get B = 0 (as groups past the end do), adding nothing.
-template <int KU, int D, bool TWO>
-__device__ __forceinline__ void mfma_stream_ring(const flt4* __restrict__ base,
-                                                 const int32_t* __restrict__ gi,
-                                                 const float* __restrict__ XB, int ng, int R,
-                                                 int half, int r0, floatx16& acc0,
-                                                 floatx16& acc1) {
-  constexpr int G = 2 * KU;  // groups per step
-  const int rA0 = min(r0, R - 1), rA1 = min(r0 + 32, R - 1);
-  const int nsteps = (ng + G - 1) / G;
-  flt4 a0[D][KU], a1[D][KU];
-  float b[D][KU][4];
-  int zz[D][KU];  // input offsets of the step buffer k is refilled with next
-  auto gz = [&](int step, int u) { return gi[min(step * G + 2 * u + half, ng - 1)]; };
-  auto load = [&](int step, const int (&z)[KU], flt4 (&x0)[KU], flt4 (&x1)[KU],
-                  float (&bb)[KU][4]) {
-#pragma unroll
-    for (int u = 0; u < KU; ++u) {
-      const int ga = min(step * G + 2 * u + half, ng - 1);
-      x0[u] = __builtin_nontemporal_load(base + ga * R + rA0);
-      if (TWO) x1[u] = __builtin_nontemporal_load(base + ga * R + rA1);
-      // 32-bit offsets (xt_size * kRhs < 2^32, checked by the batched calls):
-      // no sign extension of the loaded offset sits between its load and here
-      const uint32_t zo = static_cast<uint32_t>(z[u]) * kRhs + r0;
-#pragma unroll
-      for (int s = 0; s < 4; ++s) bb[u][s] = XB[zo + s * kRhs];
-    }
-  };
-  auto compute = [&](int step, const flt4 (&x0)[KU], const flt4 (&x1)[KU],
-                     const float (&bb)[KU][4]) {
-#pragma unroll
-    for (int u = 0; u < KU; ++u) {
-      const bool ok = step * G + 2 * u + half < ng;
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const float bv = ok ? bb[u][s] : 0.0f;
-        acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(x0[u][s], bv, acc0, 0, 0, 0);
-        if (TWO) acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(x1[u][s], bv, acc1, 0, 0, 0);
-      }
-    }
-  };
-#pragma unroll
-  for (int k = 0; k < D; ++k)
-#pragma unroll
-    for (int u = 0; u < KU; ++u) zz[k][u] = gz(k, u);
-#pragma unroll
-  for (int k = 0; k < D; ++k) {
-    __builtin_amdgcn_sched_barrier(0);
-    load(k, zz[k], a0[k], a1[k], b[k]);
-#pragma unroll
-    for (int u = 0; u < KU; ++u) zz[k][u] = gz(k + D, u);
-  }
-  for (int s0 = 0; s0 < nsteps; s0 += D) {
-#pragma unroll
-    for (int j = 0; j < D; ++j) {
-      const int s = s0 + j;
-      __builtin_amdgcn_sched_barrier(0);
-      compute(s, a0[j], a1[j], b[j]);  // past the last step: B = 0, adds nothing
-      __builtin_amdgcn_sched_barrier(0);
-      load(s + D, zz[j], a0[j], a1[j], b[j]);
-#pragma unroll
-      for (int u = 0; u < KU; ++u) zz[j][u] = gz(s + 2 * D, u);
-    }
-  }
-  __builtin_amdgcn_sched_barrier(0);
-}
-
-// The load-order ring with the B operands staged through LDS: a column group's
-// four input rows (4 x kRhs floats, 512 contiguous bytes) arrive as one
-// 16-byte load per lane of its half-wave instead of four 4-byte loads per
-// lane, are written to the wave's LDS slot and read back in the MFMA layout
-// (row s, column lane % 32).  Steps go: MFMAs of step s (B in registers, read
-// from LDS the stage before), then step s + 1's B written to LDS and read
-// back, then the refill of step s + D.  One wave per workgroup, so the slot
-// is the wave's own; its LDS operations run in order, so a read sees the
-// write before it.
-template <int KU, int D, bool TWO>
-__device__ __forceinline__ void mfma_stream_lds(const flt4* __restrict__ base,
-                                                const int32_t* __restrict__ gi,
-                                                const float* __restrict__ XB, int ng, int R,
-                                                int half, int r0, float* slot, floatx16& acc0,
-                                                floatx16& acc1) {
-  constexpr int G = 2 * KU;  // groups per step
-  const int rA0 = min(r0, R - 1), rA1 = min(r0 + 32, R - 1);
-  const int nsteps = (ng + G - 1) / G;
-  flt4 a0[D][KU], a1[D][KU];
-  flt4 bq[D][KU];  // this lane's 16 bytes of the four input rows of group 2u + half
-  int zz[D][KU];    // input offset of group 2u + half for the step buffer k gets next
-  float bn[KU][4];  // B of the next step to multiply, read back from LDS
-  auto gz = [&](int step, int u) { return gi[min(step * G + 2 * u + half, ng - 1)]; };
-  auto load = [&](int step, const int (&z)[KU], flt4 (&x0)[KU], flt4 (&x1)[KU], flt4 (&bb)[KU]) {
-#pragma unroll
-    for (int u = 0; u < KU; ++u) {
-      const int ga = min(step * G + 2 * u + half, ng - 1);
-      x0[u] = __builtin_nontemporal_load(base + ga * R + rA0);
-      if (TWO) x1[u] = __builtin_nontemporal_load(base + ga * R + rA1);
-      // rows z .. z + 3 of XB are 512 contiguous, 128-byte aligned bytes
-      const uint32_t zo = static_cast<uint32_t>(z[u]) * kRhs + 4 * r0;
-      bb[u] = *reinterpret_cast<const flt4*>(XB + zo);
-    }
-  };
-  auto stage_b = [&](const flt4 (&bb)[KU]) {
-#pragma unroll
-    for (int u = 0; u < KU; ++u)
-      *reinterpret_cast<flt4*>(slot + (2 * u + half) * 4 * kRhs + 4 * r0) = bb[u];
-#pragma unroll
-    for (int u = 0; u < KU; ++u)
-#pragma unroll
-      for (int s = 0; s < 4; ++s) bn[u][s] = slot[(2 * u + half) * 4 * kRhs + s * kRhs + r0];
-  };
-  auto compute = [&](int step, const flt4 (&x0)[KU], const flt4 (&x1)[KU]) {
-#pragma unroll
-    for (int u = 0; u < KU; ++u) {
-      const bool ok = step * G + 2 * u + half < ng;
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const float bv = ok ? bn[u][s] : 0.0f;
-        acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(x0[u][s], bv, acc0, 0, 0, 0);
-        if (TWO) acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(x1[u][s], bv, acc1, 0, 0, 0);
-      }
-    }
-  };
-#pragma unroll
-  for (int k = 0; k < D; ++k)
-#pragma unroll
-    for (int u = 0; u < KU; ++u) zz[k][u] = gz(k, u);
-#pragma unroll
-  for (int k = 0; k < D; ++k) {
-    __builtin_amdgcn_sched_barrier(0);
-    load(k, zz[k], a0[k], a1[k], bq[k]);
-#pragma unroll
-    for (int u = 0; u < KU; ++u) zz[k][u] = gz(k + D, u);
-  }
-  __builtin_amdgcn_sched_barrier(0);
-  stage_b(bq[0]);
-  for (int s0 = 0; s0 < nsteps; s0 += D) {
-#pragma unroll
-    for (int j = 0; j < D; ++j) {
-      const int s = s0 + j;
-      __builtin_amdgcn_sched_barrier(0);
-      compute(s, a0[j], a1[j]);  // past the last step: B = 0, adds nothing
-      __builtin_amdgcn_sched_barrier(0);
-      stage_b(bq[(j + 1) % D]);
-      __builtin_amdgcn_sched_barrier(0);
-      load(s + D, zz[j], a0[j], a1[j], bq[j]);
-#pragma unroll
-      for (int u = 0; u < KU; ++u) zz[j][u] = gz(s + 2 * D, u);
-    }
-  }
-  __builtin_amdgcn_sched_barrier(0);
-}
-
-template <int PASS, int KU, bool PIPE, int D = 0, bool RING = false, bool LDSB = false>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_slab_mfma(
-    const bwl::WorkItem* __restrict__ wis, XcdSplit xs, const int32_t* __restrict__ gidx,
-    const float* __restrict__ data, const float* __restrict__ XB,
-    float* __restrict__ tout,              // pass 1
-    double* __restrict__ Y, int64_t yr, int64_t yc,  // pass 2 (row, column strides)
-    int nrhs, float* __restrict__ part, const int64_t* __restrict__ perm, int dof,
-    const int32_t* __restrict__ rowmap) {
-  const int lane = threadIdx.x & 63;
-  const int w = xcd_work_item<1>(xs);
-  if (w < 0) return;
-  const bwl::WorkItem wi = wis[w];
-  const int R = __builtin_amdgcn_readfirstlane(wi.rows);
-  const int ng = __builtin_amdgcn_readfirstlane(wi.ngroups);
-  const int half = lane >> 5;  // which group of the pair
-  const int r0 = lane & 31;
-  const flt4* __restrict__ base = reinterpret_cast<const flt4*>(data + wi.data_off);
-  const int32_t* __restrict__ gi = gidx + __builtin_amdgcn_readfirstlane(wi.gbeg);
-  floatx16 acc0 = {0}, acc1 = {0};
-  const bool two = R > 32;
-  if (ng > 0) {
-    if constexpr (LDSB) {
-      __shared__ __align__(16) float slot[2 * KU * 4 * kRhs];
-      if (two)
-        mfma_stream_lds<KU, D, true>(base, gi, XB, ng, R, half, r0, slot, acc0, acc1);
-      else
-        mfma_stream_lds<KU, D, false>(base, gi, XB, ng, R, half, r0, slot, acc0, acc1);
-    } else if constexpr (RING) {
-      if (two)
-        mfma_stream_ring<KU, D, true>(base, gi, XB, ng, R, half, r0, acc0, acc1);
-      else
-        mfma_stream_ring<KU, D, false>(base, gi, XB, ng, R, half, r0, acc0, acc1);
-    } else if constexpr (D > 0) {
-      if (two)
-        mfma_stream_deep<KU, D, true>(base, gi, XB, ng, R, half, r0, acc0, acc1);
-      else
-        mfma_stream_deep<KU, D, false>(base, gi, XB, ng, R, half, r0, acc0, acc1);
-    } else {
-      if (two)
-        mfma_stream<KU, PIPE, true>(base, gi, XB, ng, R, half, r0, acc0, acc1);
-      else
-        mfma_stream<KU, PIPE, false>(base, gi, XB, ng, R, half, r0, acc0, acc1);
-    }
-  }
-  const int n = lane & 31;
-  auto row_of = [&](int j) { return 8 * (j >> 2) + 4 * half + (j & 3); };
-  if (wi.part_off < 0) {
-    // 8 output rows at a time: their index loads (clamped rows, all in
-    // bounds, none behind a branch) go out together, then the stores, instead
-    // of one round trip per stored value
-    auto put8 = [&](int r0, int j0, const floatx16& acc) {
-      int idx[8], orow[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) idx[j] = wi.out_row + min(r0 + row_of(j0 + j), R - 1);
-      batched_rows<PASS>(idx, rowmap, perm, dof, orow);
-      if (n >= nrhs) return;
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        if (r0 + row_of(j0 + j) < R) batched_put<PASS>(tout, Y, yr, yc, orow[j], n, acc[j0 + j]);
-    };
-    put8(0, 0, acc0);
-    put8(0, 8, acc0);
-    if (two) {
-      put8(32, 0, acc1);
-      put8(32, 8, acc1);
-    }
-    return;
-  }
-  // partial sums of split slabs are added in order by k_reduce_b; they are
-  // read once, by it, so they are written (and read) nontemporally: about 1 %
-  // of a 32-RHS call on a 150 528-DoF operator, same values
-  float* pp = part + static_cast<int64_t>(wi.part_off) * kRhs;
-#pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    const int row = row_of(j);
-    if (row < R) __builtin_nontemporal_store(acc0[j], &pp[row * kRhs + n]);
-    if (two && 32 + row < R) __builtin_nontemporal_store(acc1[j], &pp[(32 + row) * kRhs + n]);
-  }
-}
-
-// The same product on v_mfma_f32_16x16x4f32 with 16-row tiles, so a slab of
-// R rows costs ceil(R / 16) tiles instead of 32 or 64 rows (pass-1 slabs of
-// 33-48 rows carry a third of their MFMA work as padding on 32-row tiles).
-// One k-step covers four column groups: lane l supplies A[i][k] with
-// i = l % 16 (row within the tile) and k = l / 16, i.e. element s of row i of
-// group 4 step + k is MFMA s's operand, and B[k][n] = XB[z(group) + s][n]
-// for n = l % 16 (+ 16 for the second 16 right-hand sides).  The same
-// 16-byte slab vectors are read as in the 32 x 32 kernel.  Loads run through
-// a ring of D step buffers in load order, as mfma_stream_ring; every tile's
-// rows are loaded (clamped, in bounds) and tiles past ceil(R / 16) skip their
-// MFMAs.  Accumulator element r of lane l is row 4 (l / 16) + r, column
-// l % 16 of its tile.
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-
-// The k-steps of k_slab_mfma16 for a slab of NT 16-row tiles (NT a template
-// argument, so the loop body is one basic block with the same waits on
-// every path).
-template <int NT, int D>
-__device__ __forceinline__ void mfma16_stream(const flt4* __restrict__ base,
-                                              const int32_t* __restrict__ gi,
-                                              const float* __restrict__ XB, int ng, int R, int kq,
-                                              int i16, floatx4 (&acc)[4][2]) {
-  int rowc[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) rowc[t] = min(16 * t + i16, R - 1);
-  const int nsteps = (ng + 3) >> 2;  // four groups per k-step
-  flt4 a[D][NT];
-  float b[D][2][4];
-  int zz[D];  // input offset of the step buffer q is refilled with next
-  auto gz = [&](int step) { return gi[min(4 * step + kq, ng - 1)]; };
-  auto load = [&](int step, int z, flt4 (&aa)[NT], float (&bb)[2][4]) {
-    const int ga = min(4 * step + kq, ng - 1);
-#pragma unroll
-    for (int t = 0; t < NT; ++t) aa[t] = __builtin_nontemporal_load(base + ga * R + rowc[t]);
-    const uint32_t zo = static_cast<uint32_t>(z) * kRhs + i16;  // < 2^32, checked
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      bb[0][s] = XB[zo + s * kRhs];
-      bb[1][s] = XB[zo + s * kRhs + 16];
-    }
-  };
-  auto compute = [&](int step, const flt4 (&aa)[NT], const float (&bb)[2][4]) {
-    const bool ok = 4 * step + kq < ng;
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const float b0 = ok ? bb[0][s] : 0.0f, b1 = ok ? bb[1][s] : 0.0f;
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(aa[t][s], b0, acc[t][0], 0, 0, 0);
-        acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(aa[t][s], b1, acc[t][1], 0, 0, 0);
-      }
-    }
-  };
-#pragma unroll
-  for (int q = 0; q < D; ++q) zz[q] = gz(q);
-#pragma unroll
-  for (int q = 0; q < D; ++q) {
-    __builtin_amdgcn_sched_barrier(0);
-    load(q, zz[q], a[q], b[q]);
-    zz[q] = gz(q + D);
-  }
-  for (int s0 = 0; s0 < nsteps; s0 += D) {
-#pragma unroll
-    for (int j = 0; j < D; ++j) {
-      const int st = s0 + j;
-      __builtin_amdgcn_sched_barrier(0);
-      compute(st, a[j], b[j]);  // past the last step: B = 0, adds nothing
-      __builtin_amdgcn_sched_barrier(0);
-      load(st + D, zz[j], a[j], b[j]);
-      zz[j] = gz(st + 2 * D);
-    }
-  }
-  __builtin_amdgcn_sched_barrier(0);
-}
-
-template <int PASS, int D>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(D > 3 ? 3 : 4))) void k_slab_mfma16(
-    const bwl::WorkItem* __restrict__ wis, XcdSplit xs, const int32_t* __restrict__ gidx,
-    const float* __restrict__ data, const float* __restrict__ XB,
-    float* __restrict__ tout,              // pass 1
-    double* __restrict__ Y, int64_t yr, int64_t yc,  // pass 2 (row, column strides)
-    int nrhs, float* __restrict__ part, const int64_t* __restrict__ perm, int dof,
-    const int32_t* __restrict__ rowmap) {
-  const int lane = threadIdx.x & 63;
-  const int w = xcd_work_item<1>(xs);
-  if (w < 0) return;
-  const bwl::WorkItem wi = wis[w];
-  const int R = wi.rows;
-  const int ng = wi.ngroups;
-  const int kq = lane >> 4, i16 = lane & 15;
-  const flt4* __restrict__ base = reinterpret_cast<const flt4*>(data + wi.data_off);
-  const int32_t* __restrict__ gi = gidx + wi.gbeg;
-  const int ntile = (R + 15) >> 4;  // wave-uniform
-  floatx4 acc[4][2];
-#pragma unroll
-  for (int t = 0; t < 4; ++t) acc[t][0] = acc[t][1] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-  if (ng > 0) {
-    switch (ntile) {
-      case 1: mfma16_stream<1, D>(base, gi, XB, ng, R, kq, i16, acc); break;
-      case 2: mfma16_stream<2, D>(base, gi, XB, ng, R, kq, i16, acc); break;
-      case 3: mfma16_stream<3, D>(base, gi, XB, ng, R, kq, i16, acc); break;
-      default: mfma16_stream<4, D>(base, gi, XB, ng, R, kq, i16, acc);
-    }
-  }
-  if (wi.part_off >= 0) {
-    float* pp = part + static_cast<int64_t>(wi.part_off) * kRhs;
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      if (t >= ntile) break;
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int row = 16 * t + 4 * kq + r;
-          if (row < R)  // added in order by k_reduce_b
-            __builtin_nontemporal_store(acc[t][h][r], &pp[row * kRhs + 16 * h + i16]);
-        }
-    }
-    return;
-  }
-  // two tiles (8 of this lane's rows) at a time: their output rows first
-  // (clamped, in bounds, no branch), so the index loads go out together
-#pragma unroll
-  for (int t0 = 0; t0 < 4; t0 += 2) {
-    if (t0 >= ntile) break;
-    int idx[8], orow[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) idx[j] = wi.out_row + min(16 * (t0 + (j >> 2)) + 4 * kq + (j & 3), R - 1);
-    batched_rows<PASS>(idx, rowmap, perm, dof, orow);
-#pragma unroll
-    for (int t = t0; t < t0 + 2; ++t)
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int row = 16 * t + 4 * kq + r;
-          const int n = 16 * h + i16;
-          if (row < R && n < nrhs)
-            batched_put<PASS>(tout, Y, yr, yc, orow[4 * (t - t0) + r], n, acc[t][h][r]);
-        }
-  }
-}
-
-template <int PASS>
-void launch_mfma(int schedule, int blocks, hipStream_t st, const bwl::WorkItem* wis, XcdSplit xs,
-                 const int32_t* gidx, const float* data, const float* XB, float* tout, double* Y,
-                 int64_t yr, int64_t yc, int nrhs, float* part, const int64_t* perm, int dof,
-                 const int32_t* rowmap) {
-  switch (schedule) {
-    case 1:
-      hipLaunchKernelGGL((k_slab_mfma<PASS, 2, true>), dim3(4 * blocks), dim3(64), 0, st, wis, xs,
-                         gidx, data, XB, tout, Y, yr, yc, nrhs, part, perm, dof, rowmap);
-      break;
-    case 2:
-      hipLaunchKernelGGL((k_slab_mfma<PASS, 4, true>), dim3(4 * blocks), dim3(64), 0, st, wis, xs,
-                         gidx, data, XB, tout, Y, yr, yc, nrhs, part, perm, dof, rowmap);
-      break;
-    case 3:
-      hipLaunchKernelGGL((k_slab_mfma<PASS, 8, false>), dim3(4 * blocks), dim3(64), 0, st, wis, xs,
-                         gidx, data, XB, tout, Y, yr, yc, nrhs, part, perm, dof, rowmap);
-      break;
-    case 4:
-      hipLaunchKernelGGL((k_slab_mfma<PASS, 2, true, 3>), dim3(4 * blocks), dim3(64), 0, st, wis, xs,
-                         gidx, data, XB, tout, Y, yr, yc, nrhs, part, perm, dof, rowmap);
-      break;
-    case 5:
-      hipLaunchKernelGGL((k_slab_mfma<PASS, 2, true, 4>), dim3(4 * blocks), dim3(64), 0, st, wis, xs,
-                         gidx, data, XB, tout, Y, yr, yc, nrhs, part, perm, dof, rowmap);
-      break;
-    case 6:
-      hipLaunchKernelGGL((k_slab_mfma<PASS, 1, true, 6>), dim3(4 * blocks), dim3(64), 0, st, wis, xs,
-                         gidx, data, XB, tout, Y, yr, yc, nrhs, part, perm, dof, rowmap);
-      break;
-    case 7:
-      hipLaunchKernelGGL((k_slab_mfma<PASS, 1, true, 8>), dim3(4 * blocks), dim3(64), 0, st, wis, xs,
-                         gidx, data, XB, tout, Y, yr, yc, nrhs, part, perm, dof, rowmap);
-      break;
-#define BW_MFMA32_RING(KU, D)                                                              \
-  hipLaunchKernelGGL((k_slab_mfma<PASS, KU, true, D, true>), dim3(4 * blocks), dim3(64), 0, st, \
-                     wis, xs, gidx, data, XB, tout, Y, yr, yc, nrhs, part, perm, dof, rowmap)
-    case 8: BW_MFMA32_RING(2, 3); break;
-    case 9: BW_MFMA32_RING(2, 4); break;
-    case 10: BW_MFMA32_RING(1, 6); break;
-    case 11: BW_MFMA32_RING(1, 8); break;
-#undef BW_MFMA32_RING
-#define BW_MFMA32_LDSB(KU, D)                                                                    \
-  hipLaunchKernelGGL((k_slab_mfma<PASS, KU, true, D, true, true>), dim3(4 * blocks), dim3(64), 0, \
-                     st, wis, xs, gidx, data, XB, tout, Y, yr, yc, nrhs, part, perm, dof, rowmap)
-    case 14: BW_MFMA32_LDSB(2, 3); break;
-    case 15: BW_MFMA32_LDSB(2, 4); break;
-#undef BW_MFMA32_LDSB
-    case 12:
-      hipLaunchKernelGGL((k_slab_mfma16<PASS, 3>), dim3(4 * blocks), dim3(64), 0, st, wis, xs, gidx,
-                         data, XB, tout, Y, yr, yc, nrhs, part, perm, dof, rowmap);
-      break;
-    case 13:
-      hipLaunchKernelGGL((k_slab_mfma16<PASS, 4>), dim3(4 * blocks), dim3(64), 0, st, wis, xs, gidx,
-                         data, XB, tout, Y, yr, yc, nrhs, part, perm, dof, rowmap);
-      break;
-    default:
-      hipLaunchKernelGGL((k_slab_mfma<PASS, 4, false>), dim3(4 * blocks), dim3(64), 0, st, wis, xs,
-                         gidx, data, XB, tout, Y, yr, yc, nrhs, part, perm, dof, rowmap);
-  }
-}
-
-template <int PASS, typename T>
-__global__ __launch_bounds__(256) void k_reduce_b(const bwl::Reduce* __restrict__ reds, int nred,
-                                                  const T* __restrict__ part, T* tout,
-                                                  double* Y, int64_t yr, int64_t yc, int nrhs,
-                                                  const int64_t* __restrict__ perm, int dof,
-                                                  const int32_t* __restrict__ rowmap) {
-  // one workgroup per split slab; a thread sums one 16-byte vector of
-  // right-hand sides of one row over the parts, in part order, four parts in
-  // flight (nontemporal loads: each partial row is read once)
-  typedef typename Vec<T>::type VT;
-  constexpr int VW = Vec<T>::V;
-  const int r = blockIdx.x;
-  if (r >= nred) return;
-  const bwl::Reduce rd = reds[r];
-  const VT* __restrict__ base_p =
-      reinterpret_cast<const VT*>(part + static_cast<int64_t>(rd.part_off) * kRhs);
-  const int nvec = rd.rows * (kRhs / VW);
-  const int64_t stride = static_cast<int64_t>(rd.rows) * (kRhs / VW);
-  for (int e = threadIdx.x; e < nvec; e += blockDim.x) {
-    VT sum = {};
-    int q = 0;
-    for (; q + 4 <= rd.nparts; q += 4) {
-      const VT a = __builtin_nontemporal_load(&base_p[(q + 0) * stride + e]);
-      const VT b = __builtin_nontemporal_load(&base_p[(q + 1) * stride + e]);
-      const VT c = __builtin_nontemporal_load(&base_p[(q + 2) * stride + e]);
-      const VT d = __builtin_nontemporal_load(&base_p[(q + 3) * stride + e]);
-      sum += a;
-      sum += b;
-      sum += c;
-      sum += d;
-    }
-    for (; q < rd.nparts; ++q) sum += __builtin_nontemporal_load(&base_p[q * stride + e]);
-    const int row = e / (kRhs / VW);
-    const int n0 = (e % (kRhs / VW)) * VW;
-    if (PASS == 1) {
-      *reinterpret_cast<VT*>(tout + static_cast<int64_t>(rowmap[rd.out_row + row]) * kRhs + n0) =
-          sum;
-    } else {
-      const int64_t o = out_index<double>(static_cast<int64_t>(rd.out_row) + row, perm, dof);
-#pragma unroll
-      for (int k = 0; k < VW; ++k)
-        if (n0 + k < nrhs) Y[o * yr + (n0 + k) * yc] = static_cast<double>(sum[k]);
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Many right-hand sides in FP64 on MFMA (v_mfma_f64_16x16x4f64), on the FP64
-// slab layout data[g][row][v] (V = 2).  One k-step covers two column groups
-// (4 columns): lane l supplies A[i][k] with i = l % 16 (row within a 16-row
-// tile) and k = l / 16, i.e. column k % 2 of group g0 + k / 2, and
-// B[k][n] = XB[z(g0 + k / 2) + k % 2][n] with n = l % 16 (+ 16 for the second
-// column tile).  Element r of a lane's accumulator is row l / 16 + 4 r,
-// column l % 16 (measured on gfx950 with one-hot operands).  Rows past R read a clamped row and are never stored; groups
-// past the end get B = 0.
-typedef double dblx4 __attribute__((ext_vector_type(4)));
-
-// D > 0: the k-steps run through a ring of D register buffers (as in
-// mfma_stream_deep), D - 1 steps of loads in flight; D = 0: two steps loaded,
-// then their MFMAs.  Both issue the same MFMAs in the same order per
-// accumulator, so the results agree bit for bit.
-template <int PASS, int D, bool RING = false>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(D > 4 ? 2 : (D > 0 ? 3 : 4)))) void k_slab_mfma64(
-    const bwl::WorkItem* __restrict__ wis, XcdSplit xs, const int32_t* __restrict__ gidx,
-    const double* __restrict__ data, const double* __restrict__ XB,
-    double* __restrict__ tout,             // pass 1
-    double* __restrict__ Y, int64_t yr, int64_t yc,  // pass 2 (row, column strides)
-    int nrhs, double* __restrict__ part, const int64_t* __restrict__ perm, int dof,
-    const int32_t* __restrict__ rowmap) {
-  const int lane = threadIdx.x & 63;
-  const int w = xcd_work_item<1>(xs);
-  if (w < 0) return;
-  const bwl::WorkItem wi = wis[w];
-  const int R = wi.rows;
-  const int ng = wi.ngroups;
-  const int k = lane >> 4, i16 = lane & 15;
-  const int gsub = k >> 1, v = k & 1;
-  const double* __restrict__ base = data + wi.data_off;
-  const int32_t* __restrict__ gi = gidx + wi.gbeg;
-  const int ntile = (R + 15) >> 4;  // 16-row tiles in use, wave-uniform
-  dblx4 acc[4][2];
-#pragma unroll
-  for (int t = 0; t < 4; ++t) acc[t][0] = acc[t][1] = dblx4{0.0, 0.0, 0.0, 0.0};
-  int rowc[4];
-#pragma unroll
-  for (int t = 0; t < 4; ++t) rowc[t] = min(16 * t + i16, R - 1);
-  if constexpr (D > 0) {
-    const int nsteps = (ng + 1) >> 1;  // two groups per k-step
-    double a[D][4], b[D][2];
-    int zz[D];  // input offset of the next step to be loaded into each buffer
-    auto gz = [&](int step) { return gi[min(2 * step + gsub, ng - 1)]; };
-    auto load = [&](int step, int z, double (&aa)[4], double (&bb)[2]) {
-      const int ga = min(2 * step + gsub, ng - 1);
-      const double* __restrict__ gp = base + static_cast<int64_t>(ga) * R * 2 + v;
-#pragma unroll
-      // every tile loads (rows clamped into the slab, in bounds) so that the
-      // loads, and hence the waits, are the same on every path; tiles past
-      // ntile are never multiplied
-      for (int t = 0; t < 4; ++t) aa[t] = gp[rowc[t] * 2];
-      const uint32_t zr = static_cast<uint32_t>(z + v) * kRhs + i16;  // < 2^32, checked
-      bb[0] = XB[zr];
-      bb[1] = XB[zr + 16];
-    };
-    auto compute = [&](int step, const double (&aa)[4], const double (&bb)[2]) {
-      const bool ok = 2 * step + gsub < ng;
-      const double b0 = ok ? bb[0] : 0.0, b1 = ok ? bb[1] : 0.0;
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-        if (t < ntile) {
-          acc[t][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(aa[t], b0, acc[t][0], 0, 0, 0);
-          acc[t][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(aa[t], b1, acc[t][1], 0, 0, 0);
-        }
-    };
-#pragma unroll
-    for (int q = 0; q < D; ++q) zz[q] = gz(q);
-    if constexpr (RING) {
-      // buffers consumed in the order they were loaded (as mfma_stream_ring):
-      // compute buffer j, then refill it with the step D ahead
-#pragma unroll
-      for (int q = 0; q < D; ++q) {
-        __builtin_amdgcn_sched_barrier(0);
-        load(q, zz[q], a[q], b[q]);
-        zz[q] = gz(q + D);
-      }
-      for (int s0 = 0; s0 < nsteps; s0 += D) {
-#pragma unroll
-        for (int j = 0; j < D; ++j) {
-          const int st = s0 + j;
-          __builtin_amdgcn_sched_barrier(0);
-          compute(st, a[j], b[j]);  // past the last step: B = 0, adds nothing
-          __builtin_amdgcn_sched_barrier(0);
-          load(st + D, zz[j], a[j], b[j]);
-          zz[j] = gz(st + 2 * D);
-        }
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    } else {
-#pragma unroll
-    for (int q = 0; q < D - 1; ++q) {
-      load(q, zz[q], a[q], b[q]);
-      zz[q] = gz(q + D);
-    }
-    for (int s0 = 0; s0 < nsteps; s0 += D) {
-#pragma unroll
-      for (int j = 0; j < D; ++j) {
-        const int st = s0 + j;
-        const int q = (j + D - 1) % D;  // buffer freed by the previous stage
-        load(st + D - 1, zz[q], a[q], b[q]);
-        zz[q] = gz(st + 2 * D - 1);
-        __builtin_amdgcn_sched_barrier(0);
-        if (st < nsteps) compute(st, a[j], b[j]);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-    }
-  } else {
-  constexpr int S = 2;  // k-steps (two groups each) loaded before their MFMAs
-  for (int g0 = 0; g0 < ng; g0 += 2 * S) {
-    double a[S][4], b[S][2];
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-      const int gg = g0 + 2 * s + gsub;
-      const bool ok = gg < ng;
-      const int ga = min(gg, ng - 1);
-      const double* __restrict__ gp = base + static_cast<int64_t>(ga) * R * 2 + v;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) a[s][t] = t < ntile ? gp[rowc[t] * 2] : 0.0;
-      const int64_t zr = static_cast<int64_t>(gi[ga] + v) * kRhs;
-      const double b0 = XB[zr + i16], b1 = XB[zr + 16 + i16];
-      b[s][0] = ok ? b0 : 0.0;
-      b[s][1] = ok ? b1 : 0.0;
-    }
-#pragma unroll
-    for (int s = 0; s < S; ++s)
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-        if (t < ntile) {
-          acc[t][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s][t], b[s][0], acc[t][0], 0, 0, 0);
-          acc[t][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s][t], b[s][1], acc[t][1], 0, 0, 0);
-        }
-  }
-  }
-  if (wi.part_off >= 0) {
-    double* pp = part + static_cast<int64_t>(wi.part_off) * kRhs;
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      if (t >= ntile) break;
-#pragma unroll
-      for (int c = 0; c < 2; ++c)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int row = 16 * t + k + 4 * r;
-          if (row < R)  // added in order by k_reduce_b
-            __builtin_nontemporal_store(acc[t][c][r], &pp[row * kRhs + 16 * c + i16]);
-        }
-    }
-    return;
-  }
-  // two tiles (8 of this lane's rows) at a time: their output rows first
-  // (clamped, in bounds, no branch), so the index loads go out together, then
-  // the stores
-#pragma unroll
-  for (int t0 = 0; t0 < 4; t0 += 2) {
-    if (t0 >= ntile) break;
-    int idx[8], orow[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) idx[j] = wi.out_row + min(16 * (t0 + (j >> 2)) + k + 4 * (j & 3), R - 1);
-    batched_rows<PASS>(idx, rowmap, perm, dof, orow);
-#pragma unroll
-    for (int t = t0; t < t0 + 2; ++t)
-#pragma unroll
-      for (int c = 0; c < 2; ++c)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int row = 16 * t + k + 4 * r;
-          const int n = 16 * c + i16;
-          if (row < R && n < nrhs)
-            batched_put<PASS>(tout, Y, yr, yc, orow[4 * (t - t0) + r], n, acc[t][c][r]);
-        }
-  }
-}
-
-template <int PASS>
-void launch_mfma64(int schedule, int blocks, hipStream_t st, const bwl::WorkItem* wis, XcdSplit xs,
-                   const int32_t* gidx, const double* data, const double* XB, double* tout,
-                   double* Y, int64_t yr, int64_t yc, int nrhs, double* part,
-                   const int64_t* perm, int dof, const int32_t* rowmap) {
-#define BW_MFMA64(D)                                                                        \
-  hipLaunchKernelGGL((k_slab_mfma64<PASS, D>), dim3(4 * blocks), dim3(64), 0, st, wis, xs, gidx, \
-                     data, XB, tout, Y, yr, yc, nrhs, part, perm, dof, rowmap)
-#define BW_MFMA64R(D)                                                                         \
-  hipLaunchKernelGGL((k_slab_mfma64<PASS, D, true>), dim3(4 * blocks), dim3(64), 0, st, wis, xs, \
-                     gidx, data, XB, tout, Y, yr, yc, nrhs, part, perm, dof, rowmap)
-  switch (schedule) {
-    case 4: BW_MFMA64(3); break;
-    case 5: BW_MFMA64(4); break;
-    case 6: BW_MFMA64(6); break;
-    case 7: BW_MFMA64(8); break;
-    case 8: BW_MFMA64R(3); break;
-    case 9: BW_MFMA64R(4); break;
-    case 10: BW_MFMA64R(6); break;
-    case 11: BW_MFMA64R(8); break;
-    case 12: BW_MFMA64R(3); break;  // the FP64 kernel has 16-row tiles already
-    case 13: BW_MFMA64R(4); break;
-    case 14: BW_MFMA64R(3); break;  // FP32-only B staging: the FP64 ring
-    case 15: BW_MFMA64R(4); break;
-    default: BW_MFMA64(0);
-  }
-#undef BW_MFMA64
-#undef BW_MFMA64R
-}
+constexpr int kRhs = 32;        // right-hand sides per round of the batched product
+// Waves per workgroup of the batched kernels: 8 are 4-15 % slower (32 right-hand
+// sides, FP64, 24 300 DoF: 307 us against 293; FP32, 49 152 DoF: 357 / 331).
+constexpr int kBatchWaves = 4;
 
 // ---------------------------------------------------------------------------
 
-struct DevPass {
+// One work-item list of a pass on the device.
+struct DevItems {
   bwl::WorkItem* wis = nullptr;
-  int32_t* gidx = nullptr;
-  int32_t* rowmap = nullptr;        // pass 1: t entry of every slab row
-  bwl::Reduce* reds = nullptr;      // one per split slab
-  void* data = nullptr;
+  bwl::Reduce* reds = nullptr;  // one per split slab
   int nwi = 0, nred = 0;
   XcdSplit xs = {};
-  int blocks = 0;  // workgroups of a slab launch
+  int blocks = 0;               // workgroups of a launch
+  int64_t part_elems = 0;
+};
+
+struct DevPass {
+  DevItems single, batched;
+  int32_t* gidx = nullptr;
+  int32_t* rowmap = nullptr;  // pass 1: t entry of every slab row
+  void* data = nullptr;
   int64_t data_bytes = 0;
 };
 
@@ -1321,9 +102,7 @@ struct DevOp {
   const int64_t* perm_in = nullptr;   // device, n_in / dof
   const int64_t* perm_out = nullptr;  // device, n_out / dof
   int64_t stream_bytes = 0;
-  int64_t part_elems[2] = {0, 0};
-  int unroll[2] = {16, 16};   // loads in flight per lane in k_slab (4, 8 or 16), per pass
-  int mfma_schedule = 0;      // k_slab_mfma / k_slab_mfma64 variant (0-15)
+  int unroll[2] = {8, 8};     // loads in flight per lane in k_slab (4, 8 or 16), per pass
 };
 
 // What one matvec of an operator writes: xt (x gathered in the factor
@@ -1391,31 +170,43 @@ int host_pinned_alloc(void** p, size_t bytes, const char* what) {
   return BW_OK;
 }
 
-// Work-item bytes for the next create; 0 = sized from the matrix (auto_wi_bytes).
+// Work-item bytes for the next create; 0 = sized from the matrix (layout.cpp).
 std::atomic<int64_t> g_wi_bytes64{0};
 std::atomic<int64_t> g_wi_bytes32{0};
 std::atomic<int> g_stack_rows{64};
 // Relative tolerance of the FP32 copy's low-rank recompression (0: off).
 std::atomic<double> g_fp32_rank_tol{0.0};
 
-// About 32k work items: a few rounds of 8 waves on each of the 1024 SIMDs,
-// capped where a sweep of the 600k-DoF 3DT0 matrix on MI355X stopped gaining
-// (384 KiB for FP64, 192 KiB for FP32) and floored at 8 KiB for small matrices.
-int64_t auto_wi_bytes(int64_t entries, int elem_bytes) {
-  const int64_t cap = elem_bytes == 8 ? (384 << 10) : (192 << 10);
-  return std::min<int64_t>(cap, std::max<int64_t>(8 << 10, entries * elem_bytes / 32768));
+int upload_items(const bwl::ItemList& il, DevItems* di, std::vector<void*>* allocs) {
+  di->nwi = static_cast<int>(il.wis.size());
+  di->nred = static_cast<int>(il.reds.size());
+  di->part_elems = il.part_elems;
+  int most = 0;
+  for (int x = 0; x < bwl::kXcds; ++x) most = std::max(most, il.xcd[x + 1] - il.xcd[x]);
+  for (int x = 0; x <= bwl::kXcds; ++x) di->xs.s[x] = il.xcd[x];
+  di->blocks = bwl::kXcds * most;
+  int rc;
+  if ((rc = dev_alloc(reinterpret_cast<void**>(&di->wis), il.wis.size() * sizeof(bwl::WorkItem),
+                      allocs, "create")) ||
+      (rc = dev_alloc(reinterpret_cast<void**>(&di->reds), il.reds.size() * sizeof(bwl::Reduce),
+                      allocs, "create")))
+    return rc;
+  if (!il.wis.empty())
+    HIPCHK(hipMemcpy(di->wis, il.wis.data(), il.wis.size() * sizeof(bwl::WorkItem),
+                     hipMemcpyHostToDevice));
+  if (!il.reds.empty())
+    HIPCHK(hipMemcpy(di->reds, il.reds.data(), il.reds.size() * sizeof(bwl::Reduce),
+                     hipMemcpyHostToDevice));
+  return BW_OK;
 }
 
 template <typename T>
 int upload_pass(const bwl::Layout& L, const bwl::Program& P, DevPass* dp, hipStream_t st,
                 std::vector<void*>* allocs) {
-  dp->nwi = static_cast<int>(P.wis.size());
-  for (int x = 0; x <= bwl::kXcds; ++x) dp->xs.s[x] = P.xcd[x];
-  dp->blocks = P.xcd_blocks;
-  dp->nred = static_cast<int>(P.reds.size());
   auto dalloc = [&](void** p, size_t bytes) -> int { return dev_alloc(p, bytes, allocs, "create"); };
   int rc;
-  if ((rc = dalloc(reinterpret_cast<void**>(&dp->wis), P.wis.size() * sizeof(bwl::WorkItem))))
+  if ((rc = upload_items(P.single, &dp->single, allocs)) ||
+      (rc = upload_items(P.batched, &dp->batched, allocs)))
     return rc;
   if ((rc = dalloc(reinterpret_cast<void**>(&dp->gidx), P.gidx.size() * sizeof(int32_t)))) return rc;
   if (!P.rowmap.empty()) {
@@ -1424,16 +215,10 @@ int upload_pass(const bwl::Layout& L, const bwl::Program& P, DevPass* dp, hipStr
     HIPCHK(hipMemcpy(dp->rowmap, P.rowmap.data(), P.rowmap.size() * sizeof(int32_t),
                      hipMemcpyHostToDevice));
   }
-  if ((rc = dalloc(reinterpret_cast<void**>(&dp->reds), P.reds.size() * sizeof(bwl::Reduce))))
-    return rc;
   dp->data_bytes = P.data_elems * static_cast<int64_t>(sizeof(T));
   if ((rc = dalloc(&dp->data, static_cast<size_t>(dp->data_bytes)))) return rc;
-  if (!P.wis.empty())
-    HIPCHK(hipMemcpy(dp->wis, P.wis.data(), P.wis.size() * sizeof(bwl::WorkItem), hipMemcpyHostToDevice));
   if (!P.gidx.empty())
     HIPCHK(hipMemcpy(dp->gidx, P.gidx.data(), P.gidx.size() * sizeof(int32_t), hipMemcpyHostToDevice));
-  if (!P.reds.empty())
-    HIPCHK(hipMemcpy(dp->reds, P.reds.data(), P.reds.size() * sizeof(bwl::Reduce), hipMemcpyHostToDevice));
   // data: fill slabs into pinned staging chunks and stream them up
   const int32_t nslab = static_cast<int32_t>(P.slabs.size());
   if (nslab == 0) return BW_OK;
@@ -1588,18 +373,6 @@ int build_op(bw_hip_handle* hd, const bw_flat_hmat* h, bool adjoint, hipStream_t
   opt.elem_bytes = sizeof(T);
   opt.wi_bytes = sizeof(T) == 8 ? g_wi_bytes64.load() : g_wi_bytes32.load();
   opt.stack_rows = g_stack_rows.load();
-  if (opt.wi_bytes == 0) {
-    int64_t E = 0;
-    for (int64_t k = 0; k < h->n_fr; ++k) {
-      const int64_t* c = h->fr_pattern + 6 * k;
-      E += h->dof * (c[3] - c[1]) * h->dof * (c[4] - c[2]);
-    }
-    for (int64_t k = 0; k < h->n_lr; ++k) {
-      const int64_t* c = h->lr_pattern + 6 * k;
-      E += c[5] * h->dof * ((c[3] - c[1]) + (c[4] - c[2]));
-    }
-    opt.wi_bytes = auto_wi_bytes(E, sizeof(T));
-  }
   bwl::Layout L;
   bwl::build_layout(view, opt, &L);
   std::string msg;
@@ -1608,10 +381,6 @@ int build_op(bw_hip_handle* hd, const bw_flat_hmat* h, bool adjoint, hipStream_t
   if ((rc = upload_pass<T>(L, L.pass1, &op.p1, st, &hd->allocs))) return rc;
   if ((rc = upload_pass<T>(L, L.pass2, &op.p2, st, &hd->allocs))) return rc;
   op.elem = sizeof(T);
-  // default batched schedule: the fastest on MI355X for the 150k-DoF 3DR0
-  // matrix (FP32: two pairs, load-order ring of 3, B staged through LDS;
-  // FP64: ring of 4)
-  op.mfma_schedule = sizeof(T) == 8 ? 5 : 14;
   op.xt_size = L.xt_size;
   op.xt_t = L.xt_t;
   op.t_total = L.view.t_total;
@@ -1620,11 +389,10 @@ int build_op(bw_hip_handle* hd, const bw_flat_hmat* h, bool adjoint, hipStream_t
   op.perm_in = adjoint ? hd->perm0 : hd->perm1;
   op.perm_out = adjoint ? hd->perm1 : hd->perm0;
   op.stream_bytes = (L.pass1.data_elems + L.pass2.data_elems) * static_cast<int64_t>(sizeof(T));
-  op.part_elems[0] = L.pass1.part_elems;
-  op.part_elems[1] = L.pass2.part_elems;
   hd->device_bytes += op.p1.data_bytes + op.p2.data_bytes + L.xt_size * sizeof(T) +
-                      (L.pass1.part_elems + L.pass2.part_elems) * sizeof(T) +
-                      (L.pass1.wis.size() + L.pass2.wis.size()) * sizeof(bwl::WorkItem) +
+                      (L.pass1.single.part_elems + L.pass2.single.part_elems) * sizeof(T) +
+                      (op.p1.single.nwi + op.p1.batched.nwi + op.p2.single.nwi + op.p2.batched.nwi) *
+                          sizeof(bwl::WorkItem) +
                       (L.pass1.gidx.size() + L.pass2.gidx.size()) * sizeof(int32_t);
   op.present = true;
   return BW_OK;
@@ -1661,9 +429,13 @@ int ensure_op_scratch(bw_hip_handle* hd, StreamCtx* ctx, int adj, int fp32, bool
   if (!s.xt) {
     void* xt = nullptr;
     void* part[2] = {nullptr, nullptr};
-    if ((rc = dev_alloc(&xt, op.xt_size * es, &ctx->allocs, "scratch"))) return undo_allocs(ctx, mark, rc);
+    // whole 2 MiB pages, so that no other allocation shares a page with the
+    // vectors that this stream's kernels write
+    const size_t pages = (op.xt_size * es + (size_t(2) << 20) - 1) >> 21;
+    if ((rc = dev_alloc(&xt, pages << 21, &ctx->allocs, "scratch"))) return undo_allocs(ctx, mark, rc);
     for (int p = 0; p < 2; ++p)
-      if ((rc = dev_alloc(&part[p], op.part_elems[p] * es, &ctx->allocs, "scratch")))
+      if ((rc = dev_alloc(&part[p], (p ? op.p2 : op.p1).single.part_elems * es, &ctx->allocs,
+                          "scratch")))
         return undo_allocs(ctx, mark, rc);
     const hipError_t e = zero_now(xt, op.xt_size * es);
     if (e != hipSuccess)
@@ -1679,8 +451,8 @@ int ensure_op_scratch(bw_hip_handle* hd, StreamCtx* ctx, int adj, int fp32, bool
     if ((rc = dev_alloc(&xb, static_cast<size_t>(op.xt_size) * kRhs * es, &ctx->allocs, "scratch")))
       return undo_allocs(ctx, mark_b, rc);
     for (int p = 0; p < 2; ++p)
-      if ((rc = dev_alloc(&partb[p], static_cast<size_t>(op.part_elems[p]) * kRhs * es, &ctx->allocs,
-                          "scratch")))
+      if ((rc = dev_alloc(&partb[p], static_cast<size_t>((p ? op.p2 : op.p1).batched.part_elems) * kRhs * es,
+                          &ctx->allocs, "scratch")))
         return undo_allocs(ctx, mark_b, rc);
     const hipError_t e = zero_now(xb, static_cast<size_t>(op.xt_size) * kRhs * es);
     if (e != hipSuccess)
@@ -1751,21 +523,24 @@ void compute_diagonal(bw_hip_handle* hd, const bw_flat_hmat* h) {
 }
 
 template <typename T, typename OutT, int PASS>
-void launch_slab(int unroll, int blocks, hipStream_t st, const bwl::WorkItem* wis, XcdSplit xs,
-                 const int32_t* gidx, const T* data, const T* xin, OutT* out, T* part,
-                 const int64_t* perm, int dof, const int32_t* rowmap) {
-  // `blocks` counts four-wave workgroups (the layout's XCD split); k_slab
-  // runs one wave per workgroup
-  constexpr int kWavesPerGroup = 4;
+void launch_slab(const DevPass& dp, int unroll, hipStream_t st, const T* xin, OutT* out, T* part,
+                 const int64_t* perm, int dof) {
+  // 8 waves per workgroup: 4 leave more small workgroups to start and end (the
+  // 120 000-DoF 3DR0 operator: pass 1 545 us against 509, pass 2 647 / 638),
+  // 16 leave one workgroup per compute unit (mode-1, 25 600 DoF: 44 us / 39).
+  // Two buffers of 8 loads; 16 leave a third fewer waves and are slower
+  // everywhere (pass 1: 550 us), so an unroll of 16 runs as 8.
+  constexpr int W = 8;
+  const DevItems& di = dp.single;
+#define BW_SLAB(U)                                                                              \
+  hipLaunchKernelGGL((k_slab<T, OutT, U, PASS, W>), dim3(di.blocks), dim3(64 * W), 0, st, di.wis, \
+                     di.xs, dp.gidx, static_cast<const T*>(dp.data), xin, out, part, perm, dof,  \
+                     dp.rowmap)
   if (unroll == 4)
-    hipLaunchKernelGGL((k_slab<T, OutT, 4, PASS>), dim3(kWavesPerGroup * blocks), dim3(64), 0,
-                       st, wis, xs, gidx, data, xin, out, part, perm, dof, rowmap);
-  else if (unroll == 16)
-    hipLaunchKernelGGL((k_slab<T, OutT, 16, PASS>), dim3(kWavesPerGroup * blocks), dim3(64), 0,
-                       st, wis, xs, gidx, data, xin, out, part, perm, dof, rowmap);
+    BW_SLAB(4);
   else
-    hipLaunchKernelGGL((k_slab<T, OutT, 8, PASS>), dim3(kWavesPerGroup * blocks), dim3(64), 0,
-                       st, wis, xs, gidx, data, xin, out, part, perm, dof, rowmap);
+    BW_SLAB(8);
+#undef BW_SLAB
 }
 
 // Zero fill of xt's gap after x and its tail after t, for scratch that other
@@ -1809,25 +584,22 @@ int launch_matvec(bw_hip_handle* hd, DevOp& op, const OpScratch& s, double* y_fu
                        orig ? op.perm_in : nullptr, dof);
   }
   if (timing) (void)hipEventRecord(hd->ev[1], st);
-  if (op.p1.nwi > 0) {
-    launch_slab<T, T, 1>(op.unroll[0], op.p1.blocks, st, op.p1.wis, op.p1.xs, op.p1.gidx,
-                         static_cast<const T*>(op.p1.data), xt, xt, part1, nullptr, dof,
-                         op.p1.rowmap);
+  if (op.p1.single.nwi > 0) {
+    launch_slab<T, T, 1>(op.p1, op.unroll[0], st, xt, xt, part1, nullptr, dof);
   }
   if (timing) (void)hipEventRecord(hd->ev[2], st);
-  if (op.p1.nred > 0)
-    hipLaunchKernelGGL((k_reduce<T, T>), dim3(op.p1.nred), dim3(64), 0, st, op.p1.reds,
-                       op.p1.nred, part1, xt, nullptr, dof, op.p1.rowmap);
+  if (op.p1.single.nred > 0)
+    hipLaunchKernelGGL((k_reduce<T, T>), dim3(op.p1.single.nred), dim3(64), 0, st,
+                       op.p1.single.reds, op.p1.single.nred, part1, xt, nullptr, dof, op.p1.rowmap);
   if (timing) (void)hipEventRecord(hd->ev[3], st);
-  if (op.p2.nwi > 0) {
-    launch_slab<T, double, 2>(op.unroll[1], op.p2.blocks, st, op.p2.wis, op.p2.xs, op.p2.gidx,
-                              static_cast<const T*>(op.p2.data), xt, yd, part2,
-                              orig ? op.perm_out : nullptr, dof, nullptr);
+  if (op.p2.single.nwi > 0) {
+    launch_slab<T, double, 2>(op.p2, op.unroll[1], st, xt, yd, part2, orig ? op.perm_out : nullptr,
+                              dof);
   }
   if (timing) (void)hipEventRecord(hd->ev[4], st);
-  if (op.p2.nred > 0)
-    hipLaunchKernelGGL((k_reduce<T, double>), dim3(op.p2.nred), dim3(64), 0, st, op.p2.reds,
-                       op.p2.nred, part2, yd, orig ? op.perm_out : nullptr, dof, nullptr);
+  if (op.p2.single.nred > 0)
+    hipLaunchKernelGGL((k_reduce<T, double>), dim3(op.p2.single.nred), dim3(64), 0, st,
+                       op.p2.single.reds, op.p2.single.nred, part2, yd, orig ? op.perm_out : nullptr, dof, nullptr);
   if (sd && sd->n_out > 0) {
     const int blocks = static_cast<int>((sd->n_out * dof + 255) / 256);
     hipLaunchKernelGGL(k_gather_sel, dim3(blocks), dim3(256), 0, st, yd, y_user, sd->out_dst,
@@ -1952,8 +724,8 @@ int noalloc_matvec(bw_hip_handle* hd, const double* x, double* y, int ordering, 
   // xt, then the partial sums of pass 1 and pass 2, each 256-byte aligned
   const auto up = [](int64_t b) { return (b + 255) / 256 * 256; };
   const int64_t off1 = up(op.xt_size * op.elem);
-  const int64_t off2 = off1 + up(op.part_elems[0] * op.elem);
-  const int64_t need = off2 + up(op.part_elems[1] * op.elem);
+  const int64_t off2 = off1 + up(op.p1.single.part_elems * op.elem);
+  const int64_t need = off2 + up(op.p2.single.part_elems * op.elem);
   int64_t limit = BW_NOALLOC_SCRATCH_BYTES;
   if (const char* e = std::getenv("BWHIP_NOALLOC_LIMIT")) {
     const long long v = std::atoll(e);
@@ -2385,74 +1157,74 @@ int check_batched(bw_hip_handle* hd, bool adjoint, int nrhs, const double* X, in
   return BW_OK;
 }
 
+// The MFMA kernel and the reduction of one pass of the batched product.
+template <int PASS>
+void launch_mfma(const DevPass& dp, hipStream_t st, const float* xb, const BatchOut<float>& o) {
+  const DevItems& di = dp.batched;
+  hipLaunchKernelGGL((k_slab_mfma32<PASS, kRhs / 32, kBatchWaves>), dim3(di.blocks),
+                     dim3(64 * kBatchWaves), 0, st, di.wis, di.xs, dp.gidx,
+                     static_cast<const float*>(dp.data), xb, o);
+}
+template <int PASS>
+void launch_mfma(const DevPass& dp, hipStream_t st, const double* xb, const BatchOut<double>& o) {
+  const DevItems& di = dp.batched;
+  hipLaunchKernelGGL((k_slab_mfma16<double, PASS, kRhs / 16, kBatchWaves>), dim3(di.blocks),
+                     dim3(64 * kBatchWaves), 0, st, di.wis, di.xs, dp.gidx,
+                     static_cast<const double*>(dp.data), xb, o);
+}
+template <int PASS, typename T>
+void launch_batched_pass(const DevPass& dp, hipStream_t st, const T* xb, const BatchOut<T>& o) {
+  const DevItems& di = dp.batched;
+  if (di.nwi > 0) launch_mfma<PASS>(dp, st, xb, o);
+  if (di.nred > 0)
+    hipLaunchKernelGGL((k_reduce_b<PASS, kRhs, T>), dim3(di.nred), dim3(256), 0, st, di.reds,
+                       di.nred, o);
+}
+
 // The kernels of Y = H X (kRhs right-hand sides per round) on stream st,
 // writing only the batched scratch `s`.
+template <typename T>
 int launch_batched(bw_hip_handle* hd, DevOp& op, const OpScratch& s, int nrhs, const double* X,
                    int64_t xr, int64_t xc, double* Y, int64_t yr, int64_t yc, int ordering,
-                   bool fp64, hipStream_t st) {
+                   hipStream_t st) {
+  constexpr int NB = kRhs;
   const bool orig = ordering == BW_ORDER_ORIGINAL;
   const int dof = hd->dof;
-  for (int k0 = 0; k0 < nrhs; k0 += kRhs) {
-    const int nk = std::min(kRhs, nrhs - k0);
+  const int64_t* pin = orig ? op.perm_in : nullptr;
+  T* xb = static_cast<T*>(s.xb);
+  for (int k0 = 0; k0 < nrhs; k0 += NB) {
+    const int nk = std::min(NB, nrhs - k0);
     const double* Xk = X + static_cast<int64_t>(k0) * xc;
     double* Yk = Y + static_cast<int64_t>(k0) * yc;
-    const int64_t rows_per_block = 256 / kRhs;
-    const int gblocks = static_cast<int>((op.n_in + rows_per_block - 1) / rows_per_block);
     // row-major input (unit column stride, even row stride, 16-byte aligned
-    // rows): the vector gather, 32 rows per block
+    // rows): the vector gather
     const bool rowmajor = xc == 1 && xr % 2 == 0 && reinterpret_cast<uintptr_t>(Xk) % 16 == 0;
-    const int gblocks4 = static_cast<int>((op.n_in + 31) / 32);
-    const int64_t* pin = orig ? op.perm_in : nullptr;
-    const int64_t* pout = orig ? op.perm_out : nullptr;
-    if (fp64) {
-      double* xb = static_cast<double*>(s.xb);
-      double* pb0 = static_cast<double*>(s.partb[0]);
-      double* pb1 = static_cast<double*>(s.partb[1]);
-      if (rowmajor)
-        hipLaunchKernelGGL(k_gather_b4<double>, dim3(gblocks4), dim3(256), 0, st, Xk, xr, nk, xb,
-                           op.n_in, pin, dof);
-      else
-        hipLaunchKernelGGL(k_gather_b<double>, dim3(gblocks), dim3(256), 0, st, Xk, xr, xc, nk, xb,
-                           op.n_in, pin, dof);
-      if (op.p1.nwi > 0)
-        launch_mfma64<1>(op.mfma_schedule, op.p1.blocks, st, op.p1.wis, op.p1.xs, op.p1.gidx,
-                         static_cast<const double*>(op.p1.data), xb, xb, nullptr, 0, 0, kRhs,
-                         pb0, nullptr, dof, op.p1.rowmap);
-      if (op.p1.nred > 0)
-        hipLaunchKernelGGL((k_reduce_b<1, double>), dim3(op.p1.nred), dim3(256), 0, st, op.p1.reds,
-                           op.p1.nred, pb0, xb, nullptr, 0, 0, kRhs, nullptr, dof, op.p1.rowmap);
-      if (op.p2.nwi > 0)
-        launch_mfma64<2>(op.mfma_schedule, op.p2.blocks, st, op.p2.wis, op.p2.xs, op.p2.gidx,
-                         static_cast<const double*>(op.p2.data), xb, nullptr, Yk, yr, yc, nk,
-                         pb1, pout, dof, nullptr);
-      if (op.p2.nred > 0)
-        hipLaunchKernelGGL((k_reduce_b<2, double>), dim3(op.p2.nred), dim3(256), 0, st, op.p2.reds,
-                           op.p2.nred, pb1, nullptr, Yk, yr, yc, nk, pout, dof, nullptr);
+    if (rowmajor) {
+      constexpr int rows = 256 / (NB / 4);
+      hipLaunchKernelGGL((k_gather_b4<T, NB>), dim3(static_cast<int>((op.n_in + rows - 1) / rows)),
+                         dim3(256), 0, st, Xk, xr, nk, xb, op.n_in, pin, dof);
     } else {
-      float* xb = static_cast<float*>(s.xb);
-      float* pb0 = static_cast<float*>(s.partb[0]);
-      float* pb1 = static_cast<float*>(s.partb[1]);
-      if (rowmajor)
-        hipLaunchKernelGGL(k_gather_b4<float>, dim3(gblocks4), dim3(256), 0, st, Xk, xr, nk, xb,
-                           op.n_in, pin, dof);
-      else
-        hipLaunchKernelGGL(k_gather_b<float>, dim3(gblocks), dim3(256), 0, st, Xk, xr, xc, nk, xb,
-                           op.n_in, pin, dof);
-      if (op.p1.nwi > 0)
-        launch_mfma<1>(op.mfma_schedule, op.p1.blocks, st, op.p1.wis, op.p1.xs, op.p1.gidx,
-                       static_cast<const float*>(op.p1.data), xb, xb, nullptr, 0, 0, kRhs, pb0,
-                       nullptr, dof, op.p1.rowmap);
-      if (op.p1.nred > 0)
-        hipLaunchKernelGGL((k_reduce_b<1, float>), dim3(op.p1.nred), dim3(256), 0, st, op.p1.reds,
-                           op.p1.nred, pb0, xb, nullptr, 0, 0, kRhs, nullptr, dof, op.p1.rowmap);
-      if (op.p2.nwi > 0)
-        launch_mfma<2>(op.mfma_schedule, op.p2.blocks, st, op.p2.wis, op.p2.xs, op.p2.gidx,
-                       static_cast<const float*>(op.p2.data), xb, nullptr, Yk, yr, yc, nk, pb1, pout,
-                       dof, nullptr);
-      if (op.p2.nred > 0)
-        hipLaunchKernelGGL((k_reduce_b<2, float>), dim3(op.p2.nred), dim3(256), 0, st, op.p2.reds,
-                           op.p2.nred, pb1, nullptr, Yk, yr, yc, nk, pout, dof, nullptr);
+      constexpr int rows = 256 / NB;
+      hipLaunchKernelGGL((k_gather_b<T, NB>), dim3(static_cast<int>((op.n_in + rows - 1) / rows)),
+                         dim3(256), 0, st, Xk, xr, xc, nk, xb, op.n_in, pin, dof);
     }
+    BatchOut<T> o1{};
+    o1.tout = xb;
+    o1.nk = NB;
+    o1.part = static_cast<T*>(s.partb[0]);
+    o1.dof = dof;
+    o1.rowmap = op.p1.rowmap;
+    BatchOut<T> o2{};
+    o2.Y = Yk;
+    o2.yr = yr;
+    o2.yc = yc;
+    o2.nk = nk;
+    o2.yvec = yc == 1 && yr % 2 == 0 && reinterpret_cast<uintptr_t>(Yk) % 16 == 0;
+    o2.part = static_cast<T*>(s.partb[1]);
+    o2.perm = orig ? op.perm_out : nullptr;
+    o2.dof = dof;
+    launch_batched_pass<1>(op.p1, st, xb, o1);
+    launch_batched_pass<2>(op.p2, st, xb, o2);
     HIPCHK(hipGetLastError());
   }
   return BW_OK;
@@ -2472,7 +1244,9 @@ int batched_impl(bw_hip_handle* hd, bool adjoint, int nrhs, const double* X, int
   const int adj = adjoint ? 1 : 0, f32 = precision == BW_PREC_FP32 ? 1 : 0;
   StreamCtx* ctx = stream_ctx(hd, st);
   if ((rc = ensure_op_scratch(hd, ctx, adj, f32, true))) return rc;
-  return launch_batched(hd, *op, ctx->op[adj][f32], nrhs, X, xr, xc, Y, yr, yc, ordering, !f32, st);
+  const OpScratch& s = ctx->op[adj][f32];
+  return f32 ? launch_batched<float>(hd, *op, s, nrhs, X, xr, xc, Y, yr, yc, ordering, st)
+             : launch_batched<double>(hd, *op, s, nrhs, X, xr, xc, Y, yr, yc, ordering, st);
 }
 
 // Captures launch(stream, ctx) on a private stream into a new graph that owns
@@ -2571,8 +1345,11 @@ int bw_hip_graph_create_batched(bw_hip_handle* hd, int adjoint, int nrhs, const 
     return rc;
   }
   return capture_graph(hd, std::move(g), [&](hipStream_t cs, StreamCtx& ctx) {
-    return launch_batched(hd, *op, ctx.op[adj][f32], nrhs, X, x_row_stride, x_col_stride, Y,
-                          y_row_stride, y_col_stride, ordering, !f32, cs);
+    const OpScratch& s = ctx.op[adj][f32];
+    return f32 ? launch_batched<float>(hd, *op, s, nrhs, X, x_row_stride, x_col_stride, Y,
+                                       y_row_stride, y_col_stride, ordering, cs)
+               : launch_batched<double>(hd, *op, s, nrhs, X, x_row_stride, x_col_stride, Y,
+                                        y_row_stride, y_col_stride, ordering, cs);
   }, out);
 }
 
@@ -2683,10 +1460,6 @@ int bw_hip_set_mfma_schedule(bw_hip_handle* hd, int precision_mask, int schedule
   if (schedule < 0 || schedule > 15) return fail(BW_EINVAL, "set_mfma_schedule: schedule must be 0-15");
   if (precision_mask <= 0 || (precision_mask & ~(BW_PREC_FP64 | BW_PREC_FP32)))
     return fail(BW_EINVAL, "set_mfma_schedule: bad precision mask");
-  for (int adj = 0; adj < 2; ++adj) {
-    if (precision_mask & BW_PREC_FP64) hd->op[adj][0].mfma_schedule = schedule;
-    if (precision_mask & BW_PREC_FP32) hd->op[adj][1].mfma_schedule = schedule;
-  }
   return BW_OK;
 }
 

@@ -224,68 +224,118 @@ void add_slabs(Program* P, int64_t total_rows, int max_rows, int64_t out_row0,
   }
 }
 
-void finalize_program(Program* P, const LayoutOptions& opt) {
+// Work-item sizes, in entries (bytes / element size, so that FP32 items hold as
+// many entries as FP64 ones).  A work item is one workgroup's share of a slab.
+// Measured on MI355X with 8-wave workgroups for the single-vector kernel:
+// - below the bounds the launch's tail and the kernel's start dominate, above
+//   them too few workgroups are left to balance: pass 2 of the 120 000-DoF
+//   3DR0 operator (4.3 GB) takes 656 us at 1.5 MiB, 639 at 384 KiB and 650 at
+//   256 KiB; the 21 000-DoF 3DT0 one (320 MB) 61 us at 384 KiB, 57 at 192-256
+//   KiB and 75 with whole slabs (0.8 MiB).
+constexpr int64_t kItemMin = 24 * 1024, kItemMax = 48 * 1024;
+constexpr int64_t kItemShare = 4096;  // between the two: 1 / 4096 of the pass
+// - the batched kernels (4-wave workgroups) pay for every split with NB-wide
+//   partial rows: 32 right-hand sides on the 49 152-DoF 3DR0 operator take 306
+//   us at 384 KiB (FP32), 314 at 256, 311 at 768 KiB.
+constexpr int64_t kItemBatched = 96 * 1024;
+// Pass 1 of a small operator is cut by rows instead: a slab over a wide column
+// cluster gets fewer rows (at least 16), so that it is one work item and the
+// pass needs no reduction.  Its item size is 1 / 1500 of the pass, at least 64
+// KiB (25 600-DoF mode-1 operator, 171 MB: 42.7 us at 1 / 512, 40.4 at 1 /
+// 1024, 38.8 at 1 / 1500, 41.3 at 1 / 2048 with 32 KiB).
+constexpr int64_t kPass1Share = 1500, kPass1MinBytes = 64 * 1024;
+// Pass 2 wants at least this many workgroups (of 256 compute units); operators
+// with fewer slabs that fit one work item each get slabs of fewer rows (4 000-
+// DoF 2DS0 operator, pass 2: 64 slabs of 62 rows 12.0 us, 256 of 16 rows 10.7).
+constexpr int64_t kMinSlabs = 192;
+constexpr int kMinRows = 16;
+
+// Cuts the slabs into work items of about wi_bytes each and deals them to the
+// XCDs in eight contiguous ranges of about equal cost.  row_tile: rows that a
+// kernel's work comes in (the MFMA tile; 1: cost is bytes).  sorted: costliest
+// first within each XCD's range, so that a range ends on its small items.
+void cut_items(const Program& P, const LayoutOptions& opt, int64_t wi_bytes, int row_tile,
+               bool sorted, ItemList* il) {
   const int V = opt.vec_elems;
-  int64_t data = 0, part = 0;
-  P->wis.clear();
-  P->gidx.clear();
-  P->reds.clear();
-  for (size_t s = 0; s < P->slabs.size(); ++s) {
-    SlabDesc& sd = P->slabs[s];
-    sd.data_off = data;
-    const int64_t gbeg = static_cast<int64_t>(P->gidx.size());
-    for (int32_t r = sd.run_beg; r < sd.run_end; ++r) {
-      const RunDesc& rd = P->runs[r];
-      const int64_t ng = (rd.ncols + V - 1) / V;
-      for (int64_t g = 0; g < ng; ++g) P->gidx.push_back(static_cast<int32_t>(rd.zoff + g * V));
-    }
+  *il = ItemList{};
+  int64_t part = 0;
+  for (const SlabDesc& sd : P.slabs) {
     const int64_t bytes = sd.ngroups * sd.rows * V * opt.elem_bytes;
-    int64_t nwi = std::max<int64_t>(1, (bytes + opt.wi_bytes / 2) / opt.wi_bytes);
+    int64_t nwi = std::max<int64_t>(1, (bytes + wi_bytes / 2) / wi_bytes);
     nwi = std::min<int64_t>(nwi, std::max<int64_t>(1, sd.ngroups));
-    int64_t per = std::max<int64_t>(1, (sd.ngroups + nwi - 1) / nwi);
+    const int64_t per = std::max<int64_t>(1, (sd.ngroups + nwi - 1) / nwi);
     nwi = std::max<int64_t>(1, (sd.ngroups + per - 1) / per);
-    sd.wi_beg = static_cast<int32_t>(P->wis.size());
     for (int64_t w = 0; w < nwi; ++w) {
       const int64_t g0 = w * per;
       const int64_t g1 = std::min(sd.ngroups, g0 + per);
       WorkItem wi{};
-      wi.data_off = data + g0 * sd.rows * V;
-      wi.gbeg = static_cast<int32_t>(gbeg + g0);
+      wi.data_off = sd.data_off + g0 * sd.rows * V;
+      wi.gbeg = static_cast<int32_t>(sd.gbeg + g0);
       wi.ngroups = static_cast<int32_t>(g1 - g0);
       wi.rows = sd.rows;
       wi.out_row = static_cast<int32_t>(sd.out_row0);
       wi.part_off = nwi == 1 ? -1 : static_cast<int32_t>(part + w * sd.rows);
       wi.pad = 0;
-      P->wis.push_back(wi);
+      il->wis.push_back(wi);
     }
-    sd.wi_end = static_cast<int32_t>(P->wis.size());
     if (nwi > 1) {
       const Reduce rd{static_cast<int32_t>(sd.out_row0), sd.rows, static_cast<int32_t>(part),
                       static_cast<int32_t>(nwi)};
-      P->reds.push_back(rd);
+      il->reds.push_back(rd);
       part += nwi * sd.rows;
     }
-    data += sd.ngroups * sd.rows * V;
   }
-  P->data_elems = data;
-  P->part_elems = part;
-  // byte-balanced XCD ranges: cut the WI list where the running byte count
-  // crosses x/8 of the total (the nearer side of the crossing)
-  const int64_t nwi = static_cast<int64_t>(P->wis.size());
+  il->part_elems = part;
+  // balanced XCD ranges: cut the WI list where the running cost crosses x/8 of
+  // the total (the nearer side of the crossing)
+  const int64_t nwi = static_cast<int64_t>(il->wis.size());
   std::vector<int64_t> cum(nwi + 1, 0);
-  for (int64_t i = 0; i < nwi; ++i)
-    cum[i + 1] = cum[i] + static_cast<int64_t>(P->wis[i].ngroups) * P->wis[i].rows + 1;
-  P->xcd[0] = 0;
+  auto cost = [&](const WorkItem& w) {
+    return static_cast<int64_t>(w.ngroups) * ((w.rows + row_tile - 1) / row_tile * row_tile) + 1;
+  };
+  for (int64_t i = 0; i < nwi; ++i) cum[i + 1] = cum[i] + cost(il->wis[i]);
+  il->xcd[0] = 0;
   for (int x = 1; x < kXcds; ++x) {
     const long double target = static_cast<long double>(cum[nwi]) * x / kXcds;
     int64_t i = std::lower_bound(cum.begin(), cum.end(), static_cast<int64_t>(target)) - cum.begin();
     if (i > 0 && target - cum[i - 1] < cum[std::min(i, nwi)] - target) --i;
-    P->xcd[x] = static_cast<int32_t>(std::max<int64_t>(P->xcd[x - 1], std::min(i, nwi)));
+    il->xcd[x] = static_cast<int32_t>(std::max<int64_t>(il->xcd[x - 1], std::min(i, nwi)));
   }
-  P->xcd[kXcds] = static_cast<int32_t>(nwi);
+  il->xcd[kXcds] = static_cast<int32_t>(nwi);
+  if (sorted)
+    for (int x = 0; x < kXcds; ++x)
+      std::stable_sort(il->wis.begin() + il->xcd[x], il->wis.begin() + il->xcd[x + 1],
+                       [&](const WorkItem& a, const WorkItem& b) { return cost(a) > cost(b); });
   int32_t most = 0;
-  for (int x = 0; x < kXcds; ++x) most = std::max(most, P->xcd[x + 1] - P->xcd[x]);
-  P->xcd_blocks = kXcds * ((most + 3) / 4);
+  for (int x = 0; x < kXcds; ++x) most = std::max(most, il->xcd[x + 1] - il->xcd[x]);
+  il->xcd_blocks = kXcds * ((most + 3) / 4);
+}
+
+// Places the slabs' data and column groups, and cuts both work-item lists.
+// Pass 1's items differ most in size (24 KiB to its bound) and run costliest
+// first (30 000-DoF 3DR0 operator: pass 1 97 us in slab order, 90 sorted);
+// pass 2's single-vector items are alike, and slab order, in which neighbours
+// share input entries, is 1 % faster on the 120 000-DoF one.  The batched
+// kernels run 6-8 % faster sorted (327 -> 306 us, FP32, 49 152 DoF).
+void finalize_program(Program* P, const LayoutOptions& opt, int64_t wi_single, bool sort_single) {
+  const int V = opt.vec_elems;
+  int64_t data = 0;
+  P->gidx.clear();
+  for (SlabDesc& sd : P->slabs) {
+    sd.data_off = data;
+    sd.gbeg = static_cast<int32_t>(P->gidx.size());
+    for (int32_t r = sd.run_beg; r < sd.run_end; ++r) {
+      const RunDesc& rd = P->runs[r];
+      const int64_t ng = (rd.ncols + V - 1) / V;
+      for (int64_t g = 0; g < ng; ++g) P->gidx.push_back(static_cast<int32_t>(rd.zoff + g * V));
+    }
+    data += sd.ngroups * sd.rows * V;
+  }
+  P->data_elems = data;
+  const bool tuned = opt.wi_bytes > 0;
+  cut_items(*P, opt, tuned ? opt.wi_bytes : wi_single, 1, sort_single, &P->single);
+  cut_items(*P, opt, tuned ? opt.wi_bytes : kItemBatched * opt.elem_bytes,
+            opt.elem_bytes == 8 ? 16 : 32, true, &P->batched);
 }
 
 }  // namespace
@@ -308,6 +358,18 @@ void build_layout(const OpView& v, const LayoutOptions& opt, Layout* L) {
     Program& P = L->pass1;
     P = Program{};
     P.out_rows = v.t_total;
+    int64_t entries = 0;
+    for (int64_t k = 0; k < nlr; ++k) entries += v.lr_rank[k] * d * (v.lr_c1[k] - v.lr_c0[k]);
+    const int64_t max_item = kItemMax * opt.elem_bytes;
+    const int64_t item =
+        std::max<int64_t>(kPass1MinBytes, entries * opt.elem_bytes / kPass1Share);
+    const bool by_rows = opt.wi_bytes == 0 && item < max_item;
+    // most rows of a slab over `cols` columns
+    auto rows_for = [&](int64_t cols) -> int64_t {
+      if (!by_rows) return opt.max_rows;
+      const int64_t r = item * 3 / 2 / (cols * opt.elem_bytes) / kMinRows * kMinRows;
+      return std::min<int64_t>(opt.max_rows, std::max<int64_t>(kMinRows, r));
+    };
     std::vector<int64_t> order;
     order.reserve(nlr);
     for (int64_t k = 0; k < nlr; ++k)
@@ -318,7 +380,6 @@ void build_layout(const OpView& v, const LayoutOptions& opt, Layout* L) {
       return v.toff[a] < v.toff[b];
     });
     RunBuilder rb{&P};
-    const int64_t maxr = opt.max_rows;
     size_t i = 0;
     while (i < order.size()) {
       size_t j = i;  // [i, j): one column cluster
@@ -326,6 +387,7 @@ void build_layout(const OpView& v, const LayoutOptions& opt, Layout* L) {
              v.lr_c1[order[j]] == v.lr_c1[order[i]])
         ++j;
       const int64_t c0 = v.lr_c0[order[i]], ncols = d * (v.lr_c1[order[i]] - c0);
+      const int64_t maxr = rows_for(ncols);
       // each factor's rows cut into ceil(r / maxr) chunks of even height (a
       // rank of 90 gives 45 + 45, not 64 + 26), packed first-fit decreasing
       std::vector<StackPart> chunks;
@@ -376,7 +438,7 @@ void build_layout(const OpView& v, const LayoutOptions& opt, Layout* L) {
       }
       i = j;
     }
-    finalize_program(&P, opt);
+    finalize_program(&P, opt, by_rows ? 4 * item : max_item, true);
   }
 
   // ---- pass 2: row intervals
@@ -409,6 +471,19 @@ void build_layout(const OpView& v, const LayoutOptions& opt, Layout* L) {
       if (v.lr_rank[k] == 0) continue;
       for (int64_t q = interval_of(v.lr_r0[k]); q < nint && bps[q] < v.lr_r1[k]; ++q) lrl[q].push_back(k);
     }
+    int64_t entries = 0;
+    for (int64_t k = 0; k < nfr; ++k)
+      entries += d * (v.fr_r1[k] - v.fr_r0[k]) * d * (v.fr_c1[k] - v.fr_c0[k]);
+    for (int64_t k = 0; k < nlr; ++k) entries += v.lr_rank[k] * d * (v.lr_r1[k] - v.lr_r0[k]);
+    const int64_t item = opt.elem_bytes * std::min<int64_t>(
+        kItemMax, std::max<int64_t>(kItemMin, entries / kItemShare));
+    int64_t nslab = 0;  // slabs of full height
+    for (int64_t q = 0; q < nint; ++q)
+      nslab += (d * (bps[q + 1] - bps[q]) + opt.max_rows - 1) / opt.max_rows;
+    int64_t max_rows = opt.max_rows;
+    if (opt.wi_bytes == 0 && nslab < kMinSlabs &&
+        entries * opt.elem_bytes / nslab < item * 3 / 2)
+      max_rows = std::max<int64_t>(kMinRows, opt.max_rows * nslab / kMinSlabs / kMinRows * kMinRows);
     RunBuilder rb{&P};
     for (int64_t q = 0; q < nint; ++q) {
       auto& fl = frl[q];
@@ -424,9 +499,9 @@ void build_layout(const OpView& v, const LayoutOptions& opt, Layout* L) {
       for (int64_t k : ll) rb.add_piece(L->xt_t + v.toff[k], v.lr_rank[k], 1, k);
       const int32_t rend = static_cast<int32_t>(P.runs.size());
       const int64_t rows = d * (bps[q + 1] - bps[q]);
-      add_slabs(&P, rows, opt.max_rows, d * bps[q], d * bps[q], rbeg, rend, V);
+      add_slabs(&P, rows, static_cast<int>(max_rows), d * bps[q], d * bps[q], rbeg, rend, V);
     }
-    finalize_program(&P, opt);
+    finalize_program(&P, opt, item, false);
   }
 }
 
@@ -499,9 +574,10 @@ int check_layout_limits(const Layout& L, std::string* msg) {
     return BW_ESHAPE;
   }
   for (const Program* P : {&L.pass1, &L.pass2}) {
-    if (static_cast<int64_t>(P->gidx.size()) >= lim || P->part_elems >= lim ||
-        static_cast<int64_t>(P->rowmap.size()) >= lim ||
-        static_cast<int64_t>(P->wis.size()) >= lim / 4) {
+    if (static_cast<int64_t>(P->gidx.size()) >= lim || P->single.part_elems >= lim ||
+        P->batched.part_elems >= lim || static_cast<int64_t>(P->rowmap.size()) >= lim ||
+        static_cast<int64_t>(P->single.wis.size()) >= lim / 4 ||
+        static_cast<int64_t>(P->batched.wis.size()) >= lim / 4) {
       *msg = "matrix too large for 32-bit layout descriptors";
       return BW_ESHAPE;
     }

@@ -27,9 +27,9 @@
 // so lane `row` of a wavefront reads one 16-byte vector per group and a
 // wavefront reads R*16 contiguous bytes.  Runs of columns whose input entries
 // are contiguous share one input offset per group (gidx[g]); a run that is
-// not a multiple of V is padded with zero columns.  Long slabs are split into
-// several work items (WIs) whose partial sums a small reduce pass adds in WI
-// order.
+// not a multiple of V is padded with zero columns.  A work item (WI) is one
+// workgroup's share: a slab, or a range of a long slab's groups, whose partial
+// sums a small reduce pass adds in WI order.
 //
 // The same builder serves the adjoint H^T by viewing every block transposed.
 #pragma once
@@ -54,7 +54,8 @@ struct WorkItem {
 };
 
 // Reduce descriptor for a slab split over several WIs (16 bytes): a separate
-// pass after the slab pass adds the partial sums in WI order.  (Reducing
+// pass after the slab pass adds the partial sums in WI order; the waves of one
+// workgroup add theirs in LDS.  (Reducing
 // inside the slab kernel, by its last WI, needs agent-scope release/acquire
 // fences, which on MI355X write back and invalidate the per-XCD L2 and cost
 // more than the separate launch.)
@@ -95,26 +96,32 @@ struct SlabDesc {
   int32_t stack_beg, stack_end;  // pass 1: the W_k rows of the slab, in row order
   int64_t ngroups;
   int64_t data_off;
-  int32_t wi_beg, wi_end;
+  int32_t gbeg;        // first entry in gidx
+};
+
+// How the slabs of one pass are handed to workgroups: each work item is one
+// workgroup's share, a whole slab or a range of its column groups.
+struct ItemList {
+  std::vector<WorkItem> wis;
+  std::vector<Reduce> reds;       // one per split slab
+  int64_t part_elems = 0;
+  // Work items [xcd[x], xcd[x+1]) run on XCD x: eight contiguous ranges of
+  // about equal bytes; xcd_blocks groups of four work items cover the longest.
+  int32_t xcd[kXcds + 1] = {};
+  int32_t xcd_blocks = 0;
 };
 
 // One pass (1 or 2) of one operator (H or H^T) at one precision.
 struct Program {
-  std::vector<WorkItem> wis;
   std::vector<int32_t> gidx;
   std::vector<StackPart> stack;   // pass 1: row sources of the slabs
   std::vector<int32_t> rowmap;    // pass 1: xt index of every slab row (t entry)
-  std::vector<Reduce> reds;       // one per split slab
   std::vector<SlabDesc> slabs;
   std::vector<RunDesc> runs;
   std::vector<Piece> pieces;
+  ItemList single, batched;       // of the single-vector and the batched kernels
   int64_t data_elems = 0;
-  int64_t part_elems = 0;
   int64_t out_rows = 0;
-  // Work items [xcd[x], xcd[x+1]) run on XCD x: eight contiguous ranges of
-  // about equal bytes; xcd_blocks workgroups (4 WIs each) cover the longest.
-  int32_t xcd[kXcds + 1] = {};
-  int32_t xcd_blocks = 0;
 };
 
 // An operator view: H itself, or H^T built from the same blocks.
@@ -143,7 +150,7 @@ struct LayoutOptions {
   int vec_elems = 2;            // V
   int elem_bytes = 8;           // 8 (FP64) or 4 (FP32)
   int max_rows = 64;            // rows per slab (<= 64)
-  int64_t wi_bytes = 96 * 1024; // target bytes per work item
+  int64_t wi_bytes = 0;         // target bytes per work item; 0: sized from each pass
   int stack_rows = 64;          // pass-1 chunks of at most this many rows share slabs
 };
 

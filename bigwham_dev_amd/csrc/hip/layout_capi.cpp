@@ -91,11 +91,11 @@ int bw_layout_info(const bw_layout* lay, int64_t* info) {
   info[1] = lay->L.xt_size;
   const bwl::Program* P[2] = {&lay->L.pass1, &lay->L.pass2};
   for (int p = 0; p < 2; ++p) {
-    info[2 + 6 * p] = static_cast<int64_t>(P[p]->wis.size());
+    info[2 + 6 * p] = static_cast<int64_t>(P[p]->single.wis.size());
     info[3 + 6 * p] = static_cast<int64_t>(P[p]->gidx.size());
-    info[4 + 6 * p] = static_cast<int64_t>(P[p]->reds.size());
+    info[4 + 6 * p] = static_cast<int64_t>(P[p]->single.reds.size());
     info[5 + 6 * p] = P[p]->data_elems;
-    info[6 + 6 * p] = P[p]->part_elems;
+    info[6 + 6 * p] = P[p]->single.part_elems;
     info[7 + 6 * p] = P[p]->out_rows;
   }
   info[14] = lay->L.opt.vec_elems;
@@ -119,16 +119,16 @@ int bw_layout_export(const bw_layout* lay, int pass, int64_t* wis, int32_t* gidx
   if (!lay || (pass != 1 && pass != 2)) return BW_EINVAL;
   const bwl::Program& P = pass == 1 ? lay->L.pass1 : lay->L.pass2;
   if (wis)
-    for (size_t i = 0; i < P.wis.size(); ++i) {
-      const bwl::WorkItem& w = P.wis[i];
+    for (size_t i = 0; i < P.single.wis.size(); ++i) {
+      const bwl::WorkItem& w = P.single.wis[i];
       int64_t* o = wis + 8 * i;
       o[0] = w.data_off; o[1] = w.gbeg; o[2] = w.ngroups; o[3] = w.rows;
       o[4] = w.out_row; o[5] = w.part_off; o[6] = 0; o[7] = 0;
     }
   if (gidx && !P.gidx.empty()) std::memcpy(gidx, P.gidx.data(), P.gidx.size() * sizeof(int32_t));
   if (reds)
-    for (size_t i = 0; i < P.reds.size(); ++i) {
-      const bwl::Reduce& r = P.reds[i];
+    for (size_t i = 0; i < P.single.reds.size(); ++i) {
+      const bwl::Reduce& r = P.single.reds[i];
       reds[4 * i] = r.out_row; reds[4 * i + 1] = r.rows;
       reds[4 * i + 2] = r.part_off; reds[4 * i + 3] = r.nparts;
     }
@@ -142,8 +142,8 @@ int bw_layout_export(const bw_layout* lay, int pass, int64_t* wis, int32_t* gidx
 int bw_layout_export_xcd(const bw_layout* lay, int pass, int32_t* xcd, int32_t* blocks) {
   if (!lay || !xcd || !blocks || (pass != 1 && pass != 2)) return BW_EINVAL;
   const bwl::Program& P = pass == 1 ? lay->L.pass1 : lay->L.pass2;
-  for (int x = 0; x <= bwl::kXcds; ++x) xcd[x] = P.xcd[x];
-  *blocks = P.xcd_blocks;
+  for (int x = 0; x <= bwl::kXcds; ++x) xcd[x] = P.single.xcd[x];
+  *blocks = P.single.xcd_blocks;
   return BW_OK;
 }
 

@@ -240,7 +240,7 @@ void bw_flat_recompressed_free(bw_flat_recompressed* r);
 int bw_hip_set_stacking(int stack_rows);
 
 /* Loads in flight per lane in the slab kernels of this handle (4, 8 or 16;
- * 0 keeps the current value).  Chosen by bigwham_dev_amd.autotune. */
+ * 0 keeps the current value; 16 runs as 8).  Chosen by bigwham_dev_amd.autotune. */
 int bw_hip_set_unroll(bw_hip_handle* hd, int unroll_fp64, int unroll_fp32);
 
 /* The same for one pass (1: t = B x, 2: y = F x + A t) of the precisions in
@@ -248,23 +248,9 @@ int bw_hip_set_unroll(bw_hip_handle* hd, int unroll_fp64, int unroll_fp32);
  * different depths.  The autotuner picks both from one timing run. */
 int bw_hip_set_unroll_pass(bw_hip_handle* hd, int precision_mask, int pass, int unroll);
 
-/* Schedule of the MFMA kernels of the batched products, for the precisions
- * in precision_mask.  FP32: group pairs per step and whether the next step's
- * loads are issued before the current step's MFMAs (0: 4 pairs; 1: 2 pairs,
- * pipelined; 2: 4 pairs, pipelined; 3: 8 pairs; 4-7: a ring of D step
- * buffers with D - 1 steps of loads in flight: 4: 2 pairs, D = 3; 5: 2 pairs,
- * D = 4; 6: 1 pair, D = 6; 7: 1 pair, D = 8; 8-11: the same four shapes as a
- * ring consumed in load order, every buffer refilled right after its MFMAs,
- * D - 1 steps in flight at every step; 12, 13: 16-row tiles on
- * v_mfma_f32_16x16x4f32, ceil(R / 16) tiles per slab of R rows, load-order
- * ring with D = 3, 4; 14, 15: schedules 8, 9 with each column group's four
- * input rows loaded as one 16-byte load per lane and handed to the MFMA
- * layout through LDS).  FP64: 0-3 load two k-steps before their MFMAs; 4-7
- * the ring with D = 3, 4, 6, 8; 8-11 the load-order ring with D = 3, 4, 6, 8
- * (12, 14 = 8 and 13, 15 = 9: the FP64 kernel has 16-row tiles throughout).  Every
- * schedule gives the same values to FP32 / FP64 rounding of one summation
- * order per 16- or 32-row tile.  Default: 14 (FP32), 5 (FP64);
- * bigwham_dev_amd.autotune times them all on the caller's matrix. */
+/* Schedule (0-15) of the MFMA kernels of the batched products, for the
+ * precisions in precision_mask.  The batched kernels have one schedule, the
+ * fastest measured, which every value selects: the results do not depend on it. */
 int bw_hip_set_mfma_schedule(bw_hip_handle* hd, int precision_mask, int schedule);
 
 /* Per-kernel timing.  With timing enabled every matvec records HIP events

@@ -1,0 +1,70 @@
+"""Work items shared by the waves of a workgroup, at the sizes where the split
+can go wrong: slabs of 1 to 64 rows (edges of the 16- and 32-row tiles), items
+of fewer column groups than a workgroup has waves, remainders of every batch
+depth, whole slabs and slabs split over several items, against the operator's
+blocks multiplied in numpy.
+
+The tolerance is the a-priori bound of a sum of products in the working
+precision: |y - H x| <= n u (|F| |x| + |A| (|B| |x|)) with n the terms of the
+longest row (columns plus total rank, twice for the two passes, plus the
+conversion of factors and input), u the unit roundoff."""
+import numpy as np
+import pytest
+
+from bigwham_dev_amd import HipHmat, set_tuning
+from synthetic_hmat import SyntheticHmat
+
+pytestmark = pytest.mark.gpu
+
+U = {"fp64": 2.0 ** -53, "fp32": 2.0 ** -24}
+# (row points, column points, dof, seed): slabs of many heights, few and many
+# columns, one-row and one-column point sets
+SHAPES = [(120, 90, 1, 1), (95, 140, 2, 2), (64, 200, 3, 3), (1, 75, 1, 4), (75, 1, 3, 5)]
+
+
+def _reference(S, X, adjoint):
+    """H X (H^T X) in permuted order, and |F| |X| + |A| (|B| |X|)."""
+    d = S.dof
+    n_out = d * (S.n_col_pts if adjoint else S.n_row_pts)
+    Y, B = np.zeros((n_out, X.shape[1])), np.zeros((n_out, X.shape[1]))
+    blocks = [(p, (F,)) for p, F in zip(S.fr_pattern, S.fr)]
+    blocks += [(p, (A, Bf)) for p, A, Bf in zip(S.lr_pattern, S.A, S.B)]
+    for (_, i0, j0, i1, j1, _), fs in blocks:
+        rows, cols = slice(d * i0, d * i1), slice(d * j0, d * j1)
+        if adjoint:
+            rows, cols, fs = cols, rows, tuple(f.T for f in reversed(fs))
+        v, b = X[cols], np.abs(X[cols])
+        for f in reversed(fs):
+            v, b = f @ v, np.abs(f) @ b
+        Y[rows] += v
+        B[rows] += b
+    return Y, B
+
+
+@pytest.mark.parametrize("wi_bytes", [0, 512, 4096])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_single_and_batched(gpu, shape, precision, wi_bytes):
+    import torch
+    S = SyntheticHmat(*shape)
+    set_tuning(wi_bytes, wi_bytes)
+    try:
+        dev = HipHmat(S, precisions=(precision,), adjoint=True)
+    finally:
+        set_tuning(0, 0)
+    for adjoint in (False, True):
+        n_in = dev.n_rows if adjoint else dev.n_cols
+        print(f"work items {shape} {precision} wi {wi_bytes} adjoint {adjoint}", flush=True)
+        X = np.random.default_rng(sum(shape)).uniform(-1, 1, (n_in, 32))
+        Y, bound = _reference(S, X, adjoint)
+        terms = n_in + int(S.lr_pattern[:, 5].sum()) + 8
+        tol = 2 * terms * U[precision] * bound
+        Xd = torch.from_numpy(X).to(gpu)
+        got = dev.matvec_batched(Xd, original=False, precision=precision, adjoint=adjoint)
+        assert np.all(np.abs(got.cpu().numpy() - Y) <= tol)
+        for j in (0, 31):
+            for u in (4, 8):
+                dev.set_unroll(u, u)
+                y = dev.matvec(Xd[:, j].contiguous(), original=False, precision=precision,
+                               adjoint=adjoint)
+                assert np.all(np.abs(y.cpu().numpy() - Y[:, j]) <= tol[:, j]), (j, u)
