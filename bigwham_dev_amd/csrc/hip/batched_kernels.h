@@ -4,7 +4,12 @@
 //
 // The slab layout serves as the A operand without change.  NB is the width of
 // the gathered input XB[z][NB] (row-major) and of t; a call runs its columns
-// in rounds of NB, columns past nk are zero and never stored.
+// in rounds of NB, columns past nk are zero and never stored.  Rounds of 16
+// columns move half the input rows and partial sums of 32 (6 912 DoF, FP64 82
+// -> 65 us, FP32 61 -> 41); in FP32 a round of 64 streams the factors once for
+// twice the columns (24 300 DoF 333 -> 252 us, 49 152 DoF 612 -> 476), and wins
+// from 33 columns on (306 + 257 -> 473).  FP64 stays at 32: its time goes with
+// the columns (159 us for one vector, 237 for 16 columns, 275 for 32).
 //
 // A workgroup of W waves takes one work item: the waves take contiguous
 // shares of its k-steps, each with a full set of accumulators, and the sums
@@ -17,20 +22,34 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef double dblx4 __attribute__((ext_vector_type(4)));
 
+// Rows of XB that a gather writes: x rows 0 .. n - 1, and zeros in the gap up
+// to row t0 and in the tail t1 .. size - 1, which padded column groups read.
+// (Every call writes them, so that rounds of different widths share a buffer.)
+struct GatherRows {
+  int64_t n, t0, t1, size;
+
+  int64_t count() const { return t0 + (size - t1); }
+  __device__ __forceinline__ int64_t row(int64_t i) const { return i < t0 ? i : t1 + (i - t0); }
+};
+
 template <typename T, int NB>
 __global__ __launch_bounds__(256) void k_gather_b(const double* __restrict__ X, int64_t xr,
                                                   int64_t xc, int nrhs, T* __restrict__ XB,
-                                                  int64_t n, const int64_t* __restrict__ perm,
+                                                  GatherRows g, const int64_t* __restrict__ perm,
                                                   int dof) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * (256 / NB) + threadIdx.x / NB;
+  const int64_t i = g.row(static_cast<int64_t>(blockIdx.x) * (256 / NB) + threadIdx.x / NB);
   const int c = threadIdx.x % NB;
-  if (i >= n) return;
-  int64_t src = i;
-  if (perm) {
-    const int64_t p = i / dof;
-    src = dof * perm[p] + (i - p * dof);
+  if (i >= g.size) return;
+  T v = 0;
+  if (i < g.n && c < nrhs) {
+    int64_t src = i;
+    if (perm) {
+      const int64_t p = i / dof;
+      src = dof * perm[p] + (i - p * dof);
+    }
+    v = static_cast<T>(X[src * xr + c * xc]);
   }
-  XB[i * NB + c] = c < nrhs ? static_cast<T>(X[src * xr + c * xc]) : T(0);
+  XB[i * NB + c] = v;
 }
 
 // The same gather for a row-major X (unit column stride, even row stride,
@@ -38,26 +57,29 @@ __global__ __launch_bounds__(256) void k_gather_b(const double* __restrict__ X, 
 // loads and one 16-byte (FP32) or two (FP64) stores per thread.
 template <typename T, int NB>
 __global__ __launch_bounds__(256) void k_gather_b4(const double* __restrict__ X, int64_t xr,
-                                                   int nrhs, T* __restrict__ XB, int64_t n,
+                                                   int nrhs, T* __restrict__ XB, GatherRows g,
                                                    const int64_t* __restrict__ perm, int dof) {
   constexpr int TPR = NB / 4;  // threads per row
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * (256 / TPR) + threadIdx.x / TPR;
+  const int64_t i = g.row(static_cast<int64_t>(blockIdx.x) * (256 / TPR) + threadIdx.x / TPR);
   const int c0 = 4 * (threadIdx.x % TPR);
-  if (i >= n) return;
-  int64_t src = i;
-  if (perm) {
-    const int64_t p = i / dof;
-    src = dof * perm[p] + (i - p * dof);
-  }
-  const double* __restrict__ row = X + src * xr + c0;
-  double v[4];
-  if (c0 + 4 <= nrhs) {
-    const dbl2 a = *reinterpret_cast<const dbl2*>(row);
-    const dbl2 b = *reinterpret_cast<const dbl2*>(row + 2);
-    v[0] = a.x; v[1] = a.y; v[2] = b.x; v[3] = b.y;
-  } else {
+  if (i >= g.size) return;
+  double v[4] = {0.0, 0.0, 0.0, 0.0};
+  if (i < g.n) {
+    int64_t src = i;
+    if (perm) {
+      const int64_t p = i / dof;
+      src = dof * perm[p] + (i - p * dof);
+    }
+    const double* __restrict__ row = X + src * xr + c0;
+    if (c0 + 4 <= nrhs) {
+      const dbl2 a = *reinterpret_cast<const dbl2*>(row);
+      const dbl2 b = *reinterpret_cast<const dbl2*>(row + 2);
+      v[0] = a.x; v[1] = a.y; v[2] = b.x; v[3] = b.y;
+    } else {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) v[k] = c0 + k < nrhs ? row[k] : 0.0;
+      for (int k = 0; k < 4; ++k)
+        if (c0 + k < nrhs) v[k] = row[k];
+    }
   }
   T* dst = XB + i * NB + c0;
   if constexpr (sizeof(T) == 4) {
@@ -277,7 +299,8 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(NC > 1 ?
 k_slab_mfma32(const bwl::WorkItem* __restrict__ wis, XcdSplit xs,
               const int32_t* __restrict__ gidx, const float* __restrict__ data,
               const float* __restrict__ XB, BatchOut<float> o) {
-  constexpr int NB = 32 * NC, KU = 2, D = 3, G = 2 * KU;
+  // the 64-wide kernel holds twice the accumulators: smaller, deeper ring
+  constexpr int NB = 32 * NC, KU = NC > 1 ? 1 : 2, D = NC > 1 ? 4 : 3, G = 2 * KU;
   __shared__ __align__(16) float lds[W * 32 * NB];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
@@ -322,9 +345,9 @@ k_slab_mfma32(const bwl::WorkItem* __restrict__ wis, XcdSplit xs,
 }
 
 // 16-row tiles: v_mfma_f64_16x16x4f64 and v_mfma_f32_16x16x4f32.  One k-step
-// covers four column groups: lane l reads the 16-byte vector of row l % 16
-// (of each tile) in group 4 step + l / 16, and element s of it is A[i][k] of
-// MFMA s with i = l % 16, k = l / 16; B[k][n] = XB[z(group) + s][n], n = l % 16
+// covers four column groups: as a tile's A operand lane l holds the 16-byte
+// vector of row l % 16 in group 4 step + l / 16, and element s of it is A[i][k]
+// of MFMA s with i = l % 16, k = l / 16; B[k][n] = XB[z(group) + s][n], n = l % 16
 // (+ 16 per column tile).
 template <typename T>
 struct Mfma16;
@@ -360,7 +383,7 @@ __device__ __forceinline__ void mfma16_stream(const typename Vec<T>::type* __res
   int rowc[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) rowc[t] = min(16 * t + i16, R - 1);
-  const int nsteps = (ng + 3) >> 2;  // four groups per k-step
+  const int nsteps = (ng + 3) >> 2;
   VT a[D][NT];
   T b[D][NC][V];
   int zz[D];  // input offset of the step buffer q is refilled with next
@@ -375,7 +398,20 @@ __device__ __forceinline__ void mfma16_stream(const typename Vec<T>::type* __res
 #pragma unroll
       for (int c = 0; c < NC; ++c) bb[c][s] = XB[zo + s * NB + 16 * c];
   };
-  auto compute = [&](int step, const VT (&aa)[NT], const T (&bb)[NC][V]) {
+  // FP32: sums of two steps, added to acc after them (short chains, as in
+  // mfma32_stream: 900-DoF mode-1, 5 right-hand sides, errors against 64 bits
+  // 1.4e-7 with chains of a whole trip)
+  constexpr bool kTrip = sizeof(T) == 4;
+  typename Mfma16<T>::acc_t p[kTrip ? NT : 1][NC];
+  auto flush = [&]() {
+    if constexpr (kTrip) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) acc[t][c] += p[t][c];
+    }
+  };
+  auto compute = [&](int step, bool first, const VT (&aa)[NT], const T (&bb)[NC][V]) {
     const bool ok = 4 * step + kq < ng;
 #pragma unroll
     for (int s = 0; s < V; ++s)
@@ -383,7 +419,13 @@ __device__ __forceinline__ void mfma16_stream(const typename Vec<T>::type* __res
       for (int c = 0; c < NC; ++c) {
         const T bv = ok ? bb[c][s] : T(0);
 #pragma unroll
-        for (int t = 0; t < NT; ++t) acc[t][c] = Mfma16<T>::mfma(aa[t][s], bv, acc[t][c]);
+        for (int t = 0; t < NT; ++t) {
+          if constexpr (kTrip)
+            p[t][c] = Mfma16<T>::mfma(
+                aa[t][s], bv, first && s == 0 ? typename Mfma16<T>::acc_t{0, 0, 0, 0} : p[t][c]);
+          else
+            acc[t][c] = Mfma16<T>::mfma(aa[t][s], bv, acc[t][c]);
+        }
       }
   };
 #pragma unroll
@@ -399,10 +441,14 @@ __device__ __forceinline__ void mfma16_stream(const typename Vec<T>::type* __res
     for (int j = 0; j < D; ++j) {
       const int st = s0 + j;
       __builtin_amdgcn_sched_barrier(0);
-      compute(st, a[j], b[j]);  // past the last step: B = 0, adds nothing
+      compute(st, j % 2 == 0, a[j], b[j]);  // past the last step: B = 0, adds nothing
       __builtin_amdgcn_sched_barrier(0);
       load(st + D, zz[j], a[j], b[j]);
       zz[j] = gz(st + 2 * D);
+      if (j % 2 == 1 || j == D - 1) {
+        __builtin_amdgcn_sched_barrier(0);
+        flush();
+      }
     }
   }
   __builtin_amdgcn_sched_barrier(0);

@@ -64,7 +64,6 @@ int fail(int code, const std::string& m) {
 #include "slab_kernels.h"
 #include "batched_kernels.h"
 
-constexpr int kRhs = 32;        // right-hand sides per round of the batched product
 // Waves per workgroup of the batched kernels: 8 are 4-15 % slower (32 right-hand
 // sides, FP64, 24 300 DoF: 307 us against 293; FP32, 49 152 DoF: 357 / 331).
 constexpr int kBatchWaves = 4;
@@ -107,14 +106,16 @@ struct DevOp {
 
 // What one matvec of an operator writes: xt (x gathered in the factor
 // precision, then t = B x), the partial sums of split work items of both
-// passes, and the same for the batched products (xt_size x kRhs input and
-// rank rows, partial sums x kRhs).  xt and xb are zero where no kernel writes
-// (the gap after x and the tail after t, which padded column groups read).
+// passes, and the same for the batched products (xt_size x xb_cols input and
+// rank rows, partial sums x xb_cols).  xt is zero where no kernel writes (the
+// gap after x and the tail after t, which padded column groups read); the
+// batched gather writes those rows of xb itself.
 struct OpScratch {
   void* xt = nullptr;
   void* part[2] = {nullptr, nullptr};
   void* xb = nullptr;
   void* partb[2] = {nullptr, nullptr};
+  int xb_cols = 0;  // widest round the batched scratch holds
 };
 
 // The scratch of one stream (or of one captured graph): per operator, plus
@@ -416,9 +417,9 @@ hipError_t zero_now(void* p, size_t bytes) {
 }
 
 // Allocates what `ctx` lacks for operator [adj][fp32]: the single-vector
-// scratch, and with `batched` the kRhs-wide one.  xt / xb are zeroed here,
-// once (synchronously, before any kernel of the context can use them): the
-// kernels only ever write x and t entries, so the gap and tail stay zero.
+// scratch, and with `batched` the batched one.  xt is zeroed here, once
+// (synchronously, before any kernel of the context can use it): the kernels
+// only ever write x and t entries, so the gap and tail stay zero.
 // On failure nothing of this call stays allocated.
 int ensure_op_scratch(bw_hip_handle* hd, StreamCtx* ctx, int adj, int fp32, bool batched) {
   const DevOp& op = hd->op[adj][fp32];
@@ -445,21 +446,29 @@ int ensure_op_scratch(bw_hip_handle* hd, StreamCtx* ctx, int adj, int fp32, bool
     s.part[1] = part[1];
   }
   if (batched && !s.xb) {
-    const size_t mark_b = ctx->allocs.size();
-    void* xb = nullptr;
-    void* partb[2] = {nullptr, nullptr};
-    if ((rc = dev_alloc(&xb, static_cast<size_t>(op.xt_size) * kRhs * es, &ctx->allocs, "scratch")))
-      return undo_allocs(ctx, mark_b, rc);
-    for (int p = 0; p < 2; ++p)
-      if ((rc = dev_alloc(&partb[p], static_cast<size_t>((p ? op.p2 : op.p1).batched.part_elems) * kRhs * es,
-                          &ctx->allocs, "scratch")))
-        return undo_allocs(ctx, mark_b, rc);
-    const hipError_t e = zero_now(xb, static_cast<size_t>(op.xt_size) * kRhs * es);
-    if (e != hipSuccess)
-      return undo_allocs(ctx, mark_b, fail(BW_EHIP, std::string("scratch: zero fill: ") + hipGetErrorString(e)));
-    s.xb = xb;
-    s.partb[0] = partb[0];
-    s.partb[1] = partb[1];
+    // FP32 calls of more than 32 columns run 64 at a time where the scratch and
+    // the kernels' 32-bit offsets allow it; everything else needs 32 columns
+    int cols = fp32 && op.xt_size * 64 <= static_cast<int64_t>(UINT32_MAX) ? 64 : 32;
+    for (;; cols = 32) {
+      const size_t mark_b = ctx->allocs.size();
+      void* xb = nullptr;
+      void* partb[2] = {nullptr, nullptr};
+      rc = dev_alloc(&xb, static_cast<size_t>(op.xt_size) * cols * es, &ctx->allocs, "scratch");
+      for (int p = 0; p < 2 && !rc; ++p)
+        rc = dev_alloc(&partb[p],
+                       static_cast<size_t>((p ? op.p2 : op.p1).batched.part_elems) * cols * es,
+                       &ctx->allocs, "scratch");
+      if (rc) {
+        undo_allocs(ctx, mark_b, rc);
+        if (cols > 32) continue;
+        return rc;
+      }
+      s.xb = xb;
+      s.partb[0] = partb[0];
+      s.partb[1] = partb[1];
+      s.xb_cols = cols;
+      break;
+    }
   }
   return BW_OK;
 }
@@ -1146,8 +1155,8 @@ int check_batched(bw_hip_handle* hd, bool adjoint, int nrhs, const double* X, in
                                     : "matvec_batched: precision not built");
   if (leading_dims && (xc < op.n_in || yc < op.n_out))
     return fail(BW_ESHAPE, "matvec_batched: leading dimension too small");
-  // the MFMA kernels index the kRhs-wide input rows with 32-bit offsets
-  if (op.xt_size * kRhs > static_cast<int64_t>(UINT32_MAX))
+  // the MFMA kernels index the 32-wide input rows with 32-bit offsets
+  if (op.xt_size * 32 > static_cast<int64_t>(UINT32_MAX))
     return fail(BW_ESHAPE, "matvec_batched: input plus rank entries exceed 2^32 / 32");
   // distinct outputs must not share an address: columns apart by at least a
   // column's extent, or rows apart by at least a row's
@@ -1157,75 +1166,89 @@ int check_batched(bw_hip_handle* hd, bool adjoint, int nrhs, const double* X, in
   return BW_OK;
 }
 
-// The MFMA kernel and the reduction of one pass of the batched product.
-template <int PASS>
-void launch_mfma(const DevPass& dp, hipStream_t st, const float* xb, const BatchOut<float>& o) {
-  const DevItems& di = dp.batched;
-  hipLaunchKernelGGL((k_slab_mfma32<PASS, kRhs / 32, kBatchWaves>), dim3(di.blocks),
-                     dim3(64 * kBatchWaves), 0, st, di.wis, di.xs, dp.gidx,
-                     static_cast<const float*>(dp.data), xb, o);
-}
-template <int PASS>
-void launch_mfma(const DevPass& dp, hipStream_t st, const double* xb, const BatchOut<double>& o) {
-  const DevItems& di = dp.batched;
-  hipLaunchKernelGGL((k_slab_mfma16<double, PASS, kRhs / 16, kBatchWaves>), dim3(di.blocks),
-                     dim3(64 * kBatchWaves), 0, st, di.wis, di.xs, dp.gidx,
-                     static_cast<const double*>(dp.data), xb, o);
-}
-template <int PASS, typename T>
+// The MFMA kernel and the reduction of one pass of a round of NB columns.
+template <int PASS, int NB, typename T>
 void launch_batched_pass(const DevPass& dp, hipStream_t st, const T* xb, const BatchOut<T>& o) {
   const DevItems& di = dp.batched;
-  if (di.nwi > 0) launch_mfma<PASS>(dp, st, xb, o);
+  const dim3 grid(di.blocks), block(64 * kBatchWaves);
+  const T* data = static_cast<const T*>(dp.data);
+  if (di.nwi > 0) {
+    if constexpr (sizeof(T) == 4 && NB >= 32)
+      hipLaunchKernelGGL((k_slab_mfma32<PASS, NB / 32, kBatchWaves>), grid, block, 0, st, di.wis,
+                         di.xs, dp.gidx, data, xb, o);
+    else
+      hipLaunchKernelGGL((k_slab_mfma16<T, PASS, NB / 16, kBatchWaves>), grid, block, 0, st, di.wis,
+                         di.xs, dp.gidx, data, xb, o);
+  }
   if (di.nred > 0)
-    hipLaunchKernelGGL((k_reduce_b<PASS, kRhs, T>), dim3(di.nred), dim3(256), 0, st, di.reds,
+    hipLaunchKernelGGL((k_reduce_b<PASS, NB, T>), dim3(di.nred), dim3(256), 0, st, di.reds,
                        di.nred, o);
 }
 
-// The kernels of Y = H X (kRhs right-hand sides per round) on stream st,
-// writing only the batched scratch `s`.
-template <typename T>
-int launch_batched(bw_hip_handle* hd, DevOp& op, const OpScratch& s, int nrhs, const double* X,
-                   int64_t xr, int64_t xc, double* Y, int64_t yr, int64_t yc, int ordering,
-                   hipStream_t st) {
-  constexpr int NB = kRhs;
-  const bool orig = ordering == BW_ORDER_ORIGINAL;
+// One round: columns 0 .. nk - 1 (nk <= NB) of X and Y, writing only the
+// batched scratch `s`.
+template <typename T, int NB>
+int launch_round(bw_hip_handle* hd, const DevOp& op, const OpScratch& s, int nk, const double* X,
+                 int64_t xr, int64_t xc, double* Y, int64_t yr, int64_t yc, bool orig,
+                 hipStream_t st) {
   const int dof = hd->dof;
   const int64_t* pin = orig ? op.perm_in : nullptr;
   T* xb = static_cast<T*>(s.xb);
-  for (int k0 = 0; k0 < nrhs; k0 += NB) {
-    const int nk = std::min(NB, nrhs - k0);
+  const GatherRows g{op.n_in, op.xt_t, op.xt_t + op.t_total, op.xt_size};
+  // row-major input (unit column stride, even row stride, 16-byte aligned
+  // rows): the vector gather
+  const bool rowmajor = xc == 1 && xr % 2 == 0 && reinterpret_cast<uintptr_t>(X) % 16 == 0;
+  const int rows = rowmajor ? 256 / (NB / 4) : 256 / NB;  // per workgroup
+  const dim3 gblocks(static_cast<unsigned>((g.count() + rows - 1) / rows));
+  if (rowmajor)
+    hipLaunchKernelGGL((k_gather_b4<T, NB>), gblocks, dim3(256), 0, st, X, xr, nk, xb, g, pin, dof);
+  else
+    hipLaunchKernelGGL((k_gather_b<T, NB>), gblocks, dim3(256), 0, st, X, xr, xc, nk, xb, g, pin,
+                       dof);
+  BatchOut<T> o1{};
+  o1.tout = xb;
+  o1.nk = NB;
+  o1.part = static_cast<T*>(s.partb[0]);
+  o1.dof = dof;
+  o1.rowmap = op.p1.rowmap;
+  BatchOut<T> o2{};
+  o2.Y = Y;
+  o2.yr = yr;
+  o2.yc = yc;
+  o2.nk = nk;
+  o2.yvec = yc == 1 && yr % 2 == 0 && reinterpret_cast<uintptr_t>(Y) % 16 == 0;
+  o2.part = static_cast<T*>(s.partb[1]);
+  o2.perm = orig ? op.perm_out : nullptr;
+  o2.dof = dof;
+  launch_batched_pass<1, NB>(op.p1, st, xb, o1);
+  launch_batched_pass<2, NB>(op.p2, st, xb, o2);
+  HIPCHK(hipGetLastError());
+  return BW_OK;
+}
+
+// Y = H X on stream st in rounds of 64 (FP32), 32 or 16 columns.
+template <typename T>
+int launch_batched(bw_hip_handle* hd, const DevOp& op, const OpScratch& s, int nrhs,
+                   const double* X, int64_t xr, int64_t xc, double* Y, int64_t yr, int64_t yc,
+                   int ordering, hipStream_t st) {
+  const bool orig = ordering == BW_ORDER_ORIGINAL;
+  for (int k0 = 0; k0 < nrhs;) {
+    const int left = nrhs - k0;
     const double* Xk = X + static_cast<int64_t>(k0) * xc;
     double* Yk = Y + static_cast<int64_t>(k0) * yc;
-    // row-major input (unit column stride, even row stride, 16-byte aligned
-    // rows): the vector gather
-    const bool rowmajor = xc == 1 && xr % 2 == 0 && reinterpret_cast<uintptr_t>(Xk) % 16 == 0;
-    if (rowmajor) {
-      constexpr int rows = 256 / (NB / 4);
-      hipLaunchKernelGGL((k_gather_b4<T, NB>), dim3(static_cast<int>((op.n_in + rows - 1) / rows)),
-                         dim3(256), 0, st, Xk, xr, nk, xb, op.n_in, pin, dof);
+    int rc, nk;
+    if (sizeof(T) == 4 && left > 32 && s.xb_cols >= 64) {
+      nk = std::min(64, left);
+      rc = launch_round<float, 64>(hd, op, s, nk, Xk, xr, xc, Yk, yr, yc, orig, st);
+    } else if (left > 16) {
+      nk = std::min(32, left);
+      rc = launch_round<T, 32>(hd, op, s, nk, Xk, xr, xc, Yk, yr, yc, orig, st);
     } else {
-      constexpr int rows = 256 / NB;
-      hipLaunchKernelGGL((k_gather_b<T, NB>), dim3(static_cast<int>((op.n_in + rows - 1) / rows)),
-                         dim3(256), 0, st, Xk, xr, xc, nk, xb, op.n_in, pin, dof);
+      nk = left;
+      rc = launch_round<T, 16>(hd, op, s, nk, Xk, xr, xc, Yk, yr, yc, orig, st);
     }
-    BatchOut<T> o1{};
-    o1.tout = xb;
-    o1.nk = NB;
-    o1.part = static_cast<T*>(s.partb[0]);
-    o1.dof = dof;
-    o1.rowmap = op.p1.rowmap;
-    BatchOut<T> o2{};
-    o2.Y = Yk;
-    o2.yr = yr;
-    o2.yc = yc;
-    o2.nk = nk;
-    o2.yvec = yc == 1 && yr % 2 == 0 && reinterpret_cast<uintptr_t>(Yk) % 16 == 0;
-    o2.part = static_cast<T*>(s.partb[1]);
-    o2.perm = orig ? op.perm_out : nullptr;
-    o2.dof = dof;
-    launch_batched_pass<1>(op.p1, st, xb, o1);
-    launch_batched_pass<2>(op.p2, st, xb, o2);
-    HIPCHK(hipGetLastError());
+    if (rc) return rc;
+    k0 += nk;
   }
   return BW_OK;
 }

@@ -402,8 +402,8 @@ class HipHmat:
 
     def matvec_batched(self, X, original: bool = True, precision: str = "fp64", out=None,
                        adjoint: bool = False):
-        """Y = H X (or H^T X) for a (n, k) float64 CUDA tensor, 32 columns per
-        MFMA tile.  X may have any positive strides (row-major, column-major,
+        """Y = H X (or H^T X) for a (n, k) float64 CUDA tensor, in rounds of
+        16, 32 or (FP32) 64 columns.  X may have any positive strides (row-major, column-major,
         a column slice) and is read in place; Y is row-major like torch's
         default unless ``out`` (an (n_out, k) float64 tensor) is given."""
         import torch

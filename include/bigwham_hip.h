@@ -118,8 +118,8 @@ int bw_hip_rmatvec(bw_hip_handle* hd, const double* x, double* y, int ordering,
 
 /* Y = H X for nrhs right-hand sides.  X is (n_cols x nrhs) column-major with
  * leading dimension ldx, Y (n_rows x nrhs) with ldy; device pointers only.
- * Both precisions run the passes as thin GEMMs on MFMA, 32 right-hand sides
- * per tile (FP32: v_mfma_f32_32x32x2f32; FP64: v_mfma_f64_16x16x4f64, same
+ * Both precisions run the passes as thin GEMMs on MFMA, in rounds of
+ * 16 or 32 right-hand sides (FP32 also 64) (FP32: v_mfma_f32_32x32x2f32; FP64: v_mfma_f64_16x16x4f64, same
  * summation bar as the single-RHS FP64 path). */
 int bw_hip_matvec_batched(bw_hip_handle* hd, int nrhs, const double* X, int64_t ldx,
                           double* Y, int64_t ldy, int ordering, int precision,
@@ -164,7 +164,7 @@ int bw_hip_graph_create(bw_hip_handle* hd, const double* x, double* y, int order
                         int precision, int adjoint, bw_hip_graph** out);
 /* The batched product of bw_hip_matvec_batched_strided (same arguments and
  * checks) on fixed device operands X, Y, captured as one graph: every
- * 32-column round of both passes replays with one launch.  No counterpart in
+ * round of columns of both passes replays with one launch.  No counterpart in
  * the reference. */
 int bw_hip_graph_create_batched(bw_hip_handle* hd, int adjoint, int nrhs, const double* X,
                                 int64_t x_row_stride, int64_t x_col_stride, double* Y,

@@ -1,8 +1,9 @@
 """Work items shared by the waves of a workgroup, at the sizes where the split
 can go wrong: slabs of 1 to 64 rows (edges of the 16- and 32-row tiles), items
 of fewer column groups than a workgroup has waves, remainders of every batch
-depth, whole slabs and slabs split over several items, against the operator's
-blocks multiplied in numpy.
+depth, whole slabs and slabs split over several items; and rounds of every
+width of the batched product (16, 32 and 64 columns and their edges) in any
+order on one handle, against the operator's blocks multiplied in numpy.
 
 The tolerance is the a-priori bound of a sum of products in the working
 precision: |y - H x| <= n u (|F| |x| + |A| (|B| |x|)) with n the terms of the
@@ -68,3 +69,26 @@ def test_single_and_batched(gpu, shape, precision, wi_bytes):
                 y = dev.matvec(Xd[:, j].contiguous(), original=False, precision=precision,
                                adjoint=adjoint)
                 assert np.all(np.abs(y.cpu().numpy() - Y[:, j]) <= tol[:, j]), (j, u)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("shape", [(95, 140, 2, 2), (64, 200, 3, 3), (40, 33, 3, 6)])
+def test_round_widths(gpu, shape, precision):
+    """Column counts at the edges of the rounds, wide before narrow and back
+    (the rounds share one scratch buffer), row- and column-major operands."""
+    import torch
+    S = SyntheticHmat(*shape)
+    dev = HipHmat(S, precisions=(precision,))
+    terms = dev.n_cols + int(S.lr_pattern[:, 5].sum()) + 8
+    for k in (64, 1, 33, 16, 17, 48, 15, 65, 32, 100, 7):
+        X = np.random.default_rng(k).uniform(-1, 1, (dev.n_cols, k))
+        Y, bound = _reference(S, X, False)
+        tol = 2 * terms * U[precision] * bound
+        Xd = torch.from_numpy(X).to(gpu)
+        Xc = torch.from_numpy(np.ascontiguousarray(X.T)).to(gpu).t()
+        print(f"round widths {shape} {precision} k {k}", flush=True)
+        got = dev.matvec_batched(Xd, original=False, precision=precision)
+        assert np.all(np.abs(got.cpu().numpy() - Y) <= tol), k
+        out = torch.full((k, dev.n_rows), np.nan, dtype=torch.float64, device=gpu).t()
+        dev.matvec_batched(Xc, original=False, precision=precision, out=out)
+        assert torch.equal(out, got), k
