@@ -304,7 +304,7 @@ k_slab_mfma32(const bwl::WorkItem* __restrict__ wis, XcdSplit xs,
   __shared__ __align__(16) float lds[W * 32 * NB];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-  const int w = xcd_work_item(xs);
+  const int w = xcd_work_item(xs, blockIdx.x);
   if (w < 0) return;
   const bwl::WorkItem wi = wis[w];
   const int R = __builtin_amdgcn_readfirstlane(wi.rows);
@@ -464,7 +464,7 @@ k_slab_mfma16(const bwl::WorkItem* __restrict__ wis, XcdSplit xs,
   __shared__ __align__(16) T lds[W * 32 * NB];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-  const int w = xcd_work_item(xs);
+  const int w = xcd_work_item(xs, blockIdx.x);
   if (w < 0) return;
   const bwl::WorkItem wi = wis[w];
   const int R = wi.rows;

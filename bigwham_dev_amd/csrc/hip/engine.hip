@@ -1,10 +1,11 @@
 // MI355X (gfx950) hierarchical-matrix matvec engine and its C-ABI.
 //
-// One matvec y = H x is three to five kernels on the caller's stream:
+// One matvec y = H x is two to five kernels on the caller's stream:
 //   k_gather   x -> xt[0:n]   (permutation of matvecOriginal, hmat.cc:586-593,
 //                              or a copy; converts to the factor precision)
 //   k_slab     pass 1: t = W x   (W_k = B_k), each row written through the
 //              row map into xt[xt_t : ...]
+//              (small operators: k_slab_gather does both)
 //   k_reduce   sum of split pass-1 work items (only if any)
 //   k_slab     pass 2: y = F x + U t, each y row written once, with the
 //              permutation of matvecOriginal (hmat.cc:618-626) fused in
@@ -82,6 +83,7 @@ struct DevItems {
 
 struct DevPass {
   DevItems single, batched;
+  int gather_cols = 0;        // pass 1: longest work item's columns if it may gather x itself
   int32_t* gidx = nullptr;
   int32_t* rowmap = nullptr;  // pass 1: t entry of every slab row
   void* data = nullptr;
@@ -364,6 +366,15 @@ struct bw_hip_handle {
 
 namespace {
 
+// Pass 1 gathers x itself where its longest work item's input fits this much
+// LDS (two workgroups stay on a compute unit) and the pass is at most this
+// long: the gather launch it saves is 3.3 us where launches bound the call and
+// 1-2 us behind a longer pass, while reading x through the permutation once per
+// work item grows with the pass (16 M entries 68.3 -> 66.0 us a matvec, 46 M
+// 157.0 -> 157.2, FP32 43 M 91.6 -> 92.1).
+constexpr size_t kGatherLds = 48 << 10;
+constexpr int64_t kGatherEntries = 24 << 20;
+
 template <typename T>
 int build_op(bw_hip_handle* hd, const bw_flat_hmat* h, bool adjoint, hipStream_t st) {
   DevOp& op = hd->op[adjoint ? 1 : 0][sizeof(T) == 4 ? 1 : 0];
@@ -382,6 +393,10 @@ int build_op(bw_hip_handle* hd, const bw_flat_hmat* h, bool adjoint, hipStream_t
   if ((rc = upload_pass<T>(L, L.pass1, &op.p1, st, &hd->allocs))) return rc;
   if ((rc = upload_pass<T>(L, L.pass2, &op.p2, st, &hd->allocs))) return rc;
   op.elem = sizeof(T);
+  int cols = 0;  // columns of the longest pass-1 work item
+  for (const bwl::WorkItem& w : L.pass1.single.wis) cols = std::max(cols, w.ngroups * opt.vec_elems);
+  if (cols * sizeof(T) <= kGatherLds && L.pass1.data_elems <= kGatherEntries)
+    op.p1.gather_cols = cols;
   op.xt_size = L.xt_size;
   op.xt_t = L.xt_t;
   op.t_total = L.view.t_total;
@@ -552,6 +567,27 @@ void launch_slab(const DevPass& dp, int unroll, hipStream_t st, const T* xin, Ou
 #undef BW_SLAB
 }
 
+// Pass 1 with the gather of x in the same launch (DevPass::gather_cols > 0).
+template <typename T>
+void launch_slab_gather(const DevPass& dp, int unroll, hipStream_t st, const double* x, T* xt,
+                        int64_t n_in, T* part, const int64_t* perm, int dof) {
+  constexpr int W = 8;
+  const DevItems& di = dp.single;
+  // a multiple of 8, so that work items keep their XCD
+  const int ngather =
+      static_cast<int>(std::min<int64_t>(256, (n_in + 8 * 64 * W - 1) / (8 * 64 * W) * 8));
+  const size_t lds = (dp.gather_cols + 64 * W) * sizeof(T);
+#define BW_SLAB(U)                                                                             \
+  hipLaunchKernelGGL((k_slab_gather<T, U, W>), dim3(ngather + di.blocks), dim3(64 * W), lds, st, \
+                     di.wis, di.xs, dp.gidx, static_cast<const T*>(dp.data), x, xt,             \
+                     static_cast<int>(n_in), perm, dof, ngather, dp.gather_cols, part, dp.rowmap)
+  if (unroll == 4)
+    BW_SLAB(4);
+  else
+    BW_SLAB(8);
+#undef BW_SLAB
+}
+
 // Zero fill of xt's gap after x and its tail after t, for scratch that other
 // operators may have used before (the no-allocation entry point).
 template <typename T>
@@ -579,6 +615,7 @@ int launch_matvec(bw_hip_handle* hd, DevOp& op, const OpScratch& s, double* y_fu
   double* const y_user = yd;
   if (sd) yd = y_full;  // the passes write the full permuted y
   const bool timing = timed && hd->timing;
+  const bool fused = !sd && op.p1.gather_cols > 0;  // pass 1 gathers x
   if (timing) (void)hipEventRecord(hd->ev[0], st);
   if (sd) {
     if (sd->n_pairs > 0) {
@@ -586,14 +623,17 @@ int launch_matvec(bw_hip_handle* hd, DevOp& op, const OpScratch& s, double* y_fu
       hipLaunchKernelGGL(k_scatter_sel<T>, dim3(blocks), dim3(256), 0, st, xd, xt, sd->in_src,
                          sd->in_dst, sd->n_pairs, dof);
     }
-  } else {
+  } else if (!fused) {
     const int64_t n = op.n_in;
     const int blocks = static_cast<int>((n + 255) / 256);
     hipLaunchKernelGGL(k_gather<T>, dim3(blocks), dim3(256), 0, st, xd, xt, n,
                        orig ? op.perm_in : nullptr, dof);
   }
   if (timing) (void)hipEventRecord(hd->ev[1], st);
-  if (op.p1.single.nwi > 0) {
+  if (fused) {
+    launch_slab_gather<T>(op.p1, op.unroll[0], st, xd, xt, op.n_in, part1,
+                          orig ? op.perm_in : nullptr, dof);
+  } else if (op.p1.single.nwi > 0) {
     launch_slab<T, T, 1>(op.p1, op.unroll[0], st, xt, xt, part1, nullptr, dof);
   }
   if (timing) (void)hipEventRecord(hd->ev[2], st);

@@ -27,9 +27,9 @@ struct XcdSplit {
   int32_t s[bwl::kXcds + 1];
 };
 
-__device__ __forceinline__ int xcd_work_item(const XcdSplit& xs) {
-  const int x = blockIdx.x % bwl::kXcds;
-  const int w = xs.s[x] + static_cast<int>(blockIdx.x / bwl::kXcds);
+__device__ __forceinline__ int xcd_work_item(const XcdSplit& xs, unsigned block) {
+  const int x = block % bwl::kXcds;
+  const int w = xs.s[x] + static_cast<int>(block / bwl::kXcds);
   return w < xs.s[x + 1] ? w : -1;
 }
 
@@ -56,13 +56,58 @@ __device__ __forceinline__ int64_t out_index(int64_t idx, const int64_t* perm, i
   return dof * perm[p] + (i - p * dof);
 }
 
+// Where a slab's input entries come from.  `off(g)` gives the offset of column
+// group g and `at(off, v)` entry v of it; `ready()` is called once per wave,
+// after its first factor loads have been requested and before the first `at`.
+//
+// From xt through the group offsets; tall slabs have wave-uniform offsets
+// (scalar loads).
+template <typename T, bool TALL>
+struct XtInput {
+  const int32_t* __restrict__ gi;
+  const T* __restrict__ xin;
+
+  __device__ __forceinline__ int off(int g) const { return gi[g]; }
+  __device__ __forceinline__ T at(int o, int v) const {
+    // unsigned: no sign extension of the loaded offset is placed (and waited
+    // for) next to its load
+    if constexpr (TALL)
+      return xin[static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(o)) + v];
+    else
+      return xin[o + v];
+  }
+  __device__ __forceinline__ void ready() const {}
+};
+
+// From LDS, where ready() puts the work item's whole input: the entries
+// z0 .. z0 + ncol - 1 of the permuted x, read from the caller's vector (pass 1
+// of small operators; a pass-1 slab's columns are one run).
+template <typename T, int THREADS>
+struct StagedInput {
+  static constexpr int V = Vec<T>::V;
+  T* lds;
+  int g0;  // the wave's first group within the work item
+  const double* __restrict__ x;
+  const int64_t* __restrict__ perm;
+  int dof;
+  int n_in, z0, ncol;
+
+  __device__ __forceinline__ int off(int g) const { return (g0 + g) * V; }
+  __device__ __forceinline__ T at(int o, int v) const { return lds[o + v]; }
+  __device__ __forceinline__ void ready() const {
+    for (int c = threadIdx.x; c < ncol; c += THREADS) {
+      const int z = z0 + c;  // past x: the zeros that xt holds there
+      lds[c] = z < n_in ? static_cast<T>(x[out_index<T>(z, perm, dof)]) : T(0);
+    }
+    __syncthreads();
+  }
+};
+
 // Dot products of a wave's column groups with more than 32 rows: one column
-// group per step for the whole wavefront, so the group offset and the input
-// entries are wave-uniform (scalar loads).  U: 16-byte loads in flight per lane.
-template <typename T, int U>
-__device__ __forceinline__ T dot_tall(const typename Vec<T>::type* __restrict__ p, int R,
-                                      const int32_t* __restrict__ gi, int ng,
-                                      const T* __restrict__ xin) {
+// group per step for the whole wavefront.  U: 16-byte loads in flight per lane.
+template <typename T, int U, typename In>
+__device__ __forceinline__ T dot_tall(const typename Vec<T>::type* __restrict__ p, int R, int ng,
+                                      const In& in) {
   typedef typename Vec<T>::type VT;
   constexpr int V = Vec<T>::V;
   T acc0 = 0, acc1 = 0;
@@ -77,26 +122,24 @@ __device__ __forceinline__ T dot_tall(const typename Vec<T>::type* __restrict__ 
     int za[U], zb[U];
     auto load = [&](int g0, VT (&buf)[U], int (&zz)[U]) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) zz[u] = gi[g0 + u];
+      for (int u = 0; u < U; ++u) zz[u] = in.off(g0 + u);
 #pragma unroll
       for (int u = 0; u < U; ++u) buf[u] = __builtin_nontemporal_load(p + (g0 + u) * R);
     };
     auto use = [&](const VT (&buf)[U], const int (&zz)[U]) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        // unsigned: no sign extension of the loaded offset is placed
-        // (and waited for) next to its load
-        const uint32_t z = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(zz[u]));
+      for (int u = 0; u < U; ++u)
 #pragma unroll
         for (int v = 0; v < V; ++v) {
           if (u & 1)
-            acc1 += buf[u][v] * xin[z + v];
+            acc1 += buf[u][v] * in.at(zz[u], v);
           else
-            acc0 += buf[u][v] * xin[z + v];
+            acc0 += buf[u][v] * in.at(zz[u], v);
         }
-      }
     };
     load(0, a, za);
+    __builtin_amdgcn_sched_barrier(0);
+    in.ready();
     int bt = 0;
     for (; bt + 2 < nfull; bt += 2) {
       __builtin_amdgcn_sched_barrier(0);
@@ -120,35 +163,32 @@ __device__ __forceinline__ T dot_tall(const typename Vec<T>::type* __restrict__ 
     }
     __builtin_amdgcn_sched_barrier(0);
   }
-  // The last, partial batch in one memory round trip: 4, 8 or U loads
-  // (clamped to the last group, in bounds), of which the first rem are used.
+  // The last, partial batch in one memory round trip: 4 or U loads (clamped
+  // to the last group, in bounds), of which the first rem are used.
   const int g = nfull * U, rem = ng - g;
   auto tail = [&](auto N) {
     constexpr int n = decltype(N)::value;
     VT a[n];
     int z[n];
 #pragma unroll
-    for (int u = 0; u < n; ++u) z[u] = gi[g + min(u, rem - 1)];
+    for (int u = 0; u < n; ++u) z[u] = in.off(g + min(u, rem - 1));
 #pragma unroll
     for (int u = 0; u < n; ++u) a[u] = __builtin_nontemporal_load(p + (g + min(u, rem - 1)) * R);
+    if (nfull == 0) in.ready();
 #pragma unroll
-    for (int u = 0; u < n; ++u) {
-      const uint32_t zu = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(z[u]));
+    for (int u = 0; u < n; ++u)
       if (u < rem) {
 #pragma unroll
         for (int v = 0; v < V; ++v) {
           if (u & 1)
-            acc1 += a[u][v] * xin[zu + v];
+            acc1 += a[u][v] * in.at(z[u], v);
           else
-            acc0 += a[u][v] * xin[zu + v];
+            acc0 += a[u][v] * in.at(z[u], v);
         }
       }
-    }
   };
-  if (rem > 8)
-    tail(std::integral_constant<int, (U > 8 ? U : 8)>{});
-  else if (rem > 4)
-    tail(std::integral_constant<int, (U > 4 ? 8 : 4)>{});
+  if (rem > 4)
+    tail(std::integral_constant<int, U>{});
   else if (rem > 0)
     tail(std::integral_constant<int, 4>{});
   return acc0 + acc1;
@@ -161,10 +201,9 @@ __device__ __forceinline__ T dot_tall(const typename Vec<T>::type* __restrict__ 
 // buffers; the input offsets are loaded two steps ahead, so that one memory
 // round trip covers a step.  Offsets and groups past the end are clamped (in
 // bounds) and not used.
-template <typename T, int U>
+template <typename T, int U, typename In>
 __device__ __forceinline__ T dot_short(const typename Vec<T>::type* __restrict__ p, int R,
-                                       int nsplit, int split, const int32_t* __restrict__ gi,
-                                       int ng, const T* __restrict__ xin) {
+                                       int nsplit, int split, int ng, const In& in) {
   typedef typename Vec<T>::type VT;
   constexpr int V = Vec<T>::V;
   T acc0 = 0, acc1 = 0;
@@ -175,16 +214,18 @@ __device__ __forceinline__ T dot_short(const typename Vec<T>::type* __restrict__
   int za[U], zb[U];
   auto load_z = [&](int s, int (&z)[U]) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) z[u] = gi[min(s * step + split + u * nsplit, ng - 1)];
+    for (int u = 0; u < U; ++u) z[u] = in.off(min(s * step + split + u * nsplit, ng - 1));
   };
-  auto load = [&](int s, VT (&f)[U], T (&x)[U][V], int (&z)[U]) {
+  auto load_a = [&](int s, VT (&f)[U]) {
 #pragma unroll
     for (int u = 0; u < U; ++u)
       f[u] = __builtin_nontemporal_load(p + min(s * step + split + u * nsplit, ng - 1) * R);
+  };
+  auto load_x = [&](int s, T (&x)[U][V], int (&z)[U]) {
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int v = 0; v < V; ++v) x[u][v] = xin[z[u] + v];
+      for (int v = 0; v < V; ++v) x[u][v] = in.at(z[u], v);
     load_z(s + 2, z);
   };
   auto use = [&](const VT (&f)[U], const T (&x)[U][V]) {
@@ -213,21 +254,27 @@ __device__ __forceinline__ T dot_short(const typename Vec<T>::type* __restrict__
   };
   load_z(0, za);
   load_z(1, zb);
-  load(0, a, xa, za);
+  load_a(0, a);
+  __builtin_amdgcn_sched_barrier(0);
+  in.ready();
+  load_x(0, xa, za);
   int s = 0;
   for (; s + 2 < n; s += 2) {
     __builtin_amdgcn_sched_barrier(0);
-    load(s + 1, b, xb, zb);
+    load_a(s + 1, b);
+    load_x(s + 1, xb, zb);
     __builtin_amdgcn_sched_barrier(0);
     use(a, xa);
     __builtin_amdgcn_sched_barrier(0);
-    load(s + 2, a, xa, za);
+    load_a(s + 2, a);
+    load_x(s + 2, xa, za);
     __builtin_amdgcn_sched_barrier(0);
     use(b, xb);
   }
   __builtin_amdgcn_sched_barrier(0);
   if (s + 2 == n) {
-    load(s + 1, b, xb, zb);
+    load_a(s + 1, b);
+    load_x(s + 1, xb, zb);
     __builtin_amdgcn_sched_barrier(0);
     use(a, xa);
     __builtin_amdgcn_sched_barrier(0);
@@ -236,6 +283,34 @@ __device__ __forceinline__ T dot_short(const typename Vec<T>::type* __restrict__
     use_last(a, xa);
   }
   return acc0 + acc1;
+}
+
+// Adds the column splits of a wave onto lanes 0..R-1, in split order.
+template <typename T>
+__device__ __forceinline__ T fold_splits(T acc, int R, int nsplit, int split, int lane) {
+  for (int s = 1; s < nsplit; ++s) {
+    const T o = __shfl(acc, lane + s * R, 64);
+    if (split == 0) acc += o;
+  }
+  return acc;
+}
+
+// The waves' sums of a work item added in wave order from LDS, and its rows
+// stored by the first wave (`orow`: the lane's output row, requested before
+// the stream).
+template <typename T, typename OutT, int W>
+__device__ __forceinline__ void wave_sum_put(T acc, T (*red)[64], const bwl::WorkItem& wi,
+                                             int wave, int lane, int64_t orow, OutT* out, T* part) {
+  const int R = wi.rows;
+  if (wave > 0 && lane < R) red[wave][lane] = acc;
+  __syncthreads();
+  if (wave > 0 || lane >= R) return;
+#pragma unroll
+  for (int k = 1; k < W; ++k) acc += red[k][lane];
+  if (wi.part_off < 0)
+    out[orow] = static_cast<OutT>(acc);
+  else  // split slab: the partial sums are added in work-item order by k_reduce
+    part[wi.part_off + lane] = acc;
 }
 
 // One workgroup of W waves per work item: the waves take equal contiguous
@@ -260,9 +335,10 @@ __global__ __launch_bounds__(64 * W) void k_slab(const bwl::WorkItem* __restrict
                                                  const int32_t* __restrict__ rowmap) {
   typedef typename Vec<T>::type VT;
   constexpr int V = Vec<T>::V;
+  __shared__ T red[W][64];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-  const int w = xcd_work_item(xs);
+  const int w = xcd_work_item(xs, blockIdx.x);
   if (w < 0) return;
   const bwl::WorkItem wi = wis[w];
   const int R = wi.rows;
@@ -273,7 +349,6 @@ __global__ __launch_bounds__(64 * W) void k_slab(const bwl::WorkItem* __restrict
   const VT* __restrict__ base =
       reinterpret_cast<const VT*>(data + wi.data_off + static_cast<int64_t>(g0) * R * V);
   const int32_t* __restrict__ gi = gidx + wi.gbeg + g0;
-  // output row of this lane, requested before the stream
   int64_t orow = 0;
   if (wave == 0 && wi.part_off < 0 && lane < R) {
     // pass 1 rows go to their t entries through the row map
@@ -282,33 +357,68 @@ __global__ __launch_bounds__(64 * W) void k_slab(const bwl::WorkItem* __restrict
   }
   T acc = 0;
   if (R > 32) {
-    if (lane < R && ng > 0) acc = dot_tall<T, U>(base + lane, R, gi, ng, xin);
+    if (lane < R && ng > 0) acc = dot_tall<T, U>(base + lane, R, ng, XtInput<T, true>{gi, xin});
   } else {
     const int nsplit = 64 / R;
     const int split = lane / R;
     if (split < nsplit && ng > 0)
-      acc = dot_short<T, 4>(base + (lane - split * R), R, nsplit, split, gi, ng, xin);
-    // fold the column splits onto lanes 0..R-1, in split order
-    for (int s = 1; s < nsplit; ++s) {
-      const T o = __shfl(acc, lane + s * R, 64);
-      if (split == 0) acc += o;
-    }
+      acc = dot_short<T, 4>(base + (lane - split * R), R, nsplit, split, ng,
+                            XtInput<T, false>{gi, xin});
+    acc = fold_splits(acc, R, nsplit, split, lane);
   }
-  if constexpr (W > 1) {
-    __shared__ T red[W][64];
-    if (wave > 0 && lane < R) red[wave][lane] = acc;
-    __syncthreads();
-    if (wave > 0) return;
-    if (lane < R) {
-#pragma unroll
-      for (int k = 1; k < W; ++k) acc += red[k][lane];
-    }
+  wave_sum_put<T, OutT, W>(acc, red, wi, wave, lane, orow, out, part);
+}
+
+// Pass 1 of small operators together with the gather of x: the first
+// `ngather` workgroups write the permuted x to xt for pass 2, the others take
+// the work items and stage their own input from the caller's vector in LDS
+// (lds_cols entries), behind the first factor loads.  A launch less where
+// launches count: 4 000-DoF 2DS0 operator 15.7 -> 12.6 us a matvec, 3 072-DoF
+// 3DR0 19.6 -> 16.2.
+template <typename T, int U, int W>
+__global__ __launch_bounds__(64 * W) void k_slab_gather(
+    const bwl::WorkItem* __restrict__ wis, XcdSplit xs, const int32_t* __restrict__ gidx,
+    const T* __restrict__ data, const double* __restrict__ x, T* __restrict__ xt, int n_in,
+    const int64_t* __restrict__ perm, int dof, int ngather, int lds_cols, T* __restrict__ part,
+    const int32_t* __restrict__ rowmap) {
+  typedef typename Vec<T>::type VT;
+  constexpr int V = Vec<T>::V;
+  extern __shared__ __align__(16) unsigned char smem[];
+  T* const stage = reinterpret_cast<T*>(smem);
+  T(*const red)[64] = reinterpret_cast<T(*)[64]>(stage + lds_cols);
+  if (blockIdx.x < static_cast<unsigned>(ngather)) {
+    for (int i = blockIdx.x * (64 * W) + threadIdx.x; i < n_in; i += ngather * (64 * W))
+      xt[i] = static_cast<T>(x[out_index<T>(i, perm, dof)]);
+    return;
   }
-  if (lane >= R) return;
-  if (wi.part_off < 0)
-    out[orow] = static_cast<OutT>(acc);
-  else  // split slab: the partial sums are added in work-item order by k_reduce
-    part[wi.part_off + lane] = acc;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int w = xcd_work_item(xs, blockIdx.x - ngather);
+  if (w < 0) return;
+  const bwl::WorkItem wi = wis[w];
+  const int R = wi.rows;
+  const int per = (wi.ngroups + W - 1) / W;
+  const int g0 = min(wave * per, wi.ngroups);
+  const int ng = min(per, wi.ngroups - g0);
+  const VT* __restrict__ base =
+      reinterpret_cast<const VT*>(data + wi.data_off + static_cast<int64_t>(g0) * R * V);
+  int64_t orow = 0;
+  if (wave == 0 && wi.part_off < 0 && lane < R) orow = rowmap[wi.out_row + lane];
+  const StagedInput<T, 64 * W> in{stage, g0, x, perm, dof, n_in, gidx[wi.gbeg], wi.ngroups * V};
+  T acc = 0;
+  // every wave passes ready() once, in uniform control flow (its barrier):
+  // lanes without a row of their own repeat a loaded one and are not stored
+  if (ng == 0) {
+    in.ready();
+  } else if (R > 32) {
+    acc = dot_tall<T, U>(base + min(lane, R - 1), R, ng, in);
+  } else {
+    const int nsplit = 64 / R;
+    const int split = min(lane / R, nsplit - 1);
+    acc = dot_short<T, 4>(base + min(lane - split * R, R - 1), R, nsplit, split, ng, in);
+    acc = fold_splits(acc, R, nsplit, lane / R, lane);
+  }
+  wave_sum_put<T, T, W>(acc, red, wi, wave, lane, orow, xt, part);
 }
 
 template <typename T, typename OutT>

@@ -69,6 +69,14 @@ def test_single_and_batched(gpu, shape, precision, wi_bytes):
                 y = dev.matvec(Xd[:, j].contiguous(), original=False, precision=precision,
                                adjoint=adjoint)
                 assert np.all(np.abs(y.cpu().numpy() - Y[:, j]) <= tol[:, j]), (j, u)
+        # the same product in the original numbering, moved by both permutations
+        p_in, p_out = (S.perm0, S.perm1) if adjoint else (S.perm1, S.perm0)
+        dofs = np.arange(S.dof)
+        x = np.empty(n_in)
+        x[(S.dof * p_in[:, None] + dofs).ravel()] = X[:, 31]
+        yo = dev.matvec(torch.from_numpy(x).to(gpu), original=True, precision=precision,
+                        adjoint=adjoint).cpu().numpy()
+        assert np.array_equal(yo[(S.dof * p_out[:, None] + dofs).ravel()], y.cpu().numpy())
 
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
