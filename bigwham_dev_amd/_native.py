@@ -116,6 +116,9 @@ def hip() -> C.CDLL:
         lib.bw_hip_set_unroll.argtypes = [_vp, C.c_int, C.c_int]
         lib.bw_hip_set_unroll_pass.argtypes = [_vp, C.c_int, C.c_int, C.c_int]
         lib.bw_hip_set_mfma_schedule.argtypes = [_vp, C.c_int, C.c_int]
+        lib.bw_hip_orthogonalize_work.argtypes = [C.c_int64, C.c_int, _i64]
+        lib.bw_hip_orthogonalize.argtypes = [C.c_int, C.c_int64, C.c_int, _vp, C.c_int64, _vp,
+                                             _vp, _vp, _vp, C.c_int64, _vp]
         lib.bw_hip_set_timing.argtypes = [_vp, C.c_int]
         lib.bw_hip_timing_stats.argtypes = [_vp, _d, _i64]
         lib.bw_hip_destroy.argtypes = [_vp]
@@ -196,7 +199,7 @@ HOST_SYMBOLS = ["bwh_create", "bwh_create_rect", "bwh_create_gaussian", "bwh_bui
 HIP_SYMBOLS = ["bw_hip_create", "bw_hip_matvec", "bw_hip_matvec_noalloc", "bw_hip_rmatvec", "bw_hip_matvec_batched",
                "bw_hip_rmatvec_batched", "bw_hip_matvec_batched_strided",
                "bw_hip_diagonal", "bw_hip_sizes", "bw_hip_set_tuning", "bw_hip_set_stacking", "bw_hip_set_unroll", "bw_hip_set_unroll_pass", "bw_hip_set_mfma_schedule",
-               "bw_hip_set_timing",
+               "bw_hip_orthogonalize_work", "bw_hip_orthogonalize", "bw_hip_set_timing",
                "bw_hip_timing_stats", "bw_hip_destroy", "bw_hip_last_error",
                "bw_layout_build", "bw_layout_info", "bw_layout_export", "bw_layout_free",
                "bw_layout_export_rowmap", "bw_layout_export_xcd",

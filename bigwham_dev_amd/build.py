@@ -24,7 +24,7 @@ HOST_SOURCES = sorted((CSRC / "host").glob("hb_*.cpp"))
 # libbwhip.so: the kernels and their C-ABI (hipcc), plus host-only C++ (the
 # slab layout, composition, full blocks, recompression) compiled by g++ with
 # the host ISA of libbwhost.so
-HIP_SOURCES = [CSRC / "hip" / "engine.hip"]
+HIP_SOURCES = [CSRC / "hip" / "engine.hip", CSRC / "hip" / "krylov.hip"]
 HIP_HOST_SOURCES = [CSRC / "hip" / "layout.cpp", CSRC / "hip" / "layout_capi.cpp",
                     CSRC / "hip" / "composite.cpp", CSRC / "hip" / "fullblocks.cpp",
                     CSRC / "hip" / "recompress.cpp"]

@@ -18,11 +18,14 @@ torch FP64 vectors:
 """
 from __future__ import annotations
 
+import ctypes as C
 import math
 import time
 from dataclasses import dataclass, field
 
 import torch
+
+from . import _native as N
 
 
 @dataclass
@@ -44,8 +47,8 @@ def gmres(matvec, b: torch.Tensor, precond=None, x0: torch.Tensor | None = None,
 
     Each iteration synchronises with the host once (the Hessenberg column and
     the new basis norm come back together); the basis vector itself is
-    normalised on the device, and on the GPU the next matvec is already queued
-    when the host waits.  A restart recomputes the residual b - A x with
+    normalised on the device, and on the GPU the next iteration is already
+    queued when the host waits.  A restart recomputes the residual b - A x with
     one matvec, or, with ``implicit_restart``, forms it from the Arnoldi
     relation r = V_{m+1} (beta e_1 - Hbar y) without a matvec (used by the
     inner solves of the mixed-precision refinement, whose outer loop
@@ -57,16 +60,100 @@ def gmres(matvec, b: torch.Tensor, precond=None, x0: torch.Tensor | None = None,
         return torch.zeros_like(b), 0, 0.0
     x = torch.zeros_like(b) if x0 is None else x0.clone()
     M = precond if precond is not None else (lambda v: v)
+    V = torch.empty((restart + 1, n), dtype=dt, device=dev)
+    # On the GPU the Hessenberg columns come back through pinned memory behind
+    # events, and the next iteration (matvec and orthogonalisation) is queued
+    # before the host waits for one, so the device is not left idle while the
+    # host applies the rotations.
+    steps = _DeviceSteps(V) if b.is_cuda else _HostSteps(V)
+    try:
+        return _cycles(matvec, M, b, x0, x, V, steps, bnorm, tol, restart, maxiter, callback,
+                       implicit_restart)
+    finally:
+        steps.close()
+
+
+class _HostSteps:
+    """Orthogonalisation steps with torch: classical Gram-Schmidt with one
+    re-orthogonalisation pass, as matrix-vector products."""
+
+    ahead = False  # steps are done when queued: nothing to look ahead for
+
+    def __init__(self, V):
+        self.V = V
+
+    def _torch_step(self, k, w):
+        Vk = self.V[: k + 1]
+        h = Vk @ w
+        w = torch.addmv(w, Vk.t(), h, alpha=-1.0)
+        h2 = Vk @ w
+        w = torch.addmv(w, Vk.t(), h2, alpha=-1.0)
+        hn = torch.linalg.vector_norm(w)
+        torch.div(w, hn, out=self.V[k + 1])
+        return torch.cat([h + h2, hn.reshape(1)])
+
+    def queue(self, k, w):
+        """Orthogonalise w against V[0..k] into V[k + 1]."""
+        self.col = self._torch_step(k, w)
+
+    def column(self, k):
+        """Hessenberg column k: k + 1 coefficients and the norm of the rest."""
+        return self.col.tolist()
+
+    def close(self):
+        pass
+
+
+class _DeviceSteps(_HostSteps):
+    """The same on the GPU, queued: four kernels per step
+    (bw_hip_orthogonalize) that write the column to pinned memory."""
+
+    ahead = True
+
+    def __init__(self, V):
+        super().__init__(V)
+        restart, n = V.shape[0] - 1, V.shape[1]
+        self.cols = torch.empty((restart, restart + 2), dtype=V.dtype, pin_memory=True)
+        self.events = [torch.cuda.Event() for _ in range(2)]
+        self.queued = -1
+        self.native = None
+        if V.dtype == torch.float64:
+            need = C.c_int64()
+            if N.hip().bw_hip_orthogonalize_work(n, restart, C.byref(need)) == N.BW_OK:
+                self.native = N.hip()
+                self.work = torch.empty(need.value, dtype=V.dtype, device=V.device)
+
+    def queue(self, k, w):
+        V = self.V
+        if (self.native and w.dtype == V.dtype and w.device == V.device and w.dim() == 1
+                and w.numel() == V.shape[1] and w.is_contiguous()):
+            rc = self.native.bw_hip_orthogonalize(
+                V.device.index, V.shape[1], k + 1, V.data_ptr(), V.stride(0), w.data_ptr(),
+                V[k + 1].data_ptr(), self.cols[k].data_ptr(), self.work.data_ptr(),
+                self.work.numel(), torch.cuda.current_stream(V.device).cuda_stream)
+            if rc != N.BW_OK:
+                raise N.BigWhamError(rc, "orthogonalize")
+        else:
+            self.cols[k, : k + 2].copy_(self._torch_step(k, w), non_blocking=True)
+        self.events[k & 1].record(torch.cuda.current_stream(V.device))
+        self.queued = k
+
+    def column(self, k):
+        self.events[k & 1].synchronize()
+        return self.cols[k, : k + 2].tolist()
+
+    def close(self):
+        # a queued step still writes the pinned columns
+        if self.queued >= 0:
+            self.events[self.queued & 1].synchronize()
+
+
+def _cycles(matvec, M, b, x0, x, V, steps, bnorm, tol, restart, maxiter, callback,
+            implicit_restart):
+    """The restart cycles of gmres()."""
+    dev, dt = b.device, b.dtype
     its = 0
     rel = 1.0
-    V = torch.empty((restart + 1, n), dtype=dt, device=dev)
-    # On the GPU the Hessenberg column comes back through pinned memory behind
-    # an event, and the next matvec is queued before the host waits for it, so
-    # the device is not left idle while the host applies the rotations.
-    pipelined = b.is_cuda
-    if pipelined:
-        col_host = torch.empty(restart + 2, dtype=dt, pin_memory=True)
-        ev = torch.cuda.Event()
     r = b.clone() if x0 is None else b - matvec(x)
     while its < maxiter:
         beta = torch.linalg.vector_norm(r).item()
@@ -81,34 +168,19 @@ def gmres(matvec, b: torch.Tensor, precond=None, x0: torch.Tensor | None = None,
         g[0] = beta
         k_done = 0
         breakdown = False
-        pending = None
+        queued = -1
         for k in range(restart):
-            if pending is not None:
-                w, pending = pending, None
-            else:
-                w = matvec(M(V[k]))
+            if queued < k:
+                steps.queue(k, matvec(M(V[k])))
+                queued = k
             its += 1
-            # CGS2: two classical Gram-Schmidt passes as matrix-vector products
-            Vk = V[: k + 1]
-            h = Vk @ w
-            w = torch.addmv(w, Vk.t(), h, alpha=-1.0)
-            h2 = Vk @ w
-            w = torch.addmv(w, Vk.t(), h2, alpha=-1.0)
-            hn_t = torch.linalg.vector_norm(w)
-            torch.div(w, hn_t, out=V[k + 1])
-            col_t = torch.cat([h + h2, hn_t.reshape(1)])
-            if pipelined:
-                col_host[: k + 2].copy_(col_t, non_blocking=True)
-                ev.record()
-                # look ahead unless the cycle ends here or the last estimate is
-                # already near the tolerance (a look-ahead past convergence is
-                # one wasted matvec)
-                if k + 1 < restart and its < maxiter and rel > 1.5 * tol:
-                    pending = matvec(M(V[k + 1]))
-                ev.synchronize()
-                col = col_host[: k + 2].tolist()
-            else:
-                col = col_t.tolist()
+            # look ahead unless the cycle ends here or the last estimate is
+            # already near the tolerance (a look-ahead past convergence is
+            # one wasted matvec)
+            if steps.ahead and k + 1 < restart and its < maxiter and rel > 1.5 * tol:
+                steps.queue(k + 1, matvec(M(V[k + 1])))
+                queued = k + 1
+            col = steps.column(k)
             hn = col[k + 1]
             for i in range(k + 2):
                 Hs[i][k] = Hraw[i][k] = col[i]

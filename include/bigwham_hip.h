@@ -253,6 +253,20 @@ int bw_hip_set_unroll_pass(bw_hip_handle* hd, int precision_mask, int pass, int 
  * fastest measured, which every value selects: the results do not depend on it. */
 int bw_hip_set_mfma_schedule(bw_hip_handle* hd, int precision_mask, int schedule);
 
+/* One orthogonalisation step of a Krylov basis on the device (for the GMRES of
+ * bigwham_dev_amd.solvers; no counterpart in the reference, whose users call
+ * scipy's): w is projected out of the k vectors V + j * ldv (j < k, n entries
+ * each) by classical Gram-Schmidt, twice; next = the normalised rest (n
+ * entries), col[0..k-1] = the coefficients, col[k] = the norm of the rest.  w is
+ * left as it is.  All pointers are device memory (col may be pinned host memory);
+ * `work` holds the doubles that bw_hip_orthogonalize_work gives for the largest k
+ * (BW_ESHAPE: k is at most 1024).  Asynchronous on `stream`; the calls that share `work` must be
+ * ordered. */
+int bw_hip_orthogonalize_work(int64_t n, int k, int64_t* elems);
+int bw_hip_orthogonalize(int device, int64_t n, int k, const double* V, int64_t ldv,
+                         const double* w, double* next, double* col, double* work,
+                         int64_t work_elems, void* stream);
+
 /* Per-kernel timing.  With timing enabled every matvec records HIP events
  * between its kernels on the call's stream; bw_hip_timing_stats returns the
  * average milliseconds over the calls since bw_hip_set_timing (which resets
