@@ -244,6 +244,7 @@ constexpr int64_t kItemBatched = 96 * 1024;
 // KiB (25 600-DoF mode-1 operator, 171 MB: 42.7 us at 1 / 512, 40.4 at 1 /
 // 1024, 38.8 at 1 / 1500, 41.3 at 1 / 2048 with 32 KiB).
 constexpr int64_t kPass1Share = 1500, kPass1MinBytes = 64 * 1024;
+constexpr int64_t kSortEntries = 200 << 20;
 // Pass 2 wants at least this many workgroups (of 256 compute units); operators
 // with fewer slabs that fit one work item each get slabs of fewer rows (4 000-
 // DoF 2DS0 operator, pass 2: 64 slabs of 62 rows 12.0 us, 256 of 16 rows 10.7).
@@ -313,9 +314,11 @@ void cut_items(const Program& P, const LayoutOptions& opt, int64_t wi_bytes, int
 
 // Places the slabs' data and column groups, and cuts both work-item lists.
 // Pass 1's items differ most in size (24 KiB to its bound) and run costliest
-// first (30 000-DoF 3DR0 operator: pass 1 97 us in slab order, 90 sorted);
-// pass 2's single-vector items are alike, and slab order, in which neighbours
-// share input entries, is 1 % faster on the 120 000-DoF one.  The batched
+// first (30 000-DoF 3DR0 operator: pass 1 97 us in slab order, 90 sorted), up to
+// kSortEntries: in slab order neighbours share input entries, which is worth
+// more on long passes (600 000-DoF 3DT0, FP64 3.45 ms against 3.56).  Pass 2's
+// single-vector items are alike, and slab order is 1 % faster on the 120 000-DoF
+// operator.  The batched
 // kernels run 6-8 % faster sorted (327 -> 306 us, FP32, 49 152 DoF).
 void finalize_program(Program* P, const LayoutOptions& opt, int64_t wi_single, bool sort_single) {
   const int V = opt.vec_elems;
@@ -438,7 +441,7 @@ void build_layout(const OpView& v, const LayoutOptions& opt, Layout* L) {
       }
       i = j;
     }
-    finalize_program(&P, opt, by_rows ? 4 * item : max_item, true);
+    finalize_program(&P, opt, by_rows ? 4 * item : max_item, entries <= kSortEntries);
   }
 
   // ---- pass 2: row intervals
