@@ -102,6 +102,7 @@ struct BatchOut {
   int nk;
   int yvec;
   T* part;
+  SplitSums sp;
   const int64_t* perm;
   int dof;
   const int32_t* rowmap;
@@ -135,6 +136,68 @@ __device__ __forceinline__ void batched_put(const BatchOut<T>& o, int64_t row, i
     if (c + k < o.nk) o.Y[row * o.yr + (c + k) * o.yc] = static_cast<double>(v[k]);
 }
 
+// 16 bytes of partial sums, as two 8-byte atomic accesses.
+template <typename T>
+__device__ __forceinline__ void part_put(T* p, typename Vec<T>::type v) {
+  typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
+  const u64x2 u = __builtin_bit_cast(u64x2, v);
+  part_store(reinterpret_cast<uint64_t*>(p), static_cast<uint64_t>(u.x));
+  part_store(reinterpret_cast<uint64_t*>(p) + 1, static_cast<uint64_t>(u.y));
+}
+
+template <typename T>
+__device__ __forceinline__ typename Vec<T>::type part_get(const T* p) {
+  typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
+  const uint64_t* q = reinterpret_cast<const uint64_t*>(p);
+  return __builtin_bit_cast(typename Vec<T>::type, u64x2{part_load(q), part_load(q + 1)});
+}
+
+// The end of a split slab's work item, by every thread of the workgroup after
+// its partial sums are stored: the last work item of the slab adds them, a
+// thread summing one 16-byte vector of right-hand sides of one row over the
+// parts, in part order, four parts in flight.
+template <int PASS, int NB, int W, typename T>
+__device__ __forceinline__ void sum_parts(const bwl::WorkItem& wi, const BatchOut<T>& o) {
+  typedef typename Vec<T>::type VT;
+  constexpr int V = Vec<T>::V;
+  constexpr int VPR = NB / V;
+  if (wi.part_off < 0 || !o.sp.count) return;
+  __shared__ int last;
+  const bwl::Reduce rd = o.sp.reds[wi.red];
+  stores_arrived();
+  __syncthreads();  // of every wave
+  if (threadIdx.x == 0) last = count_in(o.sp.count + wi.red, rd.nparts);
+  __syncthreads();
+  if (!last) return;
+  const T* __restrict__ base = o.part + static_cast<int64_t>(rd.part_off) * NB;
+  const int nvec = rd.rows * VPR;
+  for (int e = threadIdx.x; e < nvec; e += 64 * W) {
+    const int64_t row = batched_row<PASS>(o, rd.out_row + e / VPR);
+    const T* p = base + static_cast<int64_t>(e) * V;
+    const int64_t stride = static_cast<int64_t>(nvec) * V;
+    VT sum = {};
+    int q = 0;
+    for (; q + 4 <= rd.nparts; q += 4) {
+      const VT a = part_get(p + (q + 0) * stride);
+      const VT b = part_get(p + (q + 1) * stride);
+      const VT c = part_get(p + (q + 2) * stride);
+      const VT d = part_get(p + (q + 3) * stride);
+      sum += a;
+      sum += b;
+      sum += c;
+      sum += d;
+    }
+    VT v[3] = {};
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      if (q + k < rd.nparts) v[k] = part_get(p + (q + k) * stride);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) sum += v[k];
+    batched_put<PASS, NB>(o, row, (e % VPR) * V, sum);
+  }
+  if (threadIdx.x == 0) part_store(o.sp.count + wi.red, int32_t{0});
+}
+
 // Sums the W images lds[wave][32][NB] (rows r0 .. r0 + 31 of the work item,
 // written by the waves before the call) in wave order and stores the rows
 // below R.  Every thread of the workgroup calls it.
@@ -166,9 +229,11 @@ __device__ __forceinline__ void wave_sum_store(const T* lds, const bwl::WorkItem
     if (wi.part_off < 0) {
       batched_put<PASS, NB>(o, orow[e], c, s);
     } else {
-      // partial rows of a split slab, read once by k_reduce_b: nontemporal
       T* pp = o.part + (static_cast<int64_t>(wi.part_off) + row) * NB + c;
-      __builtin_nontemporal_store(s, reinterpret_cast<VT*>(pp));
+      if (o.sp.count)
+        part_put(pp, s);
+      else  // read once by k_reduce_b: nontemporal
+        __builtin_nontemporal_store(s, reinterpret_cast<VT*>(pp));
     }
   }
 }
@@ -342,6 +407,7 @@ k_slab_mfma32(const bwl::WorkItem* __restrict__ wis, XcdSplit xs,
     put(acc[1]);
     wave_sum_store<PASS, NB, W>(lds, wi, 32, o);
   }
+  sum_parts<PASS, NB, W>(wi, o);
 }
 
 // 16-row tiles: v_mfma_f64_16x16x4f64 and v_mfma_f32_16x16x4f32.  One k-step
@@ -507,6 +573,7 @@ k_slab_mfma16(const bwl::WorkItem* __restrict__ wis, XcdSplit xs,
     put(2);
     wave_sum_store<PASS, NB, W>(lds, wi, 32, o);
   }
+  sum_parts<PASS, NB, W>(wi, o);
 }
 
 // One workgroup per split slab; a thread sums one 16-byte vector of

@@ -6,10 +6,10 @@
 //   k_slab     pass 1: t = W x   (W_k = B_k), each row written through the
 //              row map into xt[xt_t : ...]
 //              (small operators: k_slab_gather does both)
-//   k_reduce   sum of split pass-1 work items (only if any)
 //   k_slab     pass 2: y = F x + U t, each y row written once, with the
 //              permutation of matvecOriginal (hmat.cc:618-626) fused in
-//   k_reduce   sum of split pass-2 work items (only if any)
+// Slabs that are split over several workgroups: the last of them adds the
+// partial sums, or in passes of many workgroups a k_reduce after the pass.
 // Every byte of the factor data is streamed once per matvec with 16-byte
 // non-temporal vector loads; x and t are re-read from L2 / MALL.  See
 // layout.h for the slab format.
@@ -71,6 +71,8 @@ constexpr int kBatchWaves = 4;
 
 // ---------------------------------------------------------------------------
 
+constexpr int kInKernelItems = 1024;
+
 // One work-item list of a pass on the device.
 struct DevItems {
   bwl::WorkItem* wis = nullptr;
@@ -79,6 +81,21 @@ struct DevItems {
   XcdSplit xs = {};
   int blocks = 0;               // workgroups of a launch
   int64_t part_elems = 0;
+
+  // bytes of the scratch for `cols` columns, and the counters within it
+  size_t part_bytes(int cols, int es) const { return (part_elems * cols * es + 15) / 16 * 16; }
+  size_t scratch_bytes(int cols, int es) const { return part_bytes(cols, es) + nred * sizeof(int32_t); }
+  // Whether the last work item of a split slab adds its partial sums, or a
+  // k_reduce launch.  The launch costs 4-5 us; in the kernel every split work
+  // item holds its place for a store and an atomic round trip more, which adds
+  // up where many follow each other on a compute unit.  Whole matvecs, launch
+  // against in-kernel: 369 items in pass 2 27.6 / 26.7 us, 562 38.6 / 37.5,
+  // 1 339 78.2 / 79.1, 3 279 158 / 169.
+  bool in_kernel() const { return nwi <= kInKernelItems; }
+  SplitSums sums(void* part, int cols, int es) const {
+    if (!in_kernel()) return {reds, nullptr};
+    return {reds, reinterpret_cast<int32_t*>(static_cast<unsigned char*>(part) + part_bytes(cols, es))};
+  }
 };
 
 struct DevPass {
@@ -108,7 +125,8 @@ struct DevOp {
 
 // What one matvec of an operator writes: xt (x gathered in the factor
 // precision, then t = B x), the partial sums of split work items of both
-// passes, and the same for the batched products (xt_size x xb_cols input and
+// passes with the counters of their split slabs behind them (zero between
+// launches), and the same for the batched products (xt_size x xb_cols input and
 // rank rows, partial sums x xb_cols).  xt is zero where no kernel writes (the
 // gap after x and the tail after t, which padded column groups read); the
 // batched gather writes those rows of xb itself.
@@ -431,6 +449,12 @@ hipError_t zero_now(void* p, size_t bytes) {
   return e;
 }
 
+// Zeroes the split-slab counters of fresh scratch.
+hipError_t zero_counters(const DevItems& di, void* part, int cols, int es) {
+  if (di.nred == 0 || !di.in_kernel()) return hipSuccess;
+  return zero_now(di.sums(part, cols, es).count, di.nred * sizeof(int32_t));
+}
+
 // Allocates what `ctx` lacks for operator [adj][fp32]: the single-vector
 // scratch, and with `batched` the batched one.  xt is zeroed here, once
 // (synchronously, before any kernel of the context can use it): the kernels
@@ -450,10 +474,12 @@ int ensure_op_scratch(bw_hip_handle* hd, StreamCtx* ctx, int adj, int fp32, bool
     const size_t pages = (op.xt_size * es + (size_t(2) << 20) - 1) >> 21;
     if ((rc = dev_alloc(&xt, pages << 21, &ctx->allocs, "scratch"))) return undo_allocs(ctx, mark, rc);
     for (int p = 0; p < 2; ++p)
-      if ((rc = dev_alloc(&part[p], (p ? op.p2 : op.p1).single.part_elems * es, &ctx->allocs,
+      if ((rc = dev_alloc(&part[p], (p ? op.p2 : op.p1).single.scratch_bytes(1, es), &ctx->allocs,
                           "scratch")))
         return undo_allocs(ctx, mark, rc);
-    const hipError_t e = zero_now(xt, op.xt_size * es);
+    hipError_t e = zero_now(xt, op.xt_size * es);
+    for (int p = 0; p < 2 && e == hipSuccess; ++p)
+      e = zero_counters((p ? op.p2 : op.p1).single, part[p], 1, es);
     if (e != hipSuccess)
       return undo_allocs(ctx, mark, fail(BW_EHIP, std::string("scratch: zero fill: ") + hipGetErrorString(e)));
     s.xt = xt;
@@ -470,13 +496,17 @@ int ensure_op_scratch(bw_hip_handle* hd, StreamCtx* ctx, int adj, int fp32, bool
       void* partb[2] = {nullptr, nullptr};
       rc = dev_alloc(&xb, static_cast<size_t>(op.xt_size) * cols * es, &ctx->allocs, "scratch");
       for (int p = 0; p < 2 && !rc; ++p)
-        rc = dev_alloc(&partb[p],
-                       static_cast<size_t>((p ? op.p2 : op.p1).batched.part_elems) * cols * es,
-                       &ctx->allocs, "scratch");
+        rc = dev_alloc(&partb[p], (p ? op.p2 : op.p1).batched.scratch_bytes(cols, es), &ctx->allocs,
+                       "scratch");
       if (rc) {
         undo_allocs(ctx, mark_b, rc);
         if (cols > 32) continue;
         return rc;
+      }
+      for (int p = 0; p < 2; ++p) {
+        const hipError_t e = zero_counters((p ? op.p2 : op.p1).batched, partb[p], cols, es);
+        if (e != hipSuccess)
+          return undo_allocs(ctx, mark, fail(BW_EHIP, std::string("scratch: zero fill: ") + hipGetErrorString(e)));
       }
       s.xb = xb;
       s.partb[0] = partb[0];
@@ -558,7 +588,8 @@ void launch_slab(const DevPass& dp, int unroll, hipStream_t st, const T* xin, Ou
   const DevItems& di = dp.single;
 #define BW_SLAB(U)                                                                              \
   hipLaunchKernelGGL((k_slab<T, OutT, U, PASS, W>), dim3(di.blocks), dim3(64 * W), 0, st, di.wis, \
-                     di.xs, dp.gidx, static_cast<const T*>(dp.data), xin, out, part, perm, dof,  \
+                     di.xs, dp.gidx, static_cast<const T*>(dp.data), xin, out, part,               \
+                     di.sums(part, 1, sizeof(T)), perm, dof,                                        \
                      dp.rowmap)
   if (unroll == 4)
     BW_SLAB(4);
@@ -580,7 +611,8 @@ void launch_slab_gather(const DevPass& dp, int unroll, hipStream_t st, const dou
 #define BW_SLAB(U)                                                                             \
   hipLaunchKernelGGL((k_slab_gather<T, U, W>), dim3(ngather + di.blocks), dim3(64 * W), lds, st, \
                      di.wis, di.xs, dp.gidx, static_cast<const T*>(dp.data), x, xt,             \
-                     static_cast<int>(n_in), perm, dof, ngather, dp.gather_cols, part, dp.rowmap)
+                     static_cast<int>(n_in), perm, dof, ngather, dp.gather_cols, part,          \
+                     di.sums(part, 1, sizeof(T)), dp.rowmap)
   if (unroll == 4)
     BW_SLAB(4);
   else
@@ -588,21 +620,33 @@ void launch_slab_gather(const DevPass& dp, int unroll, hipStream_t st, const dou
 #undef BW_SLAB
 }
 
-// Zero fill of xt's gap after x and its tail after t, for scratch that other
-// operators may have used before (the no-allocation entry point).
+// Zero fill of xt's gap after x and its tail after t and of both passes'
+// counters, for scratch that other operators may have used before (the
+// no-allocation entry point).
 template <typename T>
 __global__ __launch_bounds__(256) void k_zero_ranges(T* __restrict__ xt, int64_t a0, int64_t a1,
-                                                     int64_t b0, int64_t b1) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int64_t na = a1 - a0;
-  if (i < na)
+                                                     int64_t b0, int64_t b1,
+                                                     int32_t* __restrict__ c1, int n1,
+                                                     int32_t* __restrict__ c2, int n2) {
+  int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i < a1 - a0) {
     xt[a0 + i] = T(0);
-  else if (i - na < b1 - b0)
-    xt[b0 + (i - na)] = T(0);
+    return;
+  }
+  i -= a1 - a0;
+  if (i < b1 - b0) {
+    xt[b0 + i] = T(0);
+    return;
+  }
+  i -= b1 - b0;
+  if (i < n1)
+    c1[i] = 0;
+  else if (i - n1 < n2)
+    c2[i - n1] = 0;
 }
 
-// The five (selection: six) kernels of one matvec on stream st, writing only
-// the scratch `s` (and y_full for a selection).
+// The two to five (selection: four to six) kernels of one matvec on stream st,
+// writing only the scratch `s` (and y_full for a selection).
 template <typename T>
 int launch_matvec(bw_hip_handle* hd, DevOp& op, const OpScratch& s, double* y_full,
                   const double* xd, double* yd, int ordering, hipStream_t st,
@@ -637,7 +681,7 @@ int launch_matvec(bw_hip_handle* hd, DevOp& op, const OpScratch& s, double* y_fu
     launch_slab<T, T, 1>(op.p1, op.unroll[0], st, xt, xt, part1, nullptr, dof);
   }
   if (timing) (void)hipEventRecord(hd->ev[2], st);
-  if (op.p1.single.nred > 0)
+  if (op.p1.single.nred > 0 && !op.p1.single.in_kernel())
     hipLaunchKernelGGL((k_reduce<T, T>), dim3(op.p1.single.nred), dim3(64), 0, st,
                        op.p1.single.reds, op.p1.single.nred, part1, xt, nullptr, dof, op.p1.rowmap);
   if (timing) (void)hipEventRecord(hd->ev[3], st);
@@ -646,7 +690,7 @@ int launch_matvec(bw_hip_handle* hd, DevOp& op, const OpScratch& s, double* y_fu
                               dof);
   }
   if (timing) (void)hipEventRecord(hd->ev[4], st);
-  if (op.p2.single.nred > 0)
+  if (op.p2.single.nred > 0 && !op.p2.single.in_kernel())
     hipLaunchKernelGGL((k_reduce<T, double>), dim3(op.p2.single.nred), dim3(64), 0, st,
                        op.p2.single.reds, op.p2.single.nred, part2, yd, orig ? op.perm_out : nullptr, dof, nullptr);
   if (sd && sd->n_out > 0) {
@@ -773,8 +817,8 @@ int noalloc_matvec(bw_hip_handle* hd, const double* x, double* y, int ordering, 
   // xt, then the partial sums of pass 1 and pass 2, each 256-byte aligned
   const auto up = [](int64_t b) { return (b + 255) / 256 * 256; };
   const int64_t off1 = up(op.xt_size * op.elem);
-  const int64_t off2 = off1 + up(op.p1.single.part_elems * op.elem);
-  const int64_t need = off2 + up(op.p2.single.part_elems * op.elem);
+  const int64_t off2 = off1 + up(op.p1.single.scratch_bytes(1, op.elem));
+  const int64_t need = off2 + up(op.p2.single.scratch_bytes(1, op.elem));
   int64_t limit = BW_NOALLOC_SCRATCH_BYTES;
   if (const char* e = std::getenv("BWHIP_NOALLOC_LIMIT")) {
     const long long v = std::atoll(e);
@@ -805,19 +849,23 @@ int noalloc_matvec(bw_hip_handle* hd, const double* x, double* y, int ordering, 
   // Padded column groups read xt past x (the gap) and past t (the tail), so
   // those must hold zeros; an earlier call on this GPU may have left other
   // values there.  x and t are rewritten by every call, and every partial
-  // sum is written before it is read.  A fill kernel, not hipMemsetAsync,
+  // sum is written before it is read; the split slabs' counters start at zero.
+  // A fill kernel, not hipMemsetAsync,
   // so the call can be captured into a graph.
   const int64_t na = op.xt_t - op.n_in, nb = op.xt_size - (op.xt_t + op.t_total);
-  const int zblocks = static_cast<int>((na + nb + 255) / 256);
+  const DevItems &d1 = op.p1.single, &d2 = op.p2.single;
+  int32_t* const c1 = d1.sums(s.part[0], 1, op.elem).count;
+  int32_t* const c2 = d2.sums(s.part[1], 1, op.elem).count;
+  const int zblocks = static_cast<int>((na + nb + d1.nred + d2.nred + 255) / 256);
   if (zblocks > 0) {
     if (f32)
       hipLaunchKernelGGL(k_zero_ranges<float>, dim3(zblocks), dim3(256), 0, st,
                          static_cast<float*>(s.xt), op.n_in, op.xt_t, op.xt_t + op.t_total,
-                         op.xt_size);
+                         op.xt_size, c1, d1.nred, c2, d2.nred);
     else
       hipLaunchKernelGGL(k_zero_ranges<double>, dim3(zblocks), dim3(256), 0, st,
                          static_cast<double*>(s.xt), op.n_in, op.xt_t, op.xt_t + op.t_total,
-                         op.xt_size);
+                         op.xt_size, c1, d1.nred, c2, d2.nred);
   }
   return f32 ? launch_matvec<float>(hd, op, s, nullptr, x, y, ordering, st, nullptr, false)
              : launch_matvec<double>(hd, op, s, nullptr, x, y, ordering, st, nullptr, false);
@@ -1206,7 +1254,8 @@ int check_batched(bw_hip_handle* hd, bool adjoint, int nrhs, const double* X, in
   return BW_OK;
 }
 
-// The MFMA kernel and the reduction of one pass of a round of NB columns.
+// The MFMA kernel of one pass of a round of NB columns, and the reduction of
+// its split slabs if that is a launch of its own.
 template <int PASS, int NB, typename T>
 void launch_batched_pass(const DevPass& dp, hipStream_t st, const T* xb, const BatchOut<T>& o) {
   const DevItems& di = dp.batched;
@@ -1220,7 +1269,7 @@ void launch_batched_pass(const DevPass& dp, hipStream_t st, const T* xb, const B
       hipLaunchKernelGGL((k_slab_mfma16<T, PASS, NB / 16, kBatchWaves>), grid, block, 0, st, di.wis,
                          di.xs, dp.gidx, data, xb, o);
   }
-  if (di.nred > 0)
+  if (di.nred > 0 && !di.in_kernel())
     hipLaunchKernelGGL((k_reduce_b<PASS, NB, T>), dim3(di.nred), dim3(256), 0, st, di.reds,
                        di.nred, o);
 }
@@ -1249,6 +1298,7 @@ int launch_round(bw_hip_handle* hd, const DevOp& op, const OpScratch& s, int nk,
   o1.tout = xb;
   o1.nk = NB;
   o1.part = static_cast<T*>(s.partb[0]);
+  o1.sp = op.p1.batched.sums(s.partb[0], s.xb_cols, sizeof(T));
   o1.dof = dof;
   o1.rowmap = op.p1.rowmap;
   BatchOut<T> o2{};
@@ -1258,6 +1308,7 @@ int launch_round(bw_hip_handle* hd, const DevOp& op, const OpScratch& s, int nk,
   o2.nk = nk;
   o2.yvec = yc == 1 && yr % 2 == 0 && reinterpret_cast<uintptr_t>(Y) % 16 == 0;
   o2.part = static_cast<T*>(s.partb[1]);
+  o2.sp = op.p2.batched.sums(s.partb[1], s.xb_cols, sizeof(T));
   o2.perm = orig ? op.perm_out : nullptr;
   o2.dof = dof;
   launch_batched_pass<1, NB>(op.p1, st, xb, o1);

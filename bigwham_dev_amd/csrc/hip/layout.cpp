@@ -237,16 +237,23 @@ constexpr int64_t kItemShare = 4096;  // between the two: 1 / 4096 of the pass
 // - the batched kernels (4-wave workgroups) pay for every split with NB-wide
 //   partial rows: 32 right-hand sides on the 49 152-DoF 3DR0 operator take 306
 //   us at 384 KiB (FP32), 314 at 256, 311 at 768 KiB.
-constexpr int64_t kItemBatched = 96 * 1024;
+//   Passes of fewer slabs than kMinSlabs leave compute units idle at that size
+//   and are cut to about 384 items (1 728 DoF, FP64, 32 slabs of 90 K entries:
+//   38.6 -> 27.5 us, FP32 31 -> 22.4; 6 912 DoF, 128 slabs: 84 -> 77; 1 / 512 of
+//   the pass 81, 1 / 1024 81); from 253 slabs on the cut costs more than it
+//   balances (16 cracks, FP32: 41.5 us whole, 42.8 cut).
+constexpr int64_t kItemBatched = 96 * 1024, kItemBatchedMin = 16 * 1024, kBatchedItems = 384;
 // Pass 1 of a small operator is cut by rows instead: a slab over a wide column
 // cluster gets fewer rows (at least 16), so that it is one work item and the
-// pass needs no reduction.  Its item size is 1 / 1500 of the pass, at least 64
+// pass needs no reduction.  Its item size is 1 / 1500 of the pass, at least 48
 // KiB (25 600-DoF mode-1 operator, 171 MB: 42.7 us at 1 / 512, 40.4 at 1 /
-// 1024, 38.8 at 1 / 1500, 41.3 at 1 / 2048 with 32 KiB).
-constexpr int64_t kPass1Share = 1500, kPass1MinBytes = 64 * 1024;
+// 1024, 38.8 at 1 / 1500, 41.3 at 1 / 2048; 16 000-DoF 2DS0 operator, whole
+// matvec: 26.6 us at 64 KiB, 22.8 at 48; 6 400-DoF mode-1 19.5 at 64 and 48,
+// 20.5 at 32).
+constexpr int64_t kPass1Share = 1500, kPass1MinBytes = 48 * 1024;
 constexpr int64_t kSortEntries = 200 << 20;
-// Pass 2 wants at least this many workgroups (of 256 compute units); operators
-// with fewer slabs that fit one work item each get slabs of fewer rows (4 000-
+// A pass wants at least this many workgroups (of 256 compute units); in pass 2,
+// operators with fewer slabs that fit one work item each get slabs of fewer rows (4 000-
 // DoF 2DS0 operator, pass 2: 64 slabs of 62 rows 12.0 us, 256 of 16 rows 10.7).
 constexpr int64_t kMinSlabs = 192;
 constexpr int kMinRows = 16;
@@ -276,7 +283,7 @@ void cut_items(const Program& P, const LayoutOptions& opt, int64_t wi_bytes, int
       wi.rows = sd.rows;
       wi.out_row = static_cast<int32_t>(sd.out_row0);
       wi.part_off = nwi == 1 ? -1 : static_cast<int32_t>(part + w * sd.rows);
-      wi.pad = 0;
+      wi.red = static_cast<int32_t>(il->reds.size());
       il->wis.push_back(wi);
     }
     if (nwi > 1) {
@@ -337,7 +344,11 @@ void finalize_program(Program* P, const LayoutOptions& opt, int64_t wi_single, b
   P->data_elems = data;
   const bool tuned = opt.wi_bytes > 0;
   cut_items(*P, opt, tuned ? opt.wi_bytes : wi_single, 1, sort_single, &P->single);
-  cut_items(*P, opt, tuned ? opt.wi_bytes : kItemBatched * opt.elem_bytes,
+  const int64_t batched =
+      static_cast<int64_t>(P->slabs.size()) >= kMinSlabs
+          ? kItemBatched
+          : std::min(kItemBatched, std::max(kItemBatchedMin, data / kBatchedItems));
+  cut_items(*P, opt, tuned ? opt.wi_bytes : batched * opt.elem_bytes,
             opt.elem_bytes == 8 ? 16 : 32, true, &P->batched);
 }
 

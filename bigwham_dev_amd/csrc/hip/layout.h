@@ -50,15 +50,12 @@ struct WorkItem {
   int32_t rows;      // R
   int32_t out_row;   // output row of the WI's row 0 (pass 1: index into rowmap)
   int32_t part_off;  // -1: direct write, else offset into the partial buffer
-  int32_t pad;
+  int32_t red;       // split slab: its Reduce
 };
 
-// Reduce descriptor for a slab split over several WIs (16 bytes): a separate
-// pass after the slab pass adds the partial sums in WI order; the waves of one
-// workgroup add theirs in LDS.  (Reducing
-// inside the slab kernel, by its last WI, needs agent-scope release/acquire
-// fences, which on MI355X write back and invalidate the per-XCD L2 and cost
-// more than the separate launch.)
+// A slab split over several work items (16 bytes): their partial sums are added
+// in work-item order, by the last of them to finish or by a pass of its own;
+// the waves of one workgroup add theirs in LDS.
 struct Reduce {
   int32_t out_row;
   int32_t rows;

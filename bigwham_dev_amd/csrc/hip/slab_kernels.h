@@ -295,22 +295,92 @@ __device__ __forceinline__ T fold_splits(T acc, int R, int nsplit, int split, in
   return acc;
 }
 
+// Split slabs of passes of few work items (the others: k_reduce).  Each work
+// item of one stores its partial sums, waits until they have arrived, and counts itself in; the one that finds all others
+// counted adds the partial sums in work-item order, stores the rows and sets
+// the counter back to zero for the next launch.  The work items of a slab can
+// run on different XCDs, whose L2s are not coherent: partial sums and counters
+// are only ever touched by agent-scope atomic accesses, which go past the L2.
+// They are relaxed: a release or acquire at agent scope would write back and
+// invalidate a whole L2, and the wait below is the order that is needed (a
+// store that has been acknowledged is visible to every later agent-scope load).
+// No work item waits for another.
+struct SplitSums {
+  const bwl::Reduce* reds;
+  int32_t* count;  // one per split slab, zero between launches; nullptr: k_reduce adds them
+};
+
+template <typename P>
+__device__ __forceinline__ void part_store(P* p, P v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+template <typename P>
+__device__ __forceinline__ P part_load(const P* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Waits until this wave's stores have been acknowledged.
+__device__ __forceinline__ void stores_arrived() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// Counts a work item in (one lane); true for the last of nparts.
+__device__ __forceinline__ bool count_in(int32_t* count, int nparts) {
+  return __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nparts - 1;
+}
+
 // The waves' sums of a work item added in wave order from LDS, and its rows
 // stored by the first wave (`orow`: the lane's output row, requested before
 // the stream).
 template <typename T, typename OutT, int W>
 __device__ __forceinline__ void wave_sum_put(T acc, T (*red)[64], const bwl::WorkItem& wi,
-                                             int wave, int lane, int64_t orow, OutT* out, T* part) {
+                                             int wave, int lane, int64_t orow, OutT* out, T* part,
+                                             const SplitSums& sp) {
   const int R = wi.rows;
   if (wave > 0 && lane < R) red[wave][lane] = acc;
   __syncthreads();
   if (wave > 0 || lane >= R) return;
 #pragma unroll
   for (int k = 1; k < W; ++k) acc += red[k][lane];
-  if (wi.part_off < 0)
-    out[orow] = static_cast<OutT>(acc);
-  else  // split slab: the partial sums are added in work-item order by k_reduce
-    part[wi.part_off + lane] = acc;
+  if (wi.part_off >= 0) {
+    if (!sp.count) {  // added by k_reduce
+      part[wi.part_off + lane] = acc;
+      return;
+    }
+    const bwl::Reduce rd = sp.reds[wi.red];
+    part_store(part + wi.part_off + lane, acc);
+    stores_arrived();
+    int last = 0;
+    if (lane == 0) last = count_in(sp.count + wi.red, rd.nparts);
+    if (!__builtin_amdgcn_readfirstlane(last)) return;
+    // four interleaved sums over the parts, eight loads in flight; the order
+    // of the additions is fixed, so the result is deterministic
+    const T* p = part + rd.part_off + lane;
+    T s[4] = {0, 0, 0, 0};
+    int q = 0;
+    for (; q + 8 <= rd.nparts; q += 8) {
+      T v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = part_load(p + (q + k) * R);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) s[k & 3] += v[k];
+    }
+    for (; q + 4 <= rd.nparts; q += 4) {
+      T v[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[k] = part_load(p + (q + k) * R);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) s[k] += v[k];
+    }
+    T v[3] = {0, 0, 0};
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      if (q + k < rd.nparts) v[k] = part_load(p + (q + k) * R);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) s[0] += v[k];
+    acc = (s[0] + s[1]) + (s[2] + s[3]);
+    if (lane == 0) part_store(sp.count + wi.red, int32_t{0});
+  }
+  out[orow] = static_cast<OutT>(acc);
 }
 
 // One workgroup of W waves per work item: the waves take equal contiguous
@@ -331,6 +401,7 @@ __global__ __launch_bounds__(64 * W) void k_slab(const bwl::WorkItem* __restrict
                                                  const T* __restrict__ data,
                                                  const T* __restrict__ xin,
                                                  OutT* __restrict__ out, T* __restrict__ part,
+                                                 SplitSums sp,
                                                  const int64_t* __restrict__ perm, int dof,
                                                  const int32_t* __restrict__ rowmap) {
   typedef typename Vec<T>::type VT;
@@ -350,7 +421,7 @@ __global__ __launch_bounds__(64 * W) void k_slab(const bwl::WorkItem* __restrict
       reinterpret_cast<const VT*>(data + wi.data_off + static_cast<int64_t>(g0) * R * V);
   const int32_t* __restrict__ gi = gidx + wi.gbeg + g0;
   int64_t orow = 0;
-  if (wave == 0 && wi.part_off < 0 && lane < R) {
+  if (wave == 0 && (wi.part_off < 0 || sp.count) && lane < R) {
     // pass 1 rows go to their t entries through the row map
     const int64_t r = rowmap ? rowmap[wi.out_row + lane] : static_cast<int64_t>(wi.out_row) + lane;
     orow = out_index<OutT>(r, perm, dof);
@@ -366,7 +437,7 @@ __global__ __launch_bounds__(64 * W) void k_slab(const bwl::WorkItem* __restrict
                             XtInput<T, false>{gi, xin});
     acc = fold_splits(acc, R, nsplit, split, lane);
   }
-  wave_sum_put<T, OutT, W>(acc, red, wi, wave, lane, orow, out, part);
+  wave_sum_put<T, OutT, W>(acc, red, wi, wave, lane, orow, out, part, sp);
 }
 
 // Pass 1 of small operators together with the gather of x: the first
@@ -380,6 +451,7 @@ __global__ __launch_bounds__(64 * W) void k_slab_gather(
     const bwl::WorkItem* __restrict__ wis, XcdSplit xs, const int32_t* __restrict__ gidx,
     const T* __restrict__ data, const double* __restrict__ x, T* __restrict__ xt, int n_in,
     const int64_t* __restrict__ perm, int dof, int ngather, int lds_cols, T* __restrict__ part,
+    SplitSums sp,
     const int32_t* __restrict__ rowmap) {
   typedef typename Vec<T>::type VT;
   constexpr int V = Vec<T>::V;
@@ -403,7 +475,7 @@ __global__ __launch_bounds__(64 * W) void k_slab_gather(
   const VT* __restrict__ base =
       reinterpret_cast<const VT*>(data + wi.data_off + static_cast<int64_t>(g0) * R * V);
   int64_t orow = 0;
-  if (wave == 0 && wi.part_off < 0 && lane < R) orow = rowmap[wi.out_row + lane];
+  if (wave == 0 && (wi.part_off < 0 || sp.count) && lane < R) orow = rowmap[wi.out_row + lane];
   const StagedInput<T, 64 * W> in{stage, g0, x, perm, dof, n_in, gidx[wi.gbeg], wi.ngroups * V};
   T acc = 0;
   // every wave passes ready() once, in uniform control flow (its barrier):
@@ -418,7 +490,7 @@ __global__ __launch_bounds__(64 * W) void k_slab_gather(
     acc = dot_short<T, 4>(base + min(lane - split * R, R - 1), R, nsplit, split, ng, in);
     acc = fold_splits(acc, R, nsplit, lane / R, lane);
   }
-  wave_sum_put<T, T, W>(acc, red, wi, wave, lane, orow, xt, part);
+  wave_sum_put<T, T, W>(acc, red, wi, wave, lane, orow, xt, part, sp);
 }
 
 template <typename T, typename OutT>

@@ -100,3 +100,41 @@ def test_round_widths(gpu, shape, precision):
         out = torch.full((k, dev.n_rows), np.nan, dtype=torch.float64, device=gpu).t()
         dev.matvec_batched(Xc, original=False, precision=precision, out=out)
         assert torch.equal(out, got), k
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("wi_bytes", [512, 4096])
+def test_split_slabs(gpu, precision, wi_bytes):
+    """Slabs split over several work items, in passes of few (the last item of
+    a slab adds the partial sums) and of many work items (a reduction launch
+    does): against the blocks, and the same bits on every launch, whatever
+    order the items finish in: eager, on two streams at once and in a graph."""
+    import torch
+    S = SyntheticHmat(400, 380, 2, 7)
+    set_tuning(wi_bytes, wi_bytes)
+    try:
+        dev = HipHmat(S, precisions=(precision,))
+    finally:
+        set_tuning(0, 0)
+    X = np.random.default_rng(8).uniform(-1, 1, (dev.n_cols, 40))
+    Y, bound = _reference(S, X, False)
+    tol = 2 * (dev.n_cols + int(S.lr_pattern[:, 5].sum()) + 8) * U[precision] * bound
+    Xd = torch.from_numpy(X).to(gpu)
+    x = Xd[:, 0].contiguous()
+    y = dev.matvec(x, original=False, precision=precision)
+    Yd = dev.matvec_batched(Xd, original=False, precision=precision)
+    assert np.all(np.abs(y.cpu().numpy() - Y[:, 0]) <= tol[:, 0])
+    assert np.all(np.abs(Yd.cpu().numpy() - Y) <= tol)
+    g = dev.graph(x, original=False, precision=precision)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    outs = []
+    for rep in range(20):
+        for s in streams:
+            with torch.cuda.stream(s):
+                outs.append((dev.matvec(x, original=False, precision=precision), y))
+                outs.append((dev.matvec_batched(Xd, original=False, precision=precision), Yd))
+        outs.append((g.launch().clone(), y))
+    torch.cuda.synchronize()
+    for a, b in outs:
+        assert torch.equal(a, b)
