@@ -147,6 +147,8 @@ struct StreamCtx {
   OpScratch op[2][2];  // [adjoint][fp32]
   double* x_stage = nullptr;
   double* y_stage = nullptr;
+  double* x_pin = nullptr;  // pinned, read and written by the kernels
+  double* y_pin = nullptr;
   double* y_full = nullptr;
   std::vector<void*> allocs;
 };
@@ -245,7 +247,10 @@ int upload_pass(const bwl::Layout& L, const bwl::Program& P, DevPass* dp, hipStr
   if (nslab == 0) return BW_OK;
   int64_t max_slab = 0;
   for (const auto& s : P.slabs) max_slab = std::max<int64_t>(max_slab, s.ngroups * s.rows * L.opt.vec_elems);
-  const int64_t chunk_elems = std::max<int64_t>(max_slab, (int64_t(256) << 20) / static_cast<int64_t>(sizeof(T)));
+  // no larger than the pass: pinning 2 x 256 MiB takes 5 ms, most of the upload
+  // of a small operator
+  const int64_t chunk_elems = std::max<int64_t>(
+      max_slab, std::min<int64_t>(P.data_elems, (int64_t(256) << 20) / static_cast<int64_t>(sizeof(T))));
   T* stage[2] = {nullptr, nullptr};
   if ((rc = host_pinned_alloc(reinterpret_cast<void**>(&stage[0]), chunk_elems * sizeof(T),
                               "create: upload staging")))
@@ -518,15 +523,38 @@ int ensure_op_scratch(bw_hip_handle* hd, StreamCtx* ctx, int adj, int fp32, bool
   return BW_OK;
 }
 
+// Vectors of host-pointer calls.  Up to kPinnedEntries they pass through
+// pinned memory that the kernels themselves read and write: copies from and
+// to pageable memory cost 15-20 us of a small call (two such copies and two
+// small kernels, 800 entries: 30.8 us; through pinned memory 14.9; 16 000: 36.0
+// and 22.9; 100 000: 86 and 74).  Results of at most kDirectEntries are stored
+// in pinned memory by pass 2, scattered by the permutation (800 entries: 14.9
+// us, 16.2 through device memory and a copy kernel; 4 000: 19.8 and 17.9).
+// Pass 1 gathers x from pinned memory up to kPinnedGather entries (host calls
+// of 800 entries: 22.7 us against 24.4 with a gather launch, 4 599: 42.9 / 49.6,
+// 8 000: 40.4 / 36.8).
+constexpr int64_t kPinnedEntries = 128 * 1024, kDirectEntries = 1024, kPinnedGather = 6 * 1024;
+
 // Staging vectors of host-pointer calls and a selection's full output.
 int ensure_ctx_vectors(bw_hip_handle* hd, StreamCtx* ctx, bool staging) {
   const size_t mark = ctx->allocs.size();
+  const size_t bytes = hd->stage_elems * sizeof(double);
+  const bool pinned = hd->stage_elems <= kPinnedEntries;
   int rc;
-  if (staging && !ctx->x_stage) {
+  if (staging && !ctx->y_stage) {
     void *xs = nullptr, *ys = nullptr;
-    if ((rc = dev_alloc(&xs, hd->stage_elems * sizeof(double), &ctx->allocs, "scratch")) ||
-        (rc = dev_alloc(&ys, hd->stage_elems * sizeof(double), &ctx->allocs, "scratch")))
+    if ((!pinned && (rc = dev_alloc(&xs, bytes, &ctx->allocs, "scratch"))) ||
+        (rc = dev_alloc(&ys, bytes, &ctx->allocs, "scratch")))
       return undo_allocs(ctx, mark, rc);
+    if (pinned) {
+      // one allocation, x then y
+      void* hp = nullptr;
+      const size_t xb = (bytes + 255) / 256 * 256;
+      if ((rc = host_pinned_alloc(&hp, xb + std::max<size_t>(bytes, 16), "scratch")))
+        return undo_allocs(ctx, mark, rc);
+      ctx->x_pin = static_cast<double*>(hp);
+      ctx->y_pin = reinterpret_cast<double*>(static_cast<unsigned char*>(hp) + xb);
+    }
     ctx->x_stage = static_cast<double*>(xs);
     ctx->y_stage = static_cast<double*>(ys);
   }
@@ -543,6 +571,8 @@ int ensure_ctx_vectors(bw_hip_handle* hd, StreamCtx* ctx, bool staging) {
 void free_ctx(StreamCtx* ctx) {
   for (void* p : ctx->allocs) (void)hipFree(p);
   ctx->allocs.clear();
+  if (ctx->x_pin) (void)hipHostFree(ctx->x_pin);
+  ctx->x_pin = ctx->y_pin = nullptr;
 }
 
 // The context of `stream` (created empty on its first use); caller holds hd->mu.
@@ -650,7 +680,7 @@ __global__ __launch_bounds__(256) void k_zero_ranges(T* __restrict__ xt, int64_t
 template <typename T>
 int launch_matvec(bw_hip_handle* hd, DevOp& op, const OpScratch& s, double* y_full,
                   const double* xd, double* yd, int ordering, hipStream_t st,
-                  const SelDir* sd = nullptr, bool timed = true) {
+                  const SelDir* sd = nullptr, bool timed = true, bool x_pinned = false) {
   const bool orig = !sd && ordering == BW_ORDER_ORIGINAL;
   const int dof = hd->dof;
   T* xt = static_cast<T*>(s.xt);
@@ -659,7 +689,8 @@ int launch_matvec(bw_hip_handle* hd, DevOp& op, const OpScratch& s, double* y_fu
   double* const y_user = yd;
   if (sd) yd = y_full;  // the passes write the full permuted y
   const bool timing = timed && hd->timing;
-  const bool fused = !sd && op.p1.gather_cols > 0;  // pass 1 gathers x
+  // pass 1 gathers x, unless that reads a long x many times from host memory
+  const bool fused = !sd && op.p1.gather_cols > 0 && (!x_pinned || op.n_in <= kPinnedGather);
   if (timing) (void)hipEventRecord(hd->ev[0], st);
   if (sd) {
     if (sd->n_pairs > 0) {
@@ -749,10 +780,18 @@ int do_matvec(bw_hip_handle* hd, bool adjoint, const double* x, double* y, int o
     return rc;
   const double* xd = x;
   double* yd = y;
+  const bool pinned = !on_device && ctx->x_pin;
+  // a selection stores its rows in order
+  const bool direct = pinned && (sd || n_out <= kDirectEntries);
   if (!on_device) {
-    HIPCHK(hipMemcpyAsync(ctx->x_stage, x, n_in * sizeof(double), hipMemcpyHostToDevice, st));
-    xd = ctx->x_stage;
-    yd = ctx->y_stage;
+    if (pinned) {
+      std::memcpy(ctx->x_pin, x, n_in * sizeof(double));
+      xd = ctx->x_pin;
+    } else {
+      HIPCHK(hipMemcpyAsync(ctx->x_stage, x, n_in * sizeof(double), hipMemcpyHostToDevice, st));
+      xd = ctx->x_stage;
+    }
+    yd = direct ? ctx->y_pin : ctx->y_stage;
   }
   if (hd->timing) {
     const int set = hd->cur;
@@ -763,14 +802,22 @@ int do_matvec(bw_hip_handle* hd, bool adjoint, const double* x, double* y, int o
     hd->ev = hd->evs[set];
   }
   const OpScratch& s = ctx->op[adj][f32];
-  rc = f32 ? launch_matvec<float>(hd, op, s, ctx->y_full, xd, yd, ordering, st, sd)
-           : launch_matvec<double>(hd, op, s, ctx->y_full, xd, yd, ordering, st, sd);
+  rc = f32 ? launch_matvec<float>(hd, op, s, ctx->y_full, xd, yd, ordering, st, sd, true, pinned)
+           : launch_matvec<double>(hd, op, s, ctx->y_full, xd, yd, ordering, st, sd, true, pinned);
   if (rc) return rc;
   if (hd->timing) {
     hd->pending[hd->cur] = true;
     hd->cur ^= 1;
   }
-  if (!on_device) {
+  if (pinned) {
+    if (!direct && n_out > 0) {
+      hipLaunchKernelGGL(k_copy, dim3(static_cast<unsigned>((n_out + 255) / 256)), dim3(256), 0, st,
+                         ctx->y_stage, ctx->y_pin, n_out);
+      HIPCHK(hipGetLastError());
+    }
+    HIPCHK(hipStreamSynchronize(st));
+    std::memcpy(y, ctx->y_pin, n_out * sizeof(double));
+  } else if (!on_device) {
     HIPCHK(hipMemcpyAsync(y, ctx->y_stage, n_out * sizeof(double), hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
   }

@@ -47,6 +47,13 @@ __global__ __launch_bounds__(256) void k_gather(const double* __restrict__ x,
   xt[i] = static_cast<T>(x[src]);
 }
 
+// Result of a host-pointer call to pinned memory, in order.
+__global__ __launch_bounds__(256) void k_copy(const double* __restrict__ src,
+                                              double* __restrict__ dst, int64_t n) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i < n) dst[i] = src[i];
+}
+
 template <typename OutT>
 __device__ __forceinline__ int64_t out_index(int64_t idx, const int64_t* perm, int dof) {
   if (!perm) return idx;

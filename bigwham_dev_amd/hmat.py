@@ -378,7 +378,7 @@ class HipHmat:
                     or not y.flags.c_contiguous):
                 raise ValueError(f"matvec: out must be a contiguous float64 array of {n_out}")
             fn = N.hip().bw_hip_rmatvec if adjoint else N.hip().bw_hip_matvec
-            N.check_hip(fn(self._h, x.ctypes.data_as(C.c_void_p), y.ctypes.data_as(C.c_void_p),
+            N.check_hip(fn(self._h, x.ctypes.data, y.ctypes.data,
                            N.BW_ORDER_ORIGINAL if original else N.BW_ORDER_PERMUTED,
                            self._prec(precision), 0, None))
             return y

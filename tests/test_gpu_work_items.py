@@ -138,3 +138,24 @@ def test_split_slabs(gpu, precision, wi_bytes):
     torch.cuda.synchronize()
     for a, b in outs:
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("shape", [(1024, 40, 1, 1), (1025, 40, 1, 2), (3, 131072, 1, 3),
+                                   (3, 131073, 1, 4), (350, 342, 3, 5),
+                                   (90, 2048, 3, 6), (90, 2049, 3, 7)])
+def test_host_vectors(gpu, shape, precision):
+    """Host vectors give the bits of device vectors, at the sizes where their
+    way changes (1 024 results, 6 144 and 131 072 entries), repeated with new inputs (the
+    staging is shared), in both orderings and directions."""
+    import torch
+    S = SyntheticHmat(*shape)
+    dev = HipHmat(S, precisions=(precision,), adjoint=True)
+    rng = np.random.default_rng(6)
+    for adjoint in (False, True, False):
+        for original in (True, False):
+            x = rng.uniform(-1, 1, dev.n_rows if adjoint else dev.n_cols)
+            y = dev.matvec(x, original=original, precision=precision, adjoint=adjoint)
+            yd = dev.matvec(torch.from_numpy(x).to(gpu), original=original, precision=precision,
+                            adjoint=adjoint)
+            assert np.array_equal(y, yd.cpu().numpy()), (adjoint, original)
