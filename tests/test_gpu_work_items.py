@@ -159,3 +159,48 @@ def test_host_vectors(gpu, shape, precision):
             yd = dev.matvec(torch.from_numpy(x).to(gpu), original=original, precision=precision,
                             adjoint=adjoint)
             assert np.array_equal(y, yd.cpu().numpy()), (adjoint, original)
+
+
+@pytest.mark.parametrize("cols", [20, 40])
+@pytest.mark.parametrize("a_scale, x_scale", [
+    (1.0, 1.0), (1.0, 1e-28), (1.0, 1e-33), (1.0, 1e30), (1e-22, 1e-12), (1e-22, 1e20)])
+def test_fp32_split_range(gpu, cols, a_scale, x_scale):
+    """The 32- and 64-wide FP32 rounds split their numbers into bf16 parts where
+    that is exact: operators and inputs of sizes within, at the end of and
+    outside that range, and columns of other sizes beside them.  Products
+    below 2^-126 may be lost (the last term)."""
+    import torch
+    S = SyntheticHmat(130, 150, 2, 9)
+    for blocks in (S.fr, S.A):
+        for b in blocks:
+            b *= a_scale
+    dev = HipHmat(S, precisions=("fp32",))
+    X = np.random.default_rng(10).uniform(-1, 1, (dev.n_cols, cols)) * x_scale
+    X[:, 3] /= x_scale   # columns of ordinary size, of one tiny entry, of zeros
+    X[5:, 4] = 0.0
+    X[4, 4] = 3e-38
+    X[:, 5] = 0.0
+    Y, bound = _reference(S, X, False)
+    n = dev.n_cols + int(S.lr_pattern[:, 5].sum()) + 8
+    got = dev.matvec_batched(torch.from_numpy(X).to(gpu), original=False, precision="fp32")
+    big = max(1.0, max(np.abs(b).sum(axis=1).max(initial=0.0) for b in S.fr + S.A))
+    assert np.all(np.abs(got.cpu().numpy() - Y) <= 2 * n * U["fp32"] * bound + n * big * 2.0 ** -126)
+
+
+@pytest.mark.parametrize("cols", [20, 40])
+def test_fp32_not_finite(gpu, cols):
+    """Infinities and NaN in the input of a wide FP32 round reach the entries
+    that they reach in the single-vector product, and no other column."""
+    import torch
+    S = SyntheticHmat(130, 150, 2, 9)
+    dev = HipHmat(S, precisions=("fp32",))
+    X = np.random.default_rng(11).uniform(-1, 1, (dev.n_cols, cols))
+    X[7, 2], X[90, 3], X[200, 4] = np.inf, -np.inf, np.nan
+    Xd = torch.from_numpy(X).to(gpu)
+    got = dev.matvec_batched(Xd, original=False, precision="fp32").cpu().numpy()
+    for j in range(cols):
+        y = dev.matvec(Xd[:, j].contiguous(), original=False, precision="fp32").cpu().numpy()
+        assert np.array_equal(np.isnan(got[:, j]), np.isnan(y)), j
+        assert np.array_equal(np.isposinf(got[:, j]), np.isposinf(y)), j
+        assert np.array_equal(np.isneginf(got[:, j]), np.isneginf(y)), j
+        assert j in (2, 3, 4) or np.all(np.isfinite(y))
