@@ -7,8 +7,8 @@
 // in rounds of NB, columns past nk are zero and never stored.  Rounds of 16
 // columns move half the input rows and partial sums of 32 (24 300 DoF, 32 and
 // 16 columns: FP64 275 and 237 us, FP32 156 and 135); in FP32 a round of 64
-// streams the factors once for twice the columns (312 -> 203, 49 152 DoF 580 ->
-// 391), and wins from 33 columns on (290 + 261 -> 391).  FP64 stays at 32: its
+// streams the factors once for twice the columns (312 -> 186, 49 152 DoF 580 ->
+// 367), and wins from 33 columns on (290 + 261 -> 367).  FP64 stays at 32: its
 // time goes with the columns (158 us for one vector).
 //
 // What bounds them: reads from L2 (63-69 G requests a second here and in the
@@ -242,6 +242,39 @@ __device__ __forceinline__ void wave_sum_store(const T* lds, const bwl::WorkItem
   }
 }
 
+// Where a lane's two rows of a 32-row-tile item lie: byte offsets of column group
+// g + half (at most the last), and the same as index of 16-byte vectors.
+//
+// The rows of a slab; the byte offsets are used where they fit 32 bits.
+struct SlabRows {
+  int R, ng, row0, row1;
+  __device__ __forceinline__ uint2 bytes(int g, int half) const {
+    const uint32_t b = min(16u * R * g + (half ? 16u * R : 0), 16u * R * (ng - 1));
+    return {b + 16u * row0, b + 16u * row1};
+  }
+  __device__ __forceinline__ int2 vectors(int g, int half) const {
+    const int b = min(g + half, ng - 1) * R;
+    return {b + row0, b + row1};
+  }
+};
+
+// A window of up to 64 rows over all slabs of a pass-1 column cluster (they read
+// the same input), each row with the offset and the stride of its own slab from
+// the row table (Program::rowtab).  The layout makes windows only where these
+// offsets fit 32 bits.
+struct WindowRows {
+  int ng;
+  uint32_t off0, str0, off1, str1;
+  __device__ __forceinline__ uint2 bytes(int g, int half) const {
+    const uint32_t c = min(g + half, ng - 1);
+    return {__umul24(c, str0) + off0, __umul24(c, str1) + off1};
+  }
+  __device__ __forceinline__ int2 vectors(int g, int half) const {
+    const uint2 b = bytes(g, half);
+    return {static_cast<int>(b.x >> 4), static_cast<int>(b.y >> 4)};
+  }
+};
+
 // FP32, v_mfma_f32_32x32x2f32, for the shares whose numbers split32_stream does
 // not take: lanes 0-31 read rows 0-31 of column group g,
 // lanes 32-63 rows 0-31 of group g + 1, 16 bytes (4 columns) each; element s
@@ -261,14 +294,13 @@ __device__ __forceinline__ void wave_sum_store(const T* lds, const bwl::WorkItem
 // half-wave, are written to the wave's own LDS slot and read back in the MFMA
 // layout one step ahead of their MFMAs.  LDS operations of a wave run in
 // order, so a read sees the write before it.
-template <int NC, int KU, int D, bool TWO>
+template <int NC, int KU, int D, bool TWO, typename Rows>
 __device__ __forceinline__ void mfma32_stream(const flt4* __restrict__ base,
                                               const int32_t* __restrict__ gi,
-                                              const float* __restrict__ XB, int ng, int R, int half,
+                                              const float* __restrict__ XB, int ng, const Rows& rows, int half,
                                               int r0, float* slot, floatx16 (&acc)[2][NC]) {
   constexpr int NB = 32 * NC;
   constexpr int G = 2 * KU;  // groups per step
-  const int rA0 = min(r0, R - 1), rA1 = min(r0 + 32, R - 1);
   const int nsteps = (ng + G - 1) / G;
   flt4 a0[D][KU], a1[D][KU];
   flt4 bq[D][KU][NC];  // this lane's 16-byte pieces of the four input rows of group 2u + half
@@ -279,9 +311,9 @@ __device__ __forceinline__ void mfma32_stream(const flt4* __restrict__ base,
                   flt4 (&bb)[KU][NC]) {
 #pragma unroll
     for (int u = 0; u < KU; ++u) {
-      const int ga = min(step * G + 2 * u + half, ng - 1);
-      x0[u] = __builtin_nontemporal_load(base + ga * R + rA0);
-      if (TWO) x1[u] = __builtin_nontemporal_load(base + ga * R + rA1);
+      const int2 at = rows.vectors(step * G + 2 * u, half);
+      x0[u] = __builtin_nontemporal_load(base + at.x);
+      if (TWO) x1[u] = __builtin_nontemporal_load(base + at.y);
       // rows z .. z + 3 of XB are contiguous and 128-byte aligned; 32-bit
       // offsets (xt_size * NB < 2^32, checked by the host)
       const uint32_t zo = static_cast<uint32_t>(z[u]) * NB + 4 * r0;
@@ -438,17 +470,13 @@ struct SplitRange {
 // zero) are added to acc after it: one chain per wave has 1.4e-7 against 64
 // bits on the 24 300-DoF operator, this 1.1e-7 as the FP32 instructions.
 // Returns whether all input entries were in the range of the split.
-template <int NC, int D, bool TWO>
+template <int NC, int D, bool TWO, typename Rows>
 __device__ __forceinline__ bool split32_stream(const flt4* __restrict__ base,
                                                const int32_t* __restrict__ gi,
-                                               const float* __restrict__ XB, int ng, int R,
-                                               int half, int r0, float* slot,
+                                               const float* __restrict__ XB, int ng,
+                                               const Rows& rows, int half, int r0, float* slot,
                                                floatx16 (&acc)[2][NC]) {
   constexpr int NB = 32 * NC, KU = 2, G = 4;
-  // byte offsets from base: of group 2 u + half of step 0, and of the last group
-  const uint32_t row0 = 16u * min(r0, R - 1), row1 = 16u * min(r0 + 32, R - 1);
-  const uint32_t gsz = 16u * R;
-  const uint32_t last = gsz * (ng - 1);
   flt4 a0[D][KU], a1[D][KU];
   flt4 bq[D][KU][NC];
   int zz[D][KU];
@@ -458,10 +486,10 @@ __device__ __forceinline__ bool split32_stream(const flt4* __restrict__ base,
                   flt4 (&bb)[KU][NC]) {
 #pragma unroll
     for (int u = 0; u < KU; ++u) {
-      const uint32_t g = min(gsz * static_cast<uint32_t>(step * G + 2 * u) + (half ? gsz : 0), last);
+      const uint2 at = rows.bytes(step * G + 2 * u, half);
       const char* b = reinterpret_cast<const char*>(base);
-      x0[u] = __builtin_nontemporal_load(reinterpret_cast<const flt4*>(b + (g + row0)));
-      if (TWO) x1[u] = __builtin_nontemporal_load(reinterpret_cast<const flt4*>(b + (g + row1)));
+      x0[u] = __builtin_nontemporal_load(reinterpret_cast<const flt4*>(b + at.x));
+      if (TWO) x1[u] = __builtin_nontemporal_load(reinterpret_cast<const flt4*>(b + at.y));
       const uint32_t zo = static_cast<uint32_t>(z[u]) * NB + 4 * r0;
 #pragma unroll
       for (int c = 0; c < NC; ++c) bb[u][c] = *reinterpret_cast<const flt4*>(XB + zo + 128 * c);
@@ -561,11 +589,12 @@ __device__ __forceinline__ bool split32_stream(const flt4* __restrict__ base,
   return seen.inside();
 }
 
-template <int PASS, int NC, int W>
+// WIN: the items are windows (pass 1 of long operators, rounds of 64 columns).
+template <int PASS, int NC, int W, bool WIN>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(NC > 1 ? 2 : 3))) void
 k_slab_mfma32(const bwl::WorkItem* __restrict__ wis, XcdSplit xs,
               const int32_t* __restrict__ gidx, const float* __restrict__ data,
-              const float* __restrict__ XB, BatchOut<float> o) {
+              const float* __restrict__ XB, const int64_t* __restrict__ rowtab, BatchOut<float> o) {
   constexpr int NB = 32 * NC, KU = 1, D = 2, G = 4;
   // of the FP32 stream (KU, D: a small ring, it runs rarely) and the split one;
   // with DS = 2 the 32-wide kernel has three waves per SIMD (3: two, 3-7 % slower)
@@ -583,28 +612,44 @@ k_slab_mfma32(const bwl::WorkItem* __restrict__ wis, XcdSplit xs,
   const int ng = __builtin_amdgcn_readfirstlane(min(wi.ngroups, G * (nst * (wave + 1) / W)) - g0);
   const int half = lane >> 5;  // which group of the pair
   const int r0 = lane & 31;
-  const flt4* __restrict__ base =
-      reinterpret_cast<const flt4*>(data + wi.data_off) + static_cast<int64_t>(g0) * R;
   const int32_t* __restrict__ gi = gidx + __builtin_amdgcn_readfirstlane(wi.gbeg) + g0;
   floatx16 acc[2][NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c) acc[0][c] = acc[1][c] = floatx16{0};
   float* mine = lds + wave * 32 * NB;  // the wave's B slot, then its image of the sums
   const bool two = R > 32;
-  bool done = ng <= 0;
-  if (!done && static_cast<int64_t>(ng) * R < (1 << 27)) {  // its 32-bit byte offsets
-    if (two)
-      done = split32_stream<NC, DS, true>(base, gi, XB, ng, R, half, r0, mine, acc);
-    else
-      done = split32_stream<NC, DS, false>(base, gi, XB, ng, R, half, r0, mine, acc);
-  }
-  if (!done) {
+  auto run = [&](const flt4* __restrict__ base, const auto& rows, bool fits) {
+    bool done = ng <= 0;
+    if (!done && fits) {
+      if (two)
+        done = split32_stream<NC, DS, true>(base, gi, XB, ng, rows, half, r0, mine, acc);
+      else
+        done = split32_stream<NC, DS, false>(base, gi, XB, ng, rows, half, r0, mine, acc);
+    }
+    if (!done) {
 #pragma unroll
-    for (int c = 0; c < NC; ++c) acc[0][c] = acc[1][c] = floatx16{0};
-    if (two)
-      mfma32_stream<NC, KU, D, true>(base, gi, XB, ng, R, half, r0, mine, acc);
-    else
-      mfma32_stream<NC, KU, D, false>(base, gi, XB, ng, R, half, r0, mine, acc);
+      for (int c = 0; c < NC; ++c) acc[0][c] = acc[1][c] = floatx16{0};
+      if (two)
+        mfma32_stream<NC, KU, D, true>(base, gi, XB, ng, rows, half, r0, mine, acc);
+      else
+        mfma32_stream<NC, KU, D, false>(base, gi, XB, ng, rows, half, r0, mine, acc);
+    }
+  };
+  const int row0 = min(r0, R - 1), row1 = min(r0 + 32, R - 1);
+  if constexpr (WIN) {
+    const int64_t* __restrict__ tab = rowtab + wi.out_row;
+    const int64_t e0 = tab[row0], e1 = tab[row1], e = tab[0] >> 8;
+    const int64_t first =
+        static_cast<int64_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(e >> 32))) << 32 |
+        static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(e)));
+    const uint32_t s0 = 16u * (e0 & 0xff), s1 = 16u * (e1 & 0xff);
+    const uint32_t g = static_cast<uint32_t>(wi.data_off) + g0;  // the wave's first group
+    const WindowRows rows{ng, 16u * static_cast<uint32_t>((e0 >> 8) - first) + g * s0, s0,
+                          16u * static_cast<uint32_t>((e1 >> 8) - first) + g * s1, s1};
+    run(reinterpret_cast<const flt4*>(data) + first, rows, true);
+  } else {
+    run(reinterpret_cast<const flt4*>(data + wi.data_off) + static_cast<int64_t>(g0) * R,
+        SlabRows{R, ng, row0, row1}, static_cast<int64_t>(ng) * R < (1 << 27));
   }
   auto put = [&](const floatx16 (&a)[NC]) {
 #pragma unroll

@@ -99,12 +99,18 @@ struct DevItems {
 };
 
 struct DevPass {
-  DevItems single, batched;
+  DevItems single, batched, wide;  // wide: rounds of 64 columns, if rowtab
   int gather_cols = 0;        // pass 1: longest work item's columns if it may gather x itself
   int32_t* gidx = nullptr;
   int32_t* rowmap = nullptr;  // pass 1: t entry of every slab row
+  int64_t* rowtab = nullptr;  // pass 1, windows: where every slab row lies (bwl::Program::rowtab)
   void* data = nullptr;
   int64_t data_bytes = 0;
+
+  // where the partial sums of `wide` begin in the batched scratch
+  size_t wide_offset(int cols, int es) const {
+    return (batched.scratch_bytes(cols, es) + 255) / 256 * 256;
+  }
 };
 
 // The read-only device layout of one operator (H or H^T) at one precision.
@@ -231,11 +237,18 @@ int upload_pass(const bwl::Layout& L, const bwl::Program& P, DevPass* dp, hipStr
   if ((rc = upload_items(P.single, &dp->single, allocs)) ||
       (rc = upload_items(P.batched, &dp->batched, allocs)))
     return rc;
+  if (!P.rowtab.empty() && (rc = upload_items(P.wide, &dp->wide, allocs))) return rc;
   if ((rc = dalloc(reinterpret_cast<void**>(&dp->gidx), P.gidx.size() * sizeof(int32_t)))) return rc;
   if (!P.rowmap.empty()) {
     if ((rc = dalloc(reinterpret_cast<void**>(&dp->rowmap), P.rowmap.size() * sizeof(int32_t))))
       return rc;
     HIPCHK(hipMemcpy(dp->rowmap, P.rowmap.data(), P.rowmap.size() * sizeof(int32_t),
+                     hipMemcpyHostToDevice));
+  }
+  if (!P.rowtab.empty()) {
+    if ((rc = dalloc(reinterpret_cast<void**>(&dp->rowtab), P.rowtab.size() * sizeof(int64_t))))
+      return rc;
+    HIPCHK(hipMemcpy(dp->rowtab, P.rowtab.data(), P.rowtab.size() * sizeof(int64_t),
                      hipMemcpyHostToDevice));
   }
   dp->data_bytes = P.data_elems * static_cast<int64_t>(sizeof(T));
@@ -432,7 +445,8 @@ int build_op(bw_hip_handle* hd, const bw_flat_hmat* h, bool adjoint, hipStream_t
                       (L.pass1.single.part_elems + L.pass2.single.part_elems) * sizeof(T) +
                       (op.p1.single.nwi + op.p1.batched.nwi + op.p2.single.nwi + op.p2.batched.nwi) *
                           sizeof(bwl::WorkItem) +
-                      (L.pass1.gidx.size() + L.pass2.gidx.size()) * sizeof(int32_t);
+                      (L.pass1.gidx.size() + L.pass2.gidx.size()) * sizeof(int32_t) +
+                      L.pass1.rowtab.size() * sizeof(int64_t);
   op.present = true;
   return BW_OK;
 }
@@ -501,15 +515,20 @@ int ensure_op_scratch(bw_hip_handle* hd, StreamCtx* ctx, int adj, int fp32, bool
       void* partb[2] = {nullptr, nullptr};
       rc = dev_alloc(&xb, static_cast<size_t>(op.xt_size) * cols * es, &ctx->allocs, "scratch");
       for (int p = 0; p < 2 && !rc; ++p)
-        rc = dev_alloc(&partb[p], (p ? op.p2 : op.p1).batched.scratch_bytes(cols, es), &ctx->allocs,
-                       "scratch");
+        rc = dev_alloc(&partb[p], (p ? op.p2 : op.p1).wide_offset(cols, es) +
+                                      (p ? op.p2 : op.p1).wide.scratch_bytes(cols, es),
+                       &ctx->allocs, "scratch");
       if (rc) {
         undo_allocs(ctx, mark_b, rc);
         if (cols > 32) continue;
         return rc;
       }
       for (int p = 0; p < 2; ++p) {
-        const hipError_t e = zero_counters((p ? op.p2 : op.p1).batched, partb[p], cols, es);
+        const DevPass& dp = p ? op.p2 : op.p1;
+        hipError_t e = zero_counters(dp.batched, partb[p], cols, es);
+        if (e == hipSuccess)
+          e = zero_counters(dp.wide, static_cast<unsigned char*>(partb[p]) + dp.wide_offset(cols, es),
+                            cols, es);
         if (e != hipSuccess)
           return undo_allocs(ctx, mark, fail(BW_EHIP, std::string("scratch: zero fill: ") + hipGetErrorString(e)));
       }
@@ -1304,17 +1323,33 @@ int check_batched(bw_hip_handle* hd, bool adjoint, int nrhs, const double* X, in
 // The MFMA kernel of one pass of a round of NB columns, and the reduction of
 // its split slabs if that is a launch of its own.
 template <int PASS, int NB, typename T>
-void launch_batched_pass(const DevPass& dp, hipStream_t st, const T* xb, const BatchOut<T>& o) {
-  const DevItems& di = dp.batched;
+void launch_batched_pass(const DevPass& dp, hipStream_t st, const T* xb, void* part, int cols,
+                         BatchOut<T> o) {
+  const bool wide = PASS == 1 && NB == 64 && dp.rowtab;
+  const DevItems& di = wide ? dp.wide : dp.batched;
+  if (wide) part = static_cast<unsigned char*>(part) + dp.wide_offset(cols, sizeof(T));
+  o.part = static_cast<T*>(part);
+  o.sp = di.sums(part, cols, sizeof(T));
   const dim3 grid(di.blocks), block(64 * kBatchWaves);
   const T* data = static_cast<const T*>(dp.data);
   if (di.nwi > 0) {
-    if constexpr (sizeof(T) == 4 && NB >= 32)
-      hipLaunchKernelGGL((k_slab_mfma32<PASS, NB / 32, kBatchWaves>), grid, block, 0, st, di.wis,
-                         di.xs, dp.gidx, data, xb, o);
-    else
+#define BW_MFMA32(WIN)                                                                           \
+  hipLaunchKernelGGL((k_slab_mfma32<PASS, NB / 32, kBatchWaves, WIN>), grid, block, 0, st, di.wis, \
+                     di.xs, dp.gidx, data, xb, dp.rowtab, o)
+    if constexpr (sizeof(T) == 4 && NB >= 32) {
+      if constexpr (PASS == 1 && NB == 64) {
+        if (wide)
+          BW_MFMA32(true);
+        else
+          BW_MFMA32(false);
+      } else {
+        BW_MFMA32(false);
+      }
+    } else {
       hipLaunchKernelGGL((k_slab_mfma16<T, PASS, NB / 16, kBatchWaves>), grid, block, 0, st, di.wis,
                          di.xs, dp.gidx, data, xb, o);
+    }
+#undef BW_MFMA32
   }
   if (di.nred > 0 && !di.in_kernel())
     hipLaunchKernelGGL((k_reduce_b<PASS, NB, T>), dim3(di.nred), dim3(256), 0, st, di.reds,
@@ -1344,8 +1379,6 @@ int launch_round(bw_hip_handle* hd, const DevOp& op, const OpScratch& s, int nk,
   BatchOut<T> o1{};
   o1.tout = xb;
   o1.nk = NB;
-  o1.part = static_cast<T*>(s.partb[0]);
-  o1.sp = op.p1.batched.sums(s.partb[0], s.xb_cols, sizeof(T));
   o1.dof = dof;
   o1.rowmap = op.p1.rowmap;
   BatchOut<T> o2{};
@@ -1354,12 +1387,10 @@ int launch_round(bw_hip_handle* hd, const DevOp& op, const OpScratch& s, int nk,
   o2.yc = yc;
   o2.nk = nk;
   o2.yvec = yc == 1 && yr % 2 == 0 && reinterpret_cast<uintptr_t>(Y) % 16 == 0;
-  o2.part = static_cast<T*>(s.partb[1]);
-  o2.sp = op.p2.batched.sums(s.partb[1], s.xb_cols, sizeof(T));
   o2.perm = orig ? op.perm_out : nullptr;
   o2.dof = dof;
-  launch_batched_pass<1, NB>(op.p1, st, xb, o1);
-  launch_batched_pass<2, NB>(op.p2, st, xb, o2);
+  launch_batched_pass<1, NB>(op.p1, st, xb, s.partb[0], s.xb_cols, o1);
+  launch_batched_pass<2, NB>(op.p2, st, xb, s.partb[1], s.xb_cols, o2);
   HIPCHK(hipGetLastError());
   return BW_OK;
 }

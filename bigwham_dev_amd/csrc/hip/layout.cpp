@@ -251,6 +251,14 @@ constexpr int64_t kItemBatched = 96 * 1024, kItemBatchedMin = 16 * 1024, kBatche
 // matvec: 26.6 us at 64 KiB, 22.8 at 48; 6 400-DoF mode-1 19.5 at 64 and 48,
 // 20.5 at 32).
 constexpr int64_t kPass1Share = 1500, kPass1MinBytes = 48 * 1024;
+// Rounds of 64 columns read four times the bytes of a 16-row slab as input rows,
+// and its 32-row tiles are half empty: from this size on they take pass 1 in
+// windows of 64 rows over all slabs of a column cluster instead (24 300 DoF,
+// pass 1: 115 us in slabs, 80 + 7 in windows; whole products 203 -> 186 us at 46 M
+// entries in pass 1, 97 -> 90 at 15 M, mode-1 130 -> 123 at 21 M but 71 -> 76 at
+// 10 M).  Narrower rounds lose by the split windows (16 columns 3-10 %, 32 columns
+// -4 to +4 %), and FP64 takes 277 us in slabs, 288 in windows.
+constexpr int64_t kWindowEntries = 12 << 20, kMaxWindowGroups = 1 << 20;
 constexpr int64_t kSortEntries = 200 << 20;
 // A pass wants at least this many workgroups (of 256 compute units); in pass 2,
 // operators with fewer slabs that fit one work item each get slabs of fewer rows (4 000-
@@ -262,12 +270,13 @@ constexpr int kMinRows = 16;
 // XCDs in eight contiguous ranges of about equal cost.  row_tile: rows that a
 // kernel's work comes in (the MFMA tile; 1: cost is bytes).  sorted: costliest
 // first within each XCD's range, so that a range ends on its small items.
-void cut_items(const Program& P, const LayoutOptions& opt, int64_t wi_bytes, int row_tile,
-               bool sorted, ItemList* il) {
+// windows: the slabs are windows over P.rowtab.
+void cut_items(const std::vector<SlabDesc>& slabs, const LayoutOptions& opt, int64_t wi_bytes,
+               int row_tile, bool sorted, bool windows, ItemList* il) {
   const int V = opt.vec_elems;
   *il = ItemList{};
   int64_t part = 0;
-  for (const SlabDesc& sd : P.slabs) {
+  for (const SlabDesc& sd : slabs) {
     const int64_t bytes = sd.ngroups * sd.rows * V * opt.elem_bytes;
     int64_t nwi = std::max<int64_t>(1, (bytes + wi_bytes / 2) / wi_bytes);
     nwi = std::min<int64_t>(nwi, std::max<int64_t>(1, sd.ngroups));
@@ -277,7 +286,7 @@ void cut_items(const Program& P, const LayoutOptions& opt, int64_t wi_bytes, int
       const int64_t g0 = w * per;
       const int64_t g1 = std::min(sd.ngroups, g0 + per);
       WorkItem wi{};
-      wi.data_off = sd.data_off + g0 * sd.rows * V;
+      wi.data_off = windows ? g0 : sd.data_off + g0 * sd.rows * V;
       wi.gbeg = static_cast<int32_t>(sd.gbeg + g0);
       wi.ngroups = static_cast<int32_t>(g1 - g0);
       wi.rows = sd.rows;
@@ -343,13 +352,45 @@ void finalize_program(Program* P, const LayoutOptions& opt, int64_t wi_single, b
   }
   P->data_elems = data;
   const bool tuned = opt.wi_bytes > 0;
-  cut_items(*P, opt, tuned ? opt.wi_bytes : wi_single, 1, sort_single, &P->single);
-  const int64_t batched =
-      static_cast<int64_t>(P->slabs.size()) >= kMinSlabs
-          ? kItemBatched
-          : std::min(kItemBatched, std::max(kItemBatchedMin, data / kBatchedItems));
-  cut_items(*P, opt, tuned ? opt.wi_bytes : batched * opt.elem_bytes,
-            opt.elem_bytes == 8 ? 16 : 32, true, &P->batched);
+  cut_items(P->slabs, opt, tuned ? opt.wi_bytes : wi_single, 1, sort_single, false, &P->single);
+  auto batched_bytes = [&](size_t slabs) {
+    if (tuned) return opt.wi_bytes;
+    return opt.elem_bytes * (static_cast<int64_t>(slabs) >= kMinSlabs
+                                 ? kItemBatched
+                                 : std::min(kItemBatched, std::max(kItemBatchedMin, data / kBatchedItems)));
+  };
+  const int row_tile = opt.elem_bytes == 8 ? 16 : 32;
+  cut_items(P->slabs, opt, batched_bytes(P->slabs.size()), row_tile, true, false, &P->batched);
+  P->wide = ItemList{};
+  P->rowtab.clear();
+  if (opt.elem_bytes != 4 || tuned || P->rowmap.empty() || data < kWindowEntries) return;
+  // the rows of a window lie within 192 rows of slabs: 32-bit byte offsets
+  for (const SlabDesc& sd : P->slabs)
+    if (sd.ngroups >= kMaxWindowGroups) return;
+  // Windows of up to 64 rows over the slabs of one column cluster, whose rows
+  // follow each other in the row map.
+  std::vector<SlabDesc> win;
+  size_t i = 0;
+  while (i < P->slabs.size()) {
+    const SlabDesc& a = P->slabs[i];
+    const RunDesc& ra = P->runs[a.run_beg];
+    int64_t rows = 0;
+    for (; i < P->slabs.size(); ++i) {
+      const SlabDesc& sd = P->slabs[i];
+      const RunDesc& rd = P->runs[sd.run_beg];
+      if (rd.zoff != ra.zoff || rd.ncols != ra.ncols) break;
+      for (int32_t r = 0; r < sd.rows; ++r)
+        P->rowtab.push_back((sd.data_off / V + r) << 8 | sd.rows);
+      rows += sd.rows;
+    }
+    for (int64_t r = 0; r < rows; r += 64) {
+      SlabDesc w = a;
+      w.rows = static_cast<int32_t>(std::min<int64_t>(64, rows - r));
+      w.out_row0 = a.out_row0 + r;
+      win.push_back(w);
+    }
+  }
+  cut_items(win, opt, batched_bytes(win.size()), row_tile, true, true, &P->wide);
 }
 
 }  // namespace
@@ -589,9 +630,10 @@ int check_layout_limits(const Layout& L, std::string* msg) {
   }
   for (const Program* P : {&L.pass1, &L.pass2}) {
     if (static_cast<int64_t>(P->gidx.size()) >= lim || P->single.part_elems >= lim ||
-        P->batched.part_elems >= lim || static_cast<int64_t>(P->rowmap.size()) >= lim ||
+        P->batched.part_elems >= lim || P->wide.part_elems >= lim || static_cast<int64_t>(P->rowmap.size()) >= lim ||
         static_cast<int64_t>(P->single.wis.size()) >= lim / 4 ||
-        static_cast<int64_t>(P->batched.wis.size()) >= lim / 4) {
+        static_cast<int64_t>(P->batched.wis.size()) >= lim / 4 ||
+        static_cast<int64_t>(P->wide.wis.size()) >= lim / 4) {
       *msg = "matrix too large for 32-bit layout descriptors";
       return BW_ESHAPE;
     }

@@ -117,6 +117,12 @@ struct Program {
   std::vector<RunDesc> runs;
   std::vector<Piece> pieces;
   ItemList single, batched;       // of the single-vector and the batched kernels
+  // Pass 1 of long FP32 operators, for rounds of 64 columns: items that are
+  // windows over the rows of rowtab (data_off: first column group); rowtab:
+  // (16-byte vector of the row's first group) << 8 | rows of its slab, for
+  // every row of rowmap.
+  ItemList wide;
+  std::vector<int64_t> rowtab;
   int64_t data_elems = 0;
   int64_t out_rows = 0;
 };

@@ -204,3 +204,29 @@ def test_fp32_not_finite(gpu, cols):
         assert np.array_equal(np.isposinf(got[:, j]), np.isposinf(y)), j
         assert np.array_equal(np.isneginf(got[:, j]), np.isneginf(y)), j
         assert j in (2, 3, 4) or np.all(np.isfinite(y))
+
+
+@pytest.mark.parametrize("adjoint", [False, True])
+def test_windows(gpu, adjoint):
+    """Rounds of 64 columns of long FP32 operators take pass 1 in windows over
+    the slabs of a column cluster: the same columns as narrower rounds give,
+    within the bound, and the same bits on every launch."""
+    import torch
+    S = SyntheticHmat(2300, 2400, 3, 12)
+    assert sum(b.size for b in S.B) > 13 << 20 and sum(a.size for a in S.A) > 13 << 20
+    dev = HipHmat(S, precisions=("fp32",), adjoint=True)
+    n_in = dev.n_rows if adjoint else dev.n_cols
+    X = np.random.default_rng(13).uniform(-1, 1, (n_in, 100))
+    Y, bound = _reference(S, X, adjoint)
+    tol = 2 * (n_in + int(S.lr_pattern[:, 5].sum()) + 8) * U["fp32"] * bound
+    Xd = torch.from_numpy(X).to(gpu)
+    for cols in (33, 64, 100):
+        y = dev.matvec_batched(Xd[:, :cols], original=False, precision="fp32", adjoint=adjoint)
+        assert np.all(np.abs(y.cpu().numpy() - Y[:, :cols]) <= tol[:, :cols]), cols
+        for _ in range(3):
+            assert torch.equal(y, dev.matvec_batched(Xd[:, :cols], original=False,
+                                                     precision="fp32", adjoint=adjoint))
+    # 16 at a time: no windows; FP32 errors of the two ways only
+    z = torch.cat([dev.matvec_batched(Xd[:, k:k + 16], original=False, precision="fp32",
+                                      adjoint=adjoint) for k in range(0, 100, 16)], 1)
+    assert torch.linalg.vector_norm(z - y) <= 1e-6 * torch.linalg.vector_norm(y)
