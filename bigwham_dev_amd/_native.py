@@ -130,6 +130,7 @@ def hip() -> C.CDLL:
         lib.bw_layout_export_rowmap.argtypes = [_vp, C.POINTER(C.c_int32)]
         lib.bw_layout_export_xcd.argtypes = [_vp, C.c_int, C.POINTER(C.c_int32),
                                              C.POINTER(C.c_int32)]
+        lib.bw_layout_items_info.argtypes = [_vp, C.c_int, C.c_int, _i64]
         lib.bw_layout_free.argtypes = [_vp]
         lib.bw_layout_free.restype = None
         lib.bw_layout_last_error.restype = C.c_char_p
@@ -202,7 +203,7 @@ HIP_SYMBOLS = ["bw_hip_create", "bw_hip_matvec", "bw_hip_matvec_noalloc", "bw_hi
                "bw_hip_orthogonalize_work", "bw_hip_orthogonalize", "bw_hip_set_timing",
                "bw_hip_timing_stats", "bw_hip_destroy", "bw_hip_last_error",
                "bw_layout_build", "bw_layout_info", "bw_layout_export", "bw_layout_free",
-               "bw_layout_export_rowmap", "bw_layout_export_xcd",
+               "bw_layout_export_rowmap", "bw_layout_export_xcd", "bw_layout_items_info",
                "bw_layout_last_error", "bw_layout_build_multi", "bw_hip_create_multi",
                "bw_hip_graph_create", "bw_hip_graph_launch", "bw_hip_graph_destroy",
                "bw_hip_graph_create_batched", "bw_hip_stream_release",

@@ -71,31 +71,26 @@ constexpr int kBatchWaves = 4;
 
 // ---------------------------------------------------------------------------
 
-constexpr int kInKernelItems = 1024;
-
 // One work-item list of a pass on the device.
 struct DevItems {
   bwl::WorkItem* wis = nullptr;
   bwl::Reduce* reds = nullptr;  // one per split slab
   int nwi = 0, nred = 0;
+  int ncount = 0;               // counters of split slabs (bwl::ItemList)
   XcdSplit xs = {};
   int blocks = 0;               // workgroups of a launch
   int64_t part_elems = 0;
 
   // bytes of the scratch for `cols` columns, and the counters within it
   size_t part_bytes(int cols, int es) const { return (part_elems * cols * es + 15) / 16 * 16; }
-  size_t scratch_bytes(int cols, int es) const { return part_bytes(cols, es) + nred * sizeof(int32_t); }
-  // Whether the last work item of a split slab adds its partial sums, or a
-  // k_reduce launch.  The launch costs 4-5 us; in the kernel every split work
-  // item holds its place for a store and an atomic round trip more, which adds
-  // up where many follow each other on a compute unit.  Whole matvecs, launch
-  // against in-kernel: 369 items in pass 2 27.6 / 26.7 us, 562 38.6 / 37.5,
-  // 1 339 78.2 / 79.1, 3 279 158 / 169.
-  bool in_kernel() const { return nwi <= kInKernelItems; }
-  SplitSums sums(void* part, int cols, int es) const {
-    if (!in_kernel()) return {reds, nullptr};
-    return {reds, reinterpret_cast<int32_t*>(static_cast<unsigned char*>(part) + part_bytes(cols, es))};
+  size_t scratch_bytes(int cols, int es) const { return part_bytes(cols, es) + ncount * sizeof(int32_t); }
+  // the counters: a null pointer always goes with ncount = 0
+  int32_t* counters(void* part, int cols, int es) const {
+    if (ncount == 0) return nullptr;
+    return reinterpret_cast<int32_t*>(static_cast<unsigned char*>(part) + part_bytes(cols, es));
   }
+  SplitSums sums(void* part, int cols, int es) const { return {reds, counters(part, cols, es)}; }
+  bool reduce_launch() const { return nred > ncount; }
 };
 
 struct DevPass {
@@ -209,11 +204,10 @@ std::atomic<double> g_fp32_rank_tol{0.0};
 int upload_items(const bwl::ItemList& il, DevItems* di, std::vector<void*>* allocs) {
   di->nwi = static_cast<int>(il.wis.size());
   di->nred = static_cast<int>(il.reds.size());
+  di->ncount = il.counters;
   di->part_elems = il.part_elems;
-  int most = 0;
-  for (int x = 0; x < bwl::kXcds; ++x) most = std::max(most, il.xcd[x + 1] - il.xcd[x]);
   for (int x = 0; x <= bwl::kXcds; ++x) di->xs.s[x] = il.xcd[x];
-  di->blocks = bwl::kXcds * most;
+  di->blocks = il.blocks();
   int rc;
   if ((rc = dev_alloc(reinterpret_cast<void**>(&di->wis), il.wis.size() * sizeof(bwl::WorkItem),
                       allocs, "create")) ||
@@ -470,8 +464,8 @@ hipError_t zero_now(void* p, size_t bytes) {
 
 // Zeroes the split-slab counters of fresh scratch.
 hipError_t zero_counters(const DevItems& di, void* part, int cols, int es) {
-  if (di.nred == 0 || !di.in_kernel()) return hipSuccess;
-  return zero_now(di.sums(part, cols, es).count, di.nred * sizeof(int32_t));
+  if (di.ncount == 0) return hipSuccess;
+  return zero_now(di.counters(part, cols, es), di.ncount * sizeof(int32_t));
 }
 
 // Allocates what `ctx` lacks for operator [adj][fp32]: the single-vector
@@ -731,7 +725,7 @@ int launch_matvec(bw_hip_handle* hd, DevOp& op, const OpScratch& s, double* y_fu
     launch_slab<T, T, 1>(op.p1, op.unroll[0], st, xt, xt, part1, nullptr, dof);
   }
   if (timing) (void)hipEventRecord(hd->ev[2], st);
-  if (op.p1.single.nred > 0 && !op.p1.single.in_kernel())
+  if (op.p1.single.reduce_launch())
     hipLaunchKernelGGL((k_reduce<T, T>), dim3(op.p1.single.nred), dim3(64), 0, st,
                        op.p1.single.reds, op.p1.single.nred, part1, xt, nullptr, dof, op.p1.rowmap);
   if (timing) (void)hipEventRecord(hd->ev[3], st);
@@ -740,7 +734,7 @@ int launch_matvec(bw_hip_handle* hd, DevOp& op, const OpScratch& s, double* y_fu
                               dof);
   }
   if (timing) (void)hipEventRecord(hd->ev[4], st);
-  if (op.p2.single.nred > 0 && !op.p2.single.in_kernel())
+  if (op.p2.single.reduce_launch())
     hipLaunchKernelGGL((k_reduce<T, double>), dim3(op.p2.single.nred), dim3(64), 0, st,
                        op.p2.single.reds, op.p2.single.nred, part2, yd, orig ? op.perm_out : nullptr, dof, nullptr);
   if (sd && sd->n_out > 0) {
@@ -920,18 +914,18 @@ int noalloc_matvec(bw_hip_handle* hd, const double* x, double* y, int ordering, 
   // so the call can be captured into a graph.
   const int64_t na = op.xt_t - op.n_in, nb = op.xt_size - (op.xt_t + op.t_total);
   const DevItems &d1 = op.p1.single, &d2 = op.p2.single;
-  int32_t* const c1 = d1.sums(s.part[0], 1, op.elem).count;
-  int32_t* const c2 = d2.sums(s.part[1], 1, op.elem).count;
-  const int zblocks = static_cast<int>((na + nb + d1.nred + d2.nred + 255) / 256);
+  int32_t* const c1 = d1.counters(s.part[0], 1, op.elem);
+  int32_t* const c2 = d2.counters(s.part[1], 1, op.elem);
+  const int zblocks = static_cast<int>((na + nb + d1.ncount + d2.ncount + 255) / 256);
   if (zblocks > 0) {
     if (f32)
       hipLaunchKernelGGL(k_zero_ranges<float>, dim3(zblocks), dim3(256), 0, st,
                          static_cast<float*>(s.xt), op.n_in, op.xt_t, op.xt_t + op.t_total,
-                         op.xt_size, c1, d1.nred, c2, d2.nred);
+                         op.xt_size, c1, d1.ncount, c2, d2.ncount);
     else
       hipLaunchKernelGGL(k_zero_ranges<double>, dim3(zblocks), dim3(256), 0, st,
                          static_cast<double*>(s.xt), op.n_in, op.xt_t, op.xt_t + op.t_total,
-                         op.xt_size, c1, d1.nred, c2, d2.nred);
+                         op.xt_size, c1, d1.ncount, c2, d2.ncount);
   }
   return f32 ? launch_matvec<float>(hd, op, s, nullptr, x, y, ordering, st, nullptr, false)
              : launch_matvec<double>(hd, op, s, nullptr, x, y, ordering, st, nullptr, false);
@@ -1351,7 +1345,7 @@ void launch_batched_pass(const DevPass& dp, hipStream_t st, const T* xb, void* p
     }
 #undef BW_MFMA32
   }
-  if (di.nred > 0 && !di.in_kernel())
+  if (di.reduce_launch())
     hipLaunchKernelGGL((k_reduce_b<PASS, NB, T>), dim3(di.nred), dim3(256), 0, st, di.reds,
                        di.nred, o);
 }

@@ -303,6 +303,8 @@ void cut_items(const std::vector<SlabDesc>& slabs, const LayoutOptions& opt, int
     }
   }
   il->part_elems = part;
+  if (static_cast<int64_t>(il->wis.size()) <= kInKernelItems)
+    il->counters = static_cast<int32_t>(il->reds.size());
   // balanced XCD ranges: cut the WI list where the running cost crosses x/8 of
   // the total (the nearer side of the crossing)
   const int64_t nwi = static_cast<int64_t>(il->wis.size());

@@ -96,16 +96,34 @@ struct SlabDesc {
   int32_t gbeg;        // first entry in gidx
 };
 
+// Whether the last work item of a split slab adds its partial sums, or a
+// k_reduce launch.  The launch costs 4-5 us; in the kernel every split work
+// item holds its place for a store and an atomic round trip more, which adds
+// up where many follow each other on a compute unit.  Whole matvecs, launch
+// against in-kernel: 369 items in pass 2 27.6 / 26.7 us, 562 38.6 / 37.5,
+// 1 339 78.2 / 79.1, 3 279 158 / 169.
+constexpr int64_t kInKernelItems = 1024;
+
 // How the slabs of one pass are handed to workgroups: each work item is one
 // workgroup's share, a whole slab or a range of its column groups.
 struct ItemList {
   std::vector<WorkItem> wis;
   std::vector<Reduce> reds;       // one per split slab
   int64_t part_elems = 0;
+  // Split slabs whose last work item adds the partial sums, with a counter
+  // each: all of them, or none (0) where a reduction launch adds them.
+  int32_t counters = 0;
   // Work items [xcd[x], xcd[x+1]) run on XCD x: eight contiguous ranges of
   // about equal bytes; xcd_blocks groups of four work items cover the longest.
   int32_t xcd[kXcds + 1] = {};
   int32_t xcd_blocks = 0;
+
+  // workgroups of a launch: one per work item of the longest range, on every XCD
+  int32_t blocks() const {
+    int32_t most = 0;
+    for (int x = 0; x < kXcds; ++x) most = xcd[x + 1] - xcd[x] > most ? xcd[x + 1] - xcd[x] : most;
+    return kXcds * most;
+  }
 };
 
 // One pass (1 or 2) of one operator (H or H^T) at one precision.

@@ -147,6 +147,21 @@ int bw_layout_export_xcd(const bw_layout* lay, int pass, int32_t* xcd, int32_t* 
   return BW_OK;
 }
 
+// list: 0 single-vector, 1 batched, 2 windows of rounds of 64 columns.
+// info[0..4] = work items, split slabs, partial sums (elements of one column),
+// counters of split slabs, workgroups of the launch.
+int bw_layout_items_info(const bw_layout* lay, int pass, int list, int64_t* info) {
+  if (!lay || !info || (pass != 1 && pass != 2) || list < 0 || list > 2) return BW_EINVAL;
+  const bwl::Program& P = pass == 1 ? lay->L.pass1 : lay->L.pass2;
+  const bwl::ItemList& il = list == 0 ? P.single : list == 1 ? P.batched : P.wide;
+  info[0] = static_cast<int64_t>(il.wis.size());
+  info[1] = static_cast<int64_t>(il.reds.size());
+  info[2] = il.part_elems;
+  info[3] = il.counters;
+  info[4] = il.blocks();
+  return BW_OK;
+}
+
 void bw_layout_free(bw_layout* lay) { delete lay; }
 
 }  // extern "C"

@@ -300,6 +300,11 @@ int bw_layout_export_rowmap(const bw_layout* lay, int32_t* rowmap);
 /* The split of a pass's work items over the 8 XCDs: XCD x runs work items
  * [xcd[x], xcd[x+1]) (9 entries), with `blocks` workgroups of 4 waves. */
 int bw_layout_export_xcd(const bw_layout* lay, int pass, int32_t* xcd, int32_t* blocks);
+/* One work-item list of a pass (list 0: single-vector kernels, 1: batched, 2: the
+ * windows of FP32 rounds of 64 columns): work items, split slabs, partial sums
+ * of one column, counters of the split slabs that their last work item adds (all
+ * of them, or 0: a reduction launch does), workgroups of a launch. */
+int bw_layout_items_info(const bw_layout* lay, int pass, int list, int64_t* info /* 5 */);
 void bw_layout_free(bw_layout* lay);
 const char* bw_layout_last_error(void);
 
