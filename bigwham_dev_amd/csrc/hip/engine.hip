@@ -156,8 +156,9 @@ struct StreamCtx {
 
 // Allocation-failure hook for tests of the cleanup paths: with the
 // environment variable BWHIP_FAIL_ALLOC_AT=k (k >= 1), the k-th device or
-// pinned-host allocation made by one C-ABI call fails as if the memory were
-// exhausted.  The count restarts at every call that allocates.
+// pinned-host allocation made by one C-ABI call asks the runtime for more than
+// any machine has, and fails there as if the memory were exhausted.  The count
+// restarts at every call that allocates.
 thread_local int64_t g_alloc_seq = 0;
 thread_local int64_t g_alloc_fail_at = 0;
 
@@ -167,16 +168,22 @@ void arm_alloc_hook() {
   g_alloc_fail_at = e ? std::atoll(e) : 0;
 }
 
-bool alloc_hook_fires() { return g_alloc_fail_at > 0 && ++g_alloc_seq == g_alloc_fail_at; }
+// Bytes to ask for where a caller needs `bytes`.
+size_t alloc_bytes(size_t bytes) {
+  const bool fires = g_alloc_fail_at > 0 && ++g_alloc_seq == g_alloc_fail_at;
+  return fires ? size_t(1) << 50 : std::max<size_t>(bytes, 16);
+}
 
 // hipMalloc of at least 16 bytes, recorded in `allocs`; BW_ENOMEM on failure.
+// A failure is reported here and may be handled by the caller: it must not stay
+// the thread's last error, which the checks after later launches (here and in
+// the caller's other libraries) would take for theirs.
 int dev_alloc(void** p, size_t bytes, std::vector<void*>* allocs, const char* what) {
   *p = nullptr;
-  if (alloc_hook_fires())
-    return fail(BW_ENOMEM, std::string(what) + ": hipMalloc: out of memory (BWHIP_FAIL_ALLOC_AT)");
-  const hipError_t e = hipMalloc(p, std::max<size_t>(bytes, 16));
+  const hipError_t e = hipMalloc(p, alloc_bytes(bytes));
   if (e != hipSuccess) {
     *p = nullptr;
+    (void)hipGetLastError();
     return fail(BW_ENOMEM, std::string(what) + ": hipMalloc: " + hipGetErrorString(e));
   }
   allocs->push_back(*p);
@@ -185,10 +192,9 @@ int dev_alloc(void** p, size_t bytes, std::vector<void*>* allocs, const char* wh
 
 int host_pinned_alloc(void** p, size_t bytes, const char* what) {
   *p = nullptr;
-  if (alloc_hook_fires())
-    return fail(BW_ENOMEM, std::string(what) + ": hipHostMalloc: out of memory (BWHIP_FAIL_ALLOC_AT)");
-  if (hipHostMalloc(p, bytes) != hipSuccess) {
+  if (hipHostMalloc(p, alloc_bytes(bytes)) != hipSuccess) {
     *p = nullptr;
+    (void)hipGetLastError();
     return fail(BW_ENOMEM, std::string(what) + ": hipHostMalloc failed");
   }
   return BW_OK;
@@ -857,6 +863,7 @@ void noalloc_bind(int device) {
   void* p = nullptr;
   const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
   if (e != hipSuccess || !p) {
+    (void)hipGetLastError();  // handled: only this entry point is lost
     g_noalloc_err[device] = std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(e);
     return;
   }
