@@ -159,13 +159,19 @@ struct StreamCtx {
 // pinned-host allocation made by one C-ABI call asks the runtime for more than
 // any machine has, and fails there as if the memory were exhausted.  The count
 // restarts at every call that allocates.
+// BWHIP_FAIL_FILL_AT=k fails the k-th zero fill of fresh scratch in the same way.
 thread_local int64_t g_alloc_seq = 0;
 thread_local int64_t g_alloc_fail_at = 0;
+thread_local int64_t g_fill_seq = 0;
+thread_local int64_t g_fill_fail_at = 0;
 
 void arm_alloc_hook() {
   g_alloc_seq = 0;
   const char* e = std::getenv("BWHIP_FAIL_ALLOC_AT");
   g_alloc_fail_at = e ? std::atoll(e) : 0;
+  g_fill_seq = 0;
+  const char* f = std::getenv("BWHIP_FAIL_FILL_AT");
+  g_fill_fail_at = f ? std::atoll(f) : 0;
 }
 
 // Bytes to ask for where a caller needs `bytes`.
@@ -463,6 +469,7 @@ int undo_allocs(StreamCtx* ctx, size_t mark, int rc) {
 // it completes, on the null stream, which does not order non-blocking
 // streams such as torch's.)
 hipError_t zero_now(void* p, size_t bytes) {
+  if (g_fill_fail_at > 0 && ++g_fill_seq == g_fill_fail_at) return hipErrorUnknown;
   hipError_t e = hipMemsetAsync(p, 0, bytes, nullptr);
   if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
   return e;
@@ -478,7 +485,8 @@ hipError_t zero_counters(const DevItems& di, void* part, int cols, int es) {
 // scratch, and with `batched` the batched one.  xt is zeroed here, once
 // (synchronously, before any kernel of the context can use it): the kernels
 // only ever write x and t entries, so the gap and tail stay zero.
-// On failure nothing of this call stays allocated.
+// A failure frees what it leaves incomplete; the single-vector scratch that was
+// complete by then (allocated and zeroed, held by `s`) stays for later calls.
 int ensure_op_scratch(bw_hip_handle* hd, StreamCtx* ctx, int adj, int fp32, bool batched) {
   const DevOp& op = hd->op[adj][fp32];
   OpScratch& s = ctx->op[adj][fp32];
@@ -530,7 +538,7 @@ int ensure_op_scratch(bw_hip_handle* hd, StreamCtx* ctx, int adj, int fp32, bool
           e = zero_counters(dp.wide, static_cast<unsigned char*>(partb[p]) + dp.wide_offset(cols, es),
                             cols, es);
         if (e != hipSuccess)
-          return undo_allocs(ctx, mark, fail(BW_EHIP, std::string("scratch: zero fill: ") + hipGetErrorString(e)));
+          return undo_allocs(ctx, mark_b, fail(BW_EHIP, std::string("scratch: zero fill: ") + hipGetErrorString(e)));
       }
       s.xb = xb;
       s.partb[0] = partb[0];

@@ -8,7 +8,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
-from bigwham_dev_amd import HipHmat
+from bigwham_dev_amd import HipHmat, set_tuning
 from bigwham_dev_amd import _native as N
 from synthetic_hmat import SyntheticHmat
 
@@ -78,3 +78,49 @@ def test_call_after_a_failed_one(case, gpu, monkeypatch, host):
         monkeypatch.delenv("BWHIP_FAIL_ALLOC_AT")
         assert torch.equal(dev.matvec(x, precision="fp32"), ref)
         assert torch.equal((x + x) - x, x)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_failed_zero_fill(gpu, monkeypatch, precision):
+    """A batched call that is the first on its stream makes both kinds of scratch;
+    whichever of its zero fills fails, the calls that follow on that stream
+    have scratch of their own or make it anew, and all of it is given back."""
+    import torch
+    set_tuning(16384, 16384)  # split slabs, so that there are counters to clear
+    try:
+        dev = HipHmat(SyntheticHmat(400, 380, 2, 7), precisions=(precision,))
+    finally:
+        set_tuning(0, 0)
+    X = torch.from_numpy(np.random.default_rng(2).uniform(-1, 1, (dev.n_cols, 40))).to(gpu)
+    x = X[:, 0].contiguous()
+    Y, y = dev.matvec_batched(X, precision=precision), dev.matvec(x, precision=precision)
+    s = torch.cuda.Stream(gpu)
+    with torch.cuda.stream(s):
+        torch.zeros(1, device=gpu)
+        Ys, ys = torch.empty_like(Y), torch.empty_like(y)
+    failed = 0
+    for k in range(20):  # 0: none, so that torch's own buffers are there
+        monkeypatch.setenv("BWHIP_FAIL_FILL_AT", str(k))
+        print(f"{precision}, zero fill {k} failing", flush=True)
+        with torch.cuda.stream(s):
+            try:
+                dev.matvec_batched(X, precision=precision, out=Ys)
+                ok = True
+            except N.BigWhamError as e:
+                assert "zero fill" in str(e)
+                ok = False
+            monkeypatch.delenv("BWHIP_FAIL_FILL_AT")
+            dev.matvec(x, precision=precision, out=ys)
+            assert torch.equal(ys, y)
+            dev.matvec_batched(X, precision=precision, out=Ys)
+            assert torch.equal(Ys, Y)
+        dev.release_stream(s.cuda_stream)
+        torch.cuda.synchronize()
+        if k == 0:
+            before = torch.cuda.mem_get_info(0)[0]
+            continue
+        assert torch.cuda.mem_get_info(0)[0] == before
+        if ok:
+            break
+        failed += 1
+    assert ok and failed >= 3  # xt, and counters of both kinds of scratch
