@@ -24,6 +24,7 @@ import time
 from dataclasses import dataclass, field
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _native as N
 
@@ -104,6 +105,19 @@ class _HostSteps:
         pass
 
 
+def _plain(w: torch.Tensor, V: torch.Tensor) -> bool:
+    """Whether w is one contiguous vector of V's kind that can be read through its
+    pointer: its memory holds its values (no pending negation, no subclass
+    with a meaning of its own) and nothing differentiates through the step.
+    Everything else is left to torch, which computes it or refuses it."""
+    return (type(w) is torch.Tensor and w.dtype == V.dtype and w.device == V.device
+            and w.dim() == 1 and w.numel() == V.shape[1] and w.is_contiguous()
+            and not w.is_neg()
+            and not ((w.requires_grad or V.requires_grad) and torch.is_grad_enabled())
+            and forward_ad.unpack_dual(w).tangent is None
+            and forward_ad.unpack_dual(V).tangent is None)
+
+
 class _DeviceSteps(_HostSteps):
     """The same on the GPU, queued: four kernels per step
     (bw_hip_orthogonalize) that write the column to pinned memory."""
@@ -125,8 +139,7 @@ class _DeviceSteps(_HostSteps):
 
     def queue(self, k, w):
         V = self.V
-        if (self.native and w.dtype == V.dtype and w.device == V.device and w.dim() == 1
-                and w.numel() == V.shape[1] and w.is_contiguous()):
+        if self.native and _plain(w, V):
             rc = self.native.bw_hip_orthogonalize(
                 V.device.index, V.shape[1], k + 1, V.data_ptr(), V.stride(0), w.data_ptr(),
                 V[k + 1].data_ptr(), self.cols[k].data_ptr(), self.work.data_ptr(),
