@@ -146,6 +146,23 @@ __global__ __launch_bounds__(kThreads) void k_normalize(const double* __restrict
     for (int j = threadIdx.x; j <= k; j += kThreads) col[j] = j < k ? h[j] : hn;
 }
 
+// Makes a device current for a scope.  The step stands in for torch operations
+// on vectors of any device, which leave the caller's current device as it is.
+struct CurrentDevice {
+  int before = -1;
+  bool ok;
+
+  explicit CurrentDevice(int device) {
+    ok = hipGetDevice(&before) == hipSuccess && (before == device || hipSetDevice(device) == hipSuccess);
+    if (before == device) before = -1;  // nothing to put back
+  }
+  ~CurrentDevice() {
+    if (before >= 0) (void)hipSetDevice(before);
+  }
+  CurrentDevice(const CurrentDevice&) = delete;
+  CurrentDevice& operator=(const CurrentDevice&) = delete;
+};
+
 // Chunks: at least 256 entries, about 512 workgroups, at most kMaxChunk.
 int chunk_of(int64_t n) {
   const int64_t c = std::max<int64_t>(256, (n + 511) / 512);
@@ -172,7 +189,8 @@ int bw_hip_orthogonalize(int device, int64_t n, int k, const double* V, int64_t 
   if (rc) return rc;
   if (!V || !w || !next || !col || !work || ldv < n) return BW_EINVAL;
   if (work_elems < need) return BW_ESHAPE;
-  if (hipSetDevice(device) != hipSuccess) return BW_EHIP;
+  const CurrentDevice current(device);
+  if (!current.ok) return BW_EHIP;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int chunk = chunk_of(n);
   const int nb = static_cast<int>((n + chunk - 1) / chunk);

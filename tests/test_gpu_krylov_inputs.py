@@ -73,3 +73,13 @@ def test_taken(gpu, name):
     # ||x - exact|| <= ||A^-1|| tol ||b||, and the smallest singular value of A is above 1
     assert torch.linalg.svdvals(A).min() > 1
     assert torch.linalg.vector_norm(x.cpu() - exact) <= 2e-11 * torch.linalg.vector_norm(b)
+
+
+@pytest.mark.skipif(torch.cuda.device_count() < 2, reason="needs two GPUs")
+def test_current_device_is_kept(gpu):
+    """A solve on the second GPU leaves the first one current, as torch does."""
+    A, b = _system("cuda:1")
+    with torch.cuda.device(0):
+        _, _, rel = gmres(lambda v: A @ v, b, tol=1e-11)
+        assert rel <= 1e-11
+        assert torch.empty(1, device="cuda").device.index == 0
