@@ -127,7 +127,9 @@ class _DeviceSteps(_HostSteps):
     def __init__(self, V):
         super().__init__(V)
         restart, n = V.shape[0] - 1, V.shape[1]
-        self.cols = torch.empty((restart, restart + 2), dtype=V.dtype, pin_memory=True)
+        # two rows, as two steps are in flight at most; a step that a cycle left
+        # behind is done before the next cycle's steps, on the same stream
+        self.cols = torch.empty((2, restart + 2), dtype=V.dtype, pin_memory=True)
         self.events = [torch.cuda.Event() for _ in range(2)]
         self.queued = -1
         self.native = None
@@ -142,18 +144,18 @@ class _DeviceSteps(_HostSteps):
         if self.native and _plain(w, V):
             rc = self.native.bw_hip_orthogonalize(
                 V.device.index, V.shape[1], k + 1, V.data_ptr(), V.stride(0), w.data_ptr(),
-                V[k + 1].data_ptr(), self.cols[k].data_ptr(), self.work.data_ptr(),
+                V[k + 1].data_ptr(), self.cols[k & 1].data_ptr(), self.work.data_ptr(),
                 self.work.numel(), torch.cuda.current_stream(V.device).cuda_stream)
             if rc != N.BW_OK:
                 raise N.BigWhamError(rc, "orthogonalize")
         else:
-            self.cols[k, : k + 2].copy_(self._torch_step(k, w), non_blocking=True)
+            self.cols[k & 1, : k + 2].copy_(self._torch_step(k, w), non_blocking=True)
         self.events[k & 1].record(torch.cuda.current_stream(V.device))
         self.queued = k
 
     def column(self, k):
         self.events[k & 1].synchronize()
-        return self.cols[k, : k + 2].tolist()
+        return self.cols[k & 1, : k + 2].tolist()
 
     def close(self):
         # a queued step still writes the pinned columns

@@ -6,7 +6,7 @@ import pytest
 import torch
 from torch.autograd import forward_ad
 
-from bigwham_dev_amd.solvers import gmres
+from bigwham_dev_amd.solvers import _DeviceSteps, gmres
 
 pytestmark = pytest.mark.gpu
 
@@ -83,3 +83,26 @@ def test_current_device_is_kept(gpu):
         _, _, rel = gmres(lambda v: A @ v, b, tol=1e-11)
         assert rel <= 1e-11
         assert torch.empty(1, device="cuda").device.index == 0
+
+
+def test_pinned_columns(gpu):
+    """The pinned memory of a solve grows with the restart length, not with its
+    square (a full-memory solve restarts after thousands of vectors)."""
+    steps = _DeviceSteps(torch.empty((3001, 8), dtype=torch.float64, device=gpu))
+    assert steps.cols.is_pinned() and steps.cols.numel() <= 4 * 3001
+    steps.close()
+
+
+@pytest.mark.parametrize("strided", [False, True])
+@pytest.mark.parametrize("restart", [1, 2, 3, 39])
+def test_restarts(gpu, restart, strided):
+    """Cycles of one step up to the whole space, through the native and the torch
+    step: as many iterations as on the CPU, give or take the last bits."""
+    op = lambda A: lambda v: torch.stack([A @ v, v], 1)[:, 0] if strided else A @ v
+    A, b = _system("cpu")
+    _, n, _ = gmres(op(A), b, restart=restart, tol=1e-10)
+    A, b = _system(gpu)
+    x, m, rel = gmres(op(A), b, restart=restart, tol=1e-10)
+    assert rel <= 1e-10 and abs(m - n) <= 1
+    # the residual itself: rounding of a 40-term product is far below the tolerance
+    assert torch.linalg.vector_norm(b - A @ x) <= 1.01e-10 * torch.linalg.vector_norm(b)
