@@ -6,14 +6,14 @@
 // the gathered input XB[z][NB] (row-major) and of t; a call runs its columns
 // in rounds of NB, columns past nk are zero and never stored.  Rounds of 16
 // columns move half the input rows and partial sums of 32 (24 300 DoF, 32 and
-// 16 columns: FP64 275 and 237 us, FP32 156 and 135); in FP32 a round of 64
-// streams the factors once for twice the columns (312 -> 186, 49 152 DoF 580 ->
-// 367), and wins from 33 columns on (290 + 261 -> 367).  FP64 stays at 32: its
+// 16 columns: FP64 275 and 237 us, FP32 157 and 132); in FP32 a round of 64
+// streams the factors once for twice the columns (314 -> 217, 49 152 DoF 590 ->
+// 426), and wins from 33 columns on (295 + 257 -> 426).  FP64 stays at 32: its
 // time goes with the columns (158 us for one vector).
 //
 // What bounds them: reads from L2 (63-69 G requests a second here and in the
 // single-vector kernel, input rows 25-65 % of them), and at 64 columns the
-// vector and matrix instructions about a third each.
+// FP32 matrix instructions.
 //
 // A workgroup of W waves takes one work item: the waves take contiguous
 // shares of its k-steps, each with a full set of accumulators, and the sums
@@ -242,16 +242,12 @@ __device__ __forceinline__ void wave_sum_store(const T* lds, const bwl::WorkItem
   }
 }
 
-// Where a lane's two rows of a 32-row-tile item lie: byte offsets of column group
-// g + half (at most the last), and the same as index of 16-byte vectors.
+// Where a lane's two rows of a 32-row-tile item lie: the 16-byte vectors of
+// column group g + half (at most the last).
 //
-// The rows of a slab; the byte offsets are used where they fit 32 bits.
+// The rows of a slab.
 struct SlabRows {
   int R, ng, row0, row1;
-  __device__ __forceinline__ uint2 bytes(int g, int half) const {
-    const uint32_t b = min(16u * R * g + (half ? 16u * R : 0), 16u * R * (ng - 1));
-    return {b + 16u * row0, b + 16u * row1};
-  }
   __device__ __forceinline__ int2 vectors(int g, int half) const {
     const int b = min(g + half, ng - 1) * R;
     return {b + row0, b + row1};
@@ -261,22 +257,17 @@ struct SlabRows {
 // A window of up to 64 rows over all slabs of a pass-1 column cluster (they read
 // the same input), each row with the offset and the stride of its own slab from
 // the row table (Program::rowtab).  The layout makes windows only where these
-// offsets fit 32 bits.
+// numbers fit (less than 2^20 groups a slab).
 struct WindowRows {
   int ng;
-  uint32_t off0, str0, off1, str1;
-  __device__ __forceinline__ uint2 bytes(int g, int half) const {
-    const uint32_t c = min(g + half, ng - 1);
-    return {__umul24(c, str0) + off0, __umul24(c, str1) + off1};
-  }
+  int off0, str0, off1, str1;
   __device__ __forceinline__ int2 vectors(int g, int half) const {
-    const uint2 b = bytes(g, half);
-    return {static_cast<int>(b.x >> 4), static_cast<int>(b.y >> 4)};
+    const int c = min(g + half, ng - 1);
+    return {__mul24(c, str0) + off0, __mul24(c, str1) + off1};
   }
 };
 
-// FP32, v_mfma_f32_32x32x2f32, for the shares whose numbers split32_stream does
-// not take: lanes 0-31 read rows 0-31 of column group g,
+// FP32, v_mfma_f32_32x32x2f32: lanes 0-31 read rows 0-31 of column group g,
 // lanes 32-63 rows 0-31 of group g + 1, 16 bytes (4 columns) each; element s
 // of a lane's vector is A[row][k] of MFMA step s, with k = lane / 32
 // selecting the group.  The accumulator holds rows x right-hand sides:
@@ -338,8 +329,8 @@ __device__ __forceinline__ void mfma32_stream(const flt4* __restrict__ base,
   // Sums of one trip of the ring (D steps): the first MFMA of a trip starts
   // them from zero, and they are added to acc when the trip is over.  Short
   // chains instead of a wave's whole share keep the FP32 rounding error of long
-  // work items down (49 152-DoF 3DR0, 32 right-hand sides: 1.1e-7 against 64
-  // bits with chains of 24 MFMAs; one chain per wave 2.5e-7).
+  // work items down (49 152-DoF 3DR0, 32 right-hand sides: 1.06e-7 against 64
+  // bits with chains of 12 MFMAs; one chain per wave 2.5e-7).
   floatx16 p[2][NC];
   auto compute = [&](int step, bool first, const flt4 (&x0)[KU], const flt4 (&x1)[KU]) {
 #pragma unroll
@@ -395,210 +386,16 @@ __device__ __forceinline__ void mfma32_stream(const flt4* __restrict__ base,
   __builtin_amdgcn_sched_barrier(0);
 }
 
-// FP32 products on the bf16 matrix instructions.  A float is the sum of three
-// bf16 numbers (8 + 8 + 8 significant bits, each rounded to nearest), and a
-// product of floats the sum of six products of those; the three left out are
-// below 2^-25 of it.  v_mfma_f32_32x32x16_bf16 sums 16 products in FP32 at 16
-// times the rate of v_mfma_f32_32x32x2f32, so that the matrix work is 6 / 16 of
-// it; the splits (5.5 vector instructions a number) run beside it, on every
-// factor once and on every input row once per work item.  (v_dot2_f32_bf16 with
-// -1 as unpack and subtraction in one is slower: 207 -> 211 us.)  FP32
-// instructions -> this, 64 columns: 24 300 DoF 250 -> 203 us, 49 152 DoF 472 ->
-// 391; 32 columns: 49 152 DoF 314 -> 290, 6 912 DoF 54 -> 43.
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float fltx2 __attribute__((ext_vector_type(2)));
-
-struct Split8 {
-  bf16x8 h, m, l;
-};
-
-// Entries j and j + 1 of a split.
-__device__ __forceinline__ void split2(float x, float y, int j, Split8& o) {
-  fltx2 v = {x, y};
-  const bf16x2 h = __builtin_convertvector(v, bf16x2);
-  v -= __builtin_convertvector(h, fltx2);
-  const bf16x2 m = __builtin_convertvector(v, bf16x2);
-  v -= __builtin_convertvector(m, fltx2);
-  const bf16x2 l = __builtin_convertvector(v, bf16x2);
-  o.h[j] = h.x; o.h[j + 1] = h.y;
-  o.m[j] = m.x; o.m[j + 1] = m.y;
-  o.l[j] = l.x; o.l[j + 1] = l.y;
-}
-
-// The largest magnitudes that a lane has met: in its rows of the slab (one per
-// row tile) and its columns of the input (one per column tile).  The three
-// parts of a number and the products of parts are normal numbers down to
-// 2^-126, so what is lost below it is below 2^-26 of the largest product of a
-// row and a column if their largest numbers are from 2^-100 and their product
-// from 2^-100.  A wave with other rows or columns (save zeros), or with numbers
-// that round to infinity, does its share again in FP32.
-template <int NC>
-struct SplitRange {
-  float a[2] = {0.0f, 0.0f}, b[NC] = {};
-
-  static __device__ __forceinline__ void see(float& m, float x, float y) {
-    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(x), "v"(y));
-  }
-  // for the whole wave
-  __device__ __forceinline__ bool inside() const {
-    constexpr float kInf = 3.3895e38f;  // rounds to infinity in bf16 from there
-    float lo[2] = {kInf, kInf}, hi = 0.0f;
-    auto put = [&](float& l, float m) {
-      hi = fmaxf(hi, m);
-      if (m > 0.0f) l = fminf(l, m);
-    };
-    put(lo[0], a[0]);
-    put(lo[0], a[1]);
-#pragma unroll
-    for (int c = 0; c < NC; ++c) put(lo[1], b[c]);
-#pragma unroll
-    for (int s = 1; s < 64; s *= 2) {
-      lo[0] = fminf(lo[0], __shfl_xor(lo[0], s, 64));
-      lo[1] = fminf(lo[1], __shfl_xor(lo[1], s, 64));
-    }
-    constexpr float kMin = 0x1p-100f;
-    return !__any(hi >= kInf) && lo[0] >= kMin && lo[1] >= kMin && lo[1] >= kMin / lo[0];
-  }
-};
-
-// The same operands, ring and LDS staging as mfma32_stream, 16 columns of the
-// slab (four groups) per step: lanes 0-31 hold groups 4 step and 4 step + 2,
-// lanes 32-63 the two others, so entry 4 u + s of a lane's operands is column s
-// of group 4 step + 2 u + half.  The products of a step go from the smallest
-// to the largest, and the sums of a trip of the ring (D steps, started from
-// zero) are added to acc after it: one chain per wave has 1.4e-7 against 64
-// bits on the 24 300-DoF operator, this 1.1e-7 as the FP32 instructions.
-// Returns whether all input entries were in the range of the split.
-template <int NC, int D, bool TWO, typename Rows>
-__device__ __forceinline__ bool split32_stream(const flt4* __restrict__ base,
-                                               const int32_t* __restrict__ gi,
-                                               const float* __restrict__ XB, int ng,
-                                               const Rows& rows, int half, int r0, float* slot,
-                                               floatx16 (&acc)[2][NC]) {
-  constexpr int NB = 32 * NC, KU = 2, G = 4;
-  flt4 a0[D][KU], a1[D][KU];
-  flt4 bq[D][KU][NC];
-  int zz[D][KU];
-  float bn[KU][4][NC];
-  auto gz = [&](int step, int u) { return gi[min(step * G + 2 * u + half, ng - 1)]; };
-  auto load = [&](int step, const int (&z)[KU], flt4 (&x0)[KU], flt4 (&x1)[KU],
-                  flt4 (&bb)[KU][NC]) {
-#pragma unroll
-    for (int u = 0; u < KU; ++u) {
-      const uint2 at = rows.bytes(step * G + 2 * u, half);
-      const char* b = reinterpret_cast<const char*>(base);
-      x0[u] = __builtin_nontemporal_load(reinterpret_cast<const flt4*>(b + at.x));
-      if (TWO) x1[u] = __builtin_nontemporal_load(reinterpret_cast<const flt4*>(b + at.y));
-      const uint32_t zo = static_cast<uint32_t>(z[u]) * NB + 4 * r0;
-#pragma unroll
-      for (int c = 0; c < NC; ++c) bb[u][c] = *reinterpret_cast<const flt4*>(XB + zo + 128 * c);
-    }
-  };
-  auto stage_b = [&](const flt4 (&bb)[KU][NC]) {
-#pragma unroll
-    for (int u = 0; u < KU; ++u)
-#pragma unroll
-      for (int c = 0; c < NC; ++c)
-        *reinterpret_cast<flt4*>(slot + (2 * u + half) * 4 * NB + 128 * c + 4 * r0) = bb[u][c];
-#pragma unroll
-    for (int u = 0; u < KU; ++u)
-#pragma unroll
-      for (int s = 0; s < 4; ++s)
-#pragma unroll
-        for (int c = 0; c < NC; ++c)
-          bn[u][s][c] = slot[(2 * u + half) * 4 * NB + s * NB + 32 * c + r0];
-  };
-  SplitRange<NC> seen;
-  floatx16 p[2][NC];
-  // MASK: groups past the end have B = 0
-  auto compute = [&](auto MASK, int step, bool first, const flt4 (&x0)[KU], const flt4 (&x1)[KU]) {
-    Split8 s0, s1;
-#pragma unroll
-    for (int u = 0; u < KU; ++u)
-#pragma unroll
-      for (int s = 0; s < 4; s += 2) {
-        split2(x0[u][s], x0[u][s + 1], 4 * u + s, s0);
-        seen.see(seen.a[0], x0[u][s], x0[u][s + 1]);
-        if (TWO) split2(x1[u][s], x1[u][s + 1], 4 * u + s, s1);
-        if (TWO) seen.see(seen.a[1], x1[u][s], x1[u][s + 1]);
-      }
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      Split8 b;
-#pragma unroll
-      for (int u = 0; u < KU; ++u) {
-        const bool ok = !decltype(MASK)::value || step * G + 2 * u + half < ng;
-#pragma unroll
-        for (int s = 0; s < 4; s += 2) {
-          const float y0 = ok ? bn[u][s][c] : 0.0f, y1 = ok ? bn[u][s + 1][c] : 0.0f;
-          split2(y0, y1, 4 * u + s, b);
-          seen.see(seen.b[c], y0, y1);
-        }
-      }
-      auto mul = [&](const bf16x8& x, const bf16x8& y, const bf16x8& z, bool zero) {
-        p[0][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, z, zero ? floatx16{0} : p[0][c], 0, 0, 0);
-        if (TWO)
-          p[1][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(y, z, zero ? floatx16{0} : p[1][c], 0, 0, 0);
-      };
-      mul(s0.m, s1.m, b.m, first);
-      mul(s0.l, s1.l, b.h, false);
-      mul(s0.h, s1.h, b.l, false);
-      mul(s0.m, s1.m, b.h, false);
-      mul(s0.h, s1.h, b.m, false);
-      mul(s0.h, s1.h, b.h, false);
-    }
-  };
-  auto trip = [&](auto MASK, int t0) {
-#pragma unroll
-    for (int j = 0; j < D; ++j) {
-      const int s = t0 + j;
-      __builtin_amdgcn_sched_barrier(0);
-      compute(MASK, s, j == 0, a0[j], a1[j]);
-      __builtin_amdgcn_sched_barrier(0);
-      stage_b(bq[(j + 1) % D]);
-      __builtin_amdgcn_sched_barrier(0);
-      load(s + D, zz[j], a0[j], a1[j], bq[j]);
-#pragma unroll
-      for (int u = 0; u < KU; ++u) zz[j][u] = gz(s + 2 * D, u);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      acc[0][c] += p[0][c];
-      if (TWO) acc[1][c] += p[1][c];
-    }
-  };
-#pragma unroll
-  for (int k = 0; k < D; ++k)
-#pragma unroll
-    for (int u = 0; u < KU; ++u) zz[k][u] = gz(k, u);
-#pragma unroll
-  for (int k = 0; k < D; ++k) {
-    __builtin_amdgcn_sched_barrier(0);
-    load(k, zz[k], a0[k], a1[k], bq[k]);
-#pragma unroll
-    for (int u = 0; u < KU; ++u) zz[k][u] = gz(k + D, u);
-  }
-  __builtin_amdgcn_sched_barrier(0);
-  stage_b(bq[0]);
-  const int full = ng / (G * D);
-  for (int t = 0; t < full; ++t) trip(std::false_type{}, t * D);
-  if (full * G * D < ng) trip(std::true_type{}, full * D);
-  __builtin_amdgcn_sched_barrier(0);
-  return seen.inside();
-}
-
 // WIN: the items are windows (pass 1 of long operators, rounds of 64 columns).
 template <int PASS, int NC, int W, bool WIN>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(NC > 1 ? 2 : 3))) void
 k_slab_mfma32(const bwl::WorkItem* __restrict__ wis, XcdSplit xs,
               const int32_t* __restrict__ gidx, const float* __restrict__ data,
               const float* __restrict__ XB, const int64_t* __restrict__ rowtab, BatchOut<float> o) {
-  constexpr int NB = 32 * NC, KU = 1, D = 2, G = 4;
-  // of the FP32 stream (KU, D: a small ring, it runs rarely) and the split one;
-  // with DS = 2 the 32-wide kernel has three waves per SIMD (3: two, 3-7 % slower)
-  constexpr int DS = 2;
+  // The ring: one group pair per step, three steps (2, 3 and 4 steps: 24 300 DoF,
+  // 100 columns 454, 447 and 457 us; 16 cracks, 32 columns 52.7, 49.1 and 47.9;
+  // 49 152 DoF, 32 columns 302, 306 and 307; two pairs, three steps 457, 54.2, 317)
+  constexpr int NB = 32 * NC, KU = 1, D = 3, G = 4;
   __shared__ __align__(16) float lds[W * 32 * NB];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
@@ -606,7 +403,7 @@ k_slab_mfma32(const bwl::WorkItem* __restrict__ wis, XcdSplit xs,
   if (w < 0) return;
   const bwl::WorkItem wi = wis[w];
   const int R = __builtin_amdgcn_readfirstlane(wi.rows);
-  // this wave's share of the column groups, in steps of the split stream
+  // this wave's share of the column groups
   const int nst = (wi.ngroups + G - 1) / G;
   const int g0 = __builtin_amdgcn_readfirstlane(G * (nst * wave / W));
   const int ng = __builtin_amdgcn_readfirstlane(min(wi.ngroups, G * (nst * (wave + 1) / W)) - g0);
@@ -618,22 +415,12 @@ k_slab_mfma32(const bwl::WorkItem* __restrict__ wis, XcdSplit xs,
   for (int c = 0; c < NC; ++c) acc[0][c] = acc[1][c] = floatx16{0};
   float* mine = lds + wave * 32 * NB;  // the wave's B slot, then its image of the sums
   const bool two = R > 32;
-  auto run = [&](const flt4* __restrict__ base, const auto& rows, bool fits) {
-    bool done = ng <= 0;
-    if (!done && fits) {
-      if (two)
-        done = split32_stream<NC, DS, true>(base, gi, XB, ng, rows, half, r0, mine, acc);
-      else
-        done = split32_stream<NC, DS, false>(base, gi, XB, ng, rows, half, r0, mine, acc);
-    }
-    if (!done) {
-#pragma unroll
-      for (int c = 0; c < NC; ++c) acc[0][c] = acc[1][c] = floatx16{0};
-      if (two)
-        mfma32_stream<NC, KU, D, true>(base, gi, XB, ng, rows, half, r0, mine, acc);
-      else
-        mfma32_stream<NC, KU, D, false>(base, gi, XB, ng, rows, half, r0, mine, acc);
-    }
+  auto run = [&](const flt4* __restrict__ base, const auto& rows) {
+    if (ng <= 0) return;
+    if (two)
+      mfma32_stream<NC, KU, D, true>(base, gi, XB, ng, rows, half, r0, mine, acc);
+    else
+      mfma32_stream<NC, KU, D, false>(base, gi, XB, ng, rows, half, r0, mine, acc);
   };
   const int row0 = min(r0, R - 1), row1 = min(r0 + 32, R - 1);
   if constexpr (WIN) {
@@ -642,14 +429,14 @@ k_slab_mfma32(const bwl::WorkItem* __restrict__ wis, XcdSplit xs,
     const int64_t first =
         static_cast<int64_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(e >> 32))) << 32 |
         static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(e)));
-    const uint32_t s0 = 16u * (e0 & 0xff), s1 = 16u * (e1 & 0xff);
-    const uint32_t g = static_cast<uint32_t>(wi.data_off) + g0;  // the wave's first group
-    const WindowRows rows{ng, 16u * static_cast<uint32_t>((e0 >> 8) - first) + g * s0, s0,
-                          16u * static_cast<uint32_t>((e1 >> 8) - first) + g * s1, s1};
-    run(reinterpret_cast<const flt4*>(data) + first, rows, true);
+    const int s0 = e0 & 0xff, s1 = e1 & 0xff;
+    const int g = static_cast<int>(wi.data_off) + g0;  // the wave's first group
+    const WindowRows rows{ng, static_cast<int>((e0 >> 8) - first) + g * s0, s0,
+                          static_cast<int>((e1 >> 8) - first) + g * s1, s1};
+    run(reinterpret_cast<const flt4*>(data) + first, rows);
   } else {
     run(reinterpret_cast<const flt4*>(data + wi.data_off) + static_cast<int64_t>(g0) * R,
-        SlabRows{R, ng, row0, row1}, static_cast<int64_t>(ng) * R < (1 << 27));
+        SlabRows{R, ng, row0, row1});
   }
   auto put = [&](const floatx16 (&a)[NC]) {
 #pragma unroll

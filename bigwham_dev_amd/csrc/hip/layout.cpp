@@ -253,10 +253,10 @@ constexpr int64_t kItemBatched = 96 * 1024, kItemBatchedMin = 16 * 1024, kBatche
 constexpr int64_t kPass1Share = 1500, kPass1MinBytes = 48 * 1024;
 // Rounds of 64 columns read four times the bytes of a 16-row slab as input rows,
 // and its 32-row tiles are half empty: from this size on they take pass 1 in
-// windows of 64 rows over all slabs of a column cluster instead (24 300 DoF,
-// pass 1: 115 us in slabs, 80 + 7 in windows; whole products 203 -> 186 us at 46 M
-// entries in pass 1, 97 -> 90 at 15 M, mode-1 130 -> 123 at 21 M but 71 -> 76 at
-// 10 M).  Narrower rounds lose by the split windows (16 columns 3-10 %, 32 columns
+// windows of 64 rows over all slabs of a column cluster instead (whole products,
+// slabs and windows: 470 and 426 us at 114 M entries in pass 1, 241 and 217 at
+// 46 M, 117 and 115 at 15 M, 69.6 and 68.8 at 8 M; mode-1 263 and 254 at 40 M, 141
+// and 136 at 17 M, but 80 and 87 at 8 M).  Narrower rounds lose by the split windows (16 columns 3-10 %, 32 columns
 // -4 to +4 %), and FP64 takes 277 us in slabs, 288 in windows.
 constexpr int64_t kWindowEntries = 12 << 20, kMaxWindowGroups = 1 << 20;
 constexpr int64_t kSortEntries = 200 << 20;
@@ -366,7 +366,7 @@ void finalize_program(Program* P, const LayoutOptions& opt, int64_t wi_single, b
   P->wide = ItemList{};
   P->rowtab.clear();
   if (opt.elem_bytes != 4 || tuned || P->rowmap.empty() || data < kWindowEntries) return;
-  // the rows of a window lie within 192 rows of slabs: 32-bit byte offsets
+  // the rows of a window lie within 192 rows of slabs: 32-bit offsets
   for (const SlabDesc& sd : P->slabs)
     if (sd.ngroups >= kMaxWindowGroups) return;
   // Windows of up to 64 rows over the slabs of one column cluster, whose rows

@@ -121,8 +121,7 @@ int bw_hip_rmatvec(bw_hip_handle* hd, const double* x, double* y, int ordering,
  * Both precisions run the passes as thin GEMMs on MFMA, in rounds of 16 or 32
  * right-hand sides (FP32 also 64).  FP64: v_mfma_f64_16x16x4f64, same summation
  * bar as the single-RHS FP64 path; FP32: v_mfma_f32_16x16x4f32, and in the wider
- * rounds products of three bf16 parts per float (v_mfma_f32_32x32x16_bf16), the
- * error of FP32 products. */
+ * rounds v_mfma_f32_32x32x2f32. */
 int bw_hip_matvec_batched(bw_hip_handle* hd, int nrhs, const double* X, int64_t ldx,
                           double* Y, int64_t ldy, int ordering, int precision,
                           void* stream);
