@@ -131,6 +131,8 @@ def hip() -> C.CDLL:
         lib.bw_layout_export_xcd.argtypes = [_vp, C.c_int, C.POINTER(C.c_int32),
                                              C.POINTER(C.c_int32)]
         lib.bw_layout_items_info.argtypes = [_vp, C.c_int, C.c_int, _i64]
+        lib.bw_layout_items_export.argtypes = [_vp, C.c_int, C.c_int, _i64, _i64,
+                                               C.POINTER(C.c_int32), _i64]
         lib.bw_layout_free.argtypes = [_vp]
         lib.bw_layout_free.restype = None
         lib.bw_layout_last_error.restype = C.c_char_p
@@ -203,7 +205,7 @@ HIP_SYMBOLS = ["bw_hip_create", "bw_hip_matvec", "bw_hip_matvec_noalloc", "bw_hi
                "bw_hip_orthogonalize_work", "bw_hip_orthogonalize", "bw_hip_set_timing",
                "bw_hip_timing_stats", "bw_hip_destroy", "bw_hip_last_error",
                "bw_layout_build", "bw_layout_info", "bw_layout_export", "bw_layout_free",
-               "bw_layout_export_rowmap", "bw_layout_export_xcd", "bw_layout_items_info",
+               "bw_layout_export_rowmap", "bw_layout_export_xcd", "bw_layout_items_info", "bw_layout_items_export",
                "bw_layout_last_error", "bw_layout_build_multi", "bw_hip_create_multi",
                "bw_hip_graph_create", "bw_hip_graph_launch", "bw_hip_graph_destroy",
                "bw_hip_graph_create_batched", "bw_hip_stream_release",

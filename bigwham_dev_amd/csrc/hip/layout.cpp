@@ -325,9 +325,6 @@ void cut_items(const std::vector<SlabDesc>& slabs, const LayoutOptions& opt, int
     for (int x = 0; x < kXcds; ++x)
       std::stable_sort(il->wis.begin() + il->xcd[x], il->wis.begin() + il->xcd[x + 1],
                        [&](const WorkItem& a, const WorkItem& b) { return cost(a) > cost(b); });
-  int32_t most = 0;
-  for (int x = 0; x < kXcds; ++x) most = std::max(most, il->xcd[x + 1] - il->xcd[x]);
-  il->xcd_blocks = kXcds * ((most + 3) / 4);
 }
 
 // Places the slabs' data and column groups, and cuts both work-item lists.

@@ -114,9 +114,8 @@ struct ItemList {
   // each: all of them, or none (0) where a reduction launch adds them.
   int32_t counters = 0;
   // Work items [xcd[x], xcd[x+1]) run on XCD x: eight contiguous ranges of
-  // about equal bytes; xcd_blocks groups of four work items cover the longest.
+  // about equal cost.
   int32_t xcd[kXcds + 1] = {};
-  int32_t xcd_blocks = 0;
 
   // workgroups of a launch: one per work item of the longest range, on every XCD
   int32_t blocks() const {

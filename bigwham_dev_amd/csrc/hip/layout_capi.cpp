@@ -54,6 +54,28 @@ int build_checked(const bw_flat_hmat* h, long double area, int precision, int ad
   return BW_OK;
 }
 
+// list 0: single-vector, 1: batched, 2: windows of rounds of 64 columns
+const bwl::ItemList* item_list(const bw_layout* lay, int pass, int list) {
+  if (!lay || (pass != 1 && pass != 2) || list < 0 || list > 2) return nullptr;
+  const bwl::Program& P = pass == 1 ? lay->L.pass1 : lay->L.pass2;
+  return list == 0 ? &P.single : list == 1 ? &P.batched : &P.wide;
+}
+
+void put_items(const bwl::ItemList& il, int64_t* o) {
+  for (const bwl::WorkItem& w : il.wis) {
+    o[0] = w.data_off; o[1] = w.gbeg; o[2] = w.ngroups; o[3] = w.rows;
+    o[4] = w.out_row; o[5] = w.part_off; o[6] = w.red; o[7] = 0;
+    o += 8;
+  }
+}
+
+void put_reduces(const bwl::ItemList& il, int64_t* o) {
+  for (const bwl::Reduce& r : il.reds) {
+    o[0] = r.out_row; o[1] = r.rows; o[2] = r.part_off; o[3] = r.nparts;
+    o += 4;
+  }
+}
+
 }  // namespace
 
 int bw_layout_build(const bw_flat_hmat* h, int precision, int adjoint, int64_t wi_bytes,
@@ -111,54 +133,60 @@ int bw_layout_export_rowmap(const bw_layout* lay, int32_t* rowmap) {
   return BW_OK;
 }
 
-// wis: 8 int64 per WI (data_off, gbeg, ngroups, rows, out_row, part_off, 0, 0);
+// wis: 8 int64 per WI (data_off, gbeg, ngroups, rows, out_row, part_off, red, 0);
 // reds: 4 int64 per reduce (one per split slab);
 // data in double regardless of precision.
 int bw_layout_export(const bw_layout* lay, int pass, int64_t* wis, int32_t* gidx, int64_t* reds,
                      double* data) {
   if (!lay || (pass != 1 && pass != 2)) return BW_EINVAL;
   const bwl::Program& P = pass == 1 ? lay->L.pass1 : lay->L.pass2;
-  if (wis)
-    for (size_t i = 0; i < P.single.wis.size(); ++i) {
-      const bwl::WorkItem& w = P.single.wis[i];
-      int64_t* o = wis + 8 * i;
-      o[0] = w.data_off; o[1] = w.gbeg; o[2] = w.ngroups; o[3] = w.rows;
-      o[4] = w.out_row; o[5] = w.part_off; o[6] = 0; o[7] = 0;
-    }
+  if (wis) put_items(P.single, wis);
   if (gidx && !P.gidx.empty()) std::memcpy(gidx, P.gidx.data(), P.gidx.size() * sizeof(int32_t));
-  if (reds)
-    for (size_t i = 0; i < P.single.reds.size(); ++i) {
-      const bwl::Reduce& r = P.single.reds[i];
-      reds[4 * i] = r.out_row; reds[4 * i + 1] = r.rows;
-      reds[4 * i + 2] = r.part_off; reds[4 * i + 3] = r.nparts;
-    }
+  if (reds) put_reduces(P.single, reds);
   if (data && !P.slabs.empty())
     bwl::fill_slabs<double>(lay->L, P, 0, static_cast<int32_t>(P.slabs.size()), data);
   return BW_OK;
 }
 
-// xcd: 9 int32 (XCD x runs work items [xcd[x], xcd[x+1])); blocks: the
-// workgroup count of the pass's launch.
+// xcd: 9 int32 (XCD x runs work items [xcd[x], xcd[x+1])) of the single-vector
+// list; blocks: groups of four work items that cover the longest range, times 8.
 int bw_layout_export_xcd(const bw_layout* lay, int pass, int32_t* xcd, int32_t* blocks) {
   if (!lay || !xcd || !blocks || (pass != 1 && pass != 2)) return BW_EINVAL;
   const bwl::Program& P = pass == 1 ? lay->L.pass1 : lay->L.pass2;
   for (int x = 0; x <= bwl::kXcds; ++x) xcd[x] = P.single.xcd[x];
-  *blocks = P.single.xcd_blocks;
+  *blocks = bwl::kXcds * ((P.single.blocks() / bwl::kXcds + 3) / 4);
   return BW_OK;
 }
 
-// list: 0 single-vector, 1 batched, 2 windows of rounds of 64 columns.
 // info[0..4] = work items, split slabs, partial sums (elements of one column),
 // counters of split slabs, workgroups of the launch.
 int bw_layout_items_info(const bw_layout* lay, int pass, int list, int64_t* info) {
-  if (!lay || !info || (pass != 1 && pass != 2) || list < 0 || list > 2) return BW_EINVAL;
-  const bwl::Program& P = pass == 1 ? lay->L.pass1 : lay->L.pass2;
-  const bwl::ItemList& il = list == 0 ? P.single : list == 1 ? P.batched : P.wide;
-  info[0] = static_cast<int64_t>(il.wis.size());
-  info[1] = static_cast<int64_t>(il.reds.size());
-  info[2] = il.part_elems;
-  info[3] = il.counters;
-  info[4] = il.blocks();
+  const bwl::ItemList* il = item_list(lay, pass, list);
+  if (!il || !info) return BW_EINVAL;
+  info[0] = static_cast<int64_t>(il->wis.size());
+  info[1] = static_cast<int64_t>(il->reds.size());
+  info[2] = il->part_elems;
+  info[3] = il->counters;
+  info[4] = il->blocks();
+  return BW_OK;
+}
+
+// wis: 8 int64 per work item (data_off, gbeg, ngroups, rows, out_row, part_off,
+// red, 0; of a window data_off is its first column group); reds: 4 int64 per
+// split slab; xcd: 9 int32; rowtab (list 2): one int64 per entry of the row map.
+// Null pointers are skipped.
+int bw_layout_items_export(const bw_layout* lay, int pass, int list, int64_t* wis, int64_t* reds,
+                           int32_t* xcd, int64_t* rowtab) {
+  const bwl::ItemList* il = item_list(lay, pass, list);
+  if (!il) return BW_EINVAL;
+  if (wis) put_items(*il, wis);
+  if (reds) put_reduces(*il, reds);
+  if (xcd)
+    for (int x = 0; x <= bwl::kXcds; ++x) xcd[x] = il->xcd[x];
+  if (rowtab && list == 2) {
+    const auto& t = (pass == 1 ? lay->L.pass1 : lay->L.pass2).rowtab;
+    if (!t.empty()) std::memcpy(rowtab, t.data(), t.size() * sizeof(int64_t));
+  }
   return BW_OK;
 }
 

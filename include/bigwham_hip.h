@@ -296,14 +296,19 @@ int bw_layout_export(const bw_layout* lay, int pass, int64_t* wis, int32_t* gidx
 /* The pass-1 row map (info[15] int32 entries): work item / reduce rows of
  * pass 1 are indices into it, and it gives each row's t entry in xt. */
 int bw_layout_export_rowmap(const bw_layout* lay, int32_t* rowmap);
-/* The split of a pass's work items over the 8 XCDs: XCD x runs work items
- * [xcd[x], xcd[x+1]) (9 entries), with `blocks` workgroups of 4 waves. */
+/* The split of a pass's single-vector work items over the 8 XCDs: XCD x runs
+ * work items [xcd[x], xcd[x+1]) (9 entries); blocks / 8 groups of four items cover
+ * the longest range (bw_layout_items_info: the workgroups of a launch). */
 int bw_layout_export_xcd(const bw_layout* lay, int pass, int32_t* xcd, int32_t* blocks);
 /* One work-item list of a pass (list 0: single-vector kernels, 1: batched, 2: the
  * windows of FP32 rounds of 64 columns): work items, split slabs, partial sums
  * of one column, counters of the split slabs that their last work item adds (all
  * of them, or 0: a reduction launch does), workgroups of a launch. */
 int bw_layout_items_info(const bw_layout* lay, int pass, int list, int64_t* info /* 5 */);
+/* Its work items (8 int64 each), split slabs (4 int64 each), XCD ranges (9
+ * int32) and, for list 2, the row table (one int64 per row-map entry). */
+int bw_layout_items_export(const bw_layout* lay, int pass, int list, int64_t* wis,
+                           int64_t* reds, int32_t* xcd, int64_t* rowtab);
 void bw_layout_free(bw_layout* lay);
 const char* bw_layout_last_error(void);
 
