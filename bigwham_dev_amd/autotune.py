@@ -23,6 +23,8 @@ import os
 from dataclasses import dataclass, field
 
 UNROLLS = (4, 8)
+# the batched kernels have one schedule, which every accepted number selects
+MFMA_SCHEDULES = MFMA64_SCHEDULES = (0,)
 WI_BYTES = (128 << 10, 192 << 10, 384 << 10, 768 << 10)
 
 
@@ -111,20 +113,27 @@ def tune_unroll(dev, precisions=None, reps: int = 5, use_cache: bool = True) -> 
 
 
 def tune_mfma(dev, nrhs: int = 32, reps: int = 5, precision: str = "fp32") -> dict:
-    """Time the batched product of one precision on `nrhs` right-hand sides.
-    Its kernels have one schedule (0): returns {0: ms per call, "best": 0}."""
+    """Time the schedules of the batched product of one precision on `nrhs`
+    right-hand sides and keep the fastest.  Returns {schedule: ms per call,
+    "best": schedule}; there is one schedule now."""
     import time
 
     import torch
     X = torch.ones((dev.n_cols, nrhs), dtype=torch.float64, device=dev.torch_device)
     Y = torch.empty((dev.n_rows, nrhs), dtype=torch.float64, device=dev.torch_device)
-    dev.matvec_batched(X, precision=precision, out=Y)
-    torch.cuda.synchronize()
-    t0 = time.perf_counter()
-    for _ in range(reps):
+    ms = {}
+    for sch in MFMA_SCHEDULES if precision == "fp32" else MFMA64_SCHEDULES:
+        dev.set_mfma_schedule(sch, precision)
         dev.matvec_batched(X, precision=precision, out=Y)
-    torch.cuda.synchronize()
-    return {0: (time.perf_counter() - t0) / reps * 1e3, "best": 0}
+        torch.cuda.synchronize()
+        t0 = time.perf_counter()
+        for _ in range(reps):
+            dev.matvec_batched(X, precision=precision, out=Y)
+        torch.cuda.synchronize()
+        ms[sch] = (time.perf_counter() - t0) / reps * 1e3
+    best = min(ms, key=ms.get)
+    dev.set_mfma_schedule(best, precision)
+    return {**ms, "best": best}
 
 
 def tune_layout(make_dev, precisions=("fp64", "fp32"), candidates=WI_BYTES, reps: int = 5):
