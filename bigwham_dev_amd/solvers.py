@@ -105,19 +105,6 @@ class _HostSteps:
         pass
 
 
-def _plain(w: torch.Tensor, V: torch.Tensor) -> bool:
-    """Whether w is one contiguous vector of V's kind that can be read through its
-    pointer: its memory holds its values (no pending negation, no subclass
-    with a meaning of its own) and nothing differentiates through the step.
-    Everything else is left to torch, which computes it or refuses it."""
-    return (type(w) is torch.Tensor and w.dtype == V.dtype and w.device == V.device
-            and w.dim() == 1 and w.numel() == V.shape[1] and w.is_contiguous()
-            and not w.is_neg()
-            and not ((w.requires_grad or V.requires_grad) and torch.is_grad_enabled())
-            and forward_ad.unpack_dual(w).tangent is None
-            and forward_ad.unpack_dual(V).tangent is None)
-
-
 class _DeviceSteps(_HostSteps):
     """The same on the GPU, queued: four kernels per step
     (bw_hip_orthogonalize) that write the column to pinned memory."""
@@ -127,6 +114,7 @@ class _DeviceSteps(_HostSteps):
     def __init__(self, V):
         super().__init__(V)
         restart, n = V.shape[0] - 1, V.shape[1]
+        self.n, self.index = n, V.get_device()
         # two rows, as two steps are in flight at most; a step that a cycle left
         # behind is done before the next cycle's steps, on the same stream
         self.cols = torch.empty((2, restart + 2), dtype=V.dtype, pin_memory=True)
@@ -139,9 +127,23 @@ class _DeviceSteps(_HostSteps):
                 self.native = N.hip()
                 self.work = torch.empty(need.value, dtype=V.dtype, device=V.device)
 
+    def _plain(self, w):
+        """Whether w is one contiguous vector of V's kind that can be read through its
+        pointer: its memory holds its values (no pending negation, no subclass
+        with a meaning of its own) and nothing differentiates through the step.
+        Everything else is left to torch, which computes it or refuses it."""
+        V = self.V
+        return (type(w) is torch.Tensor and w.dtype is V.dtype and w.get_device() == self.index
+                and w.dim() == 1 and w.numel() == self.n and w.is_contiguous()
+                and not w.is_neg()
+                and not ((w.requires_grad or V.requires_grad) and torch.is_grad_enabled())
+                and (forward_ad._current_level < 0  # no dual numbers about
+                     or (forward_ad.unpack_dual(w).tangent is None
+                         and forward_ad.unpack_dual(V).tangent is None)))
+
     def queue(self, k, w):
         V = self.V
-        if self.native and _plain(w, V):
+        if self.native and self._plain(w):
             rc = self.native.bw_hip_orthogonalize(
                 V.device.index, V.shape[1], k + 1, V.data_ptr(), V.stride(0), w.data_ptr(),
                 V[k + 1].data_ptr(), self.cols[k & 1].data_ptr(), self.work.data_ptr(),
