@@ -11,9 +11,9 @@
 // 426), and wins from 33 columns on (295 + 257 -> 426).  FP64 stays at 32: its
 // time goes with the columns (158 us for one vector).
 //
-// What bounds them: reads from L2 (63-69 G requests a second here and in the
-// single-vector kernel, input rows 25-65 % of them), and at 64 columns the
-// FP32 matrix instructions.
+// What bounds them: reads from L2 (53-75 G requests a second up to 32 columns and
+// in the single-vector kernel, input rows 40-50 % of them); at 64 columns 46-55 G,
+// with the FP32 matrix instructions busy 47-68 % of the time.
 //
 // A workgroup of W waves takes one work item: the waves take contiguous
 // shares of its k-steps, each with a full set of accumulators, and the sums

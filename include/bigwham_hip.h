@@ -206,7 +206,10 @@ int bw_flat_full_blocks(const bw_flat_hmat* h, int ordering, const int64_t* rows
 const char* bw_flat_full_blocks_last_error(void);
 
 /* Tuning knobs for the next create: work-item target bytes (0 = sized from
- * the matrix: about 32k work items, 8 KiB to 384 KiB FP64 / 192 KiB FP32). */
+ * the matrix, single-vector and batched products apart).  A size above 0 is used
+ * for both, and turns off what the automatic sizes choose by the operator: low
+ * slabs of small operators and, in FP32 products of more than 32 columns, the
+ * windows over a column cluster's slabs. */
 int bw_hip_set_tuning(int64_t wi_bytes_fp64, int64_t wi_bytes_fp32);
 
 /* Low-rank recompression of the FP32 copy for the next create (0, the
